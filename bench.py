@@ -35,10 +35,10 @@ TRAFFIC_BYTES_PER_LAUNCH = {"rhs": (2.0 * 13548 + 12420) * 1024, "rhs_combine": 
 # (profiles/k_rhs_disk512x1024_sq_counters.md)
 VALU_FLOOR_US = {"rhs": 9.55, "rhs_combine": 12.87, "remap": 2.69, "rhs_end": 10.89}
 KERNEL_NAMES = {
-    "rhs": "fv::k_rhs<double,3,VANLEER,64,3,M_STAGE>: stage 2 (stage sum over k_1, ghost cells, RHS)",
-    "rhs_combine": "fv::k_rhs<double,3,VANLEER,64,3,M_LAST>: stage 3 with the final combination and "
+    "rhs": "fv::k_rhs<double,3,VANLEER,1,M_STAGE>: stage 2 (stage sum over k_1, ghost cells, RHS)",
+    "rhs_combine": "fv::k_rhs<double,3,VANLEER,2,M_LAST>: stage 3 with the final combination and "
                    "embedded error",
-    "rhs_end": "fv::k_rhs<double,3,VANLEER,64,3,M_END>: end-of-step RHS (CFL, data checks, new state)",
+    "rhs_end": "fv::k_rhs<double,3,VANLEER,0,M_END>: end-of-step RHS (CFL, data checks, new state)",
     "remap": "fv::k_remap<double,3>: FARGO azimuthal remap",
 }
 METRIC = "cell-updates/s & HBM GB/s vs plain FP64 at stated err; p50/p99 run latency"

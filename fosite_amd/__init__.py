@@ -385,8 +385,8 @@ class Batch:
     kernel of a step is one launch over all members, the steps of a round one
     HIP graph.  Results are bit-identical to running each member alone.
 
-    tiling: 0/1 = 64-wide RHS tiles in row-major / XCD-chunked order, 2/3 =
-    the same with 32-wide tiles; with ``autotune`` the batch times all four
+    tiling: 0/1 = tall RHS strips in row-major / XCD-chunked order, 2/3 = the
+    same with strips of half the rows; with ``autotune`` the batch times all four
     on its first device steps and keeps the fastest."""
 
     def __init__(self, sims=(), autotune=True, tiling=0, max_graph_steps=0, reuse_tuning=False):

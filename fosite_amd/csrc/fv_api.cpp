@@ -424,7 +424,7 @@ int rhs_main(fv_ctx *ctx, int checkbm, int remap, double t) {
   ctx->pvalid = true;
   ctx->pflag = ctx->fl_pvar;
   ctx->cvar = outb;
-  int rc = reduce(ctx, ctx->part_r, ctx->nb_rhs, &ctx->invdt, &ctx->flags);
+  int rc = reduce(ctx, ctx->part_r, ctx->nb_rhs + 1, &ctx->invdt, &ctx->flags);
   if (rc) return rc;
   if (checkbm != CHECK_NOTHING) {
     if ((checkbm & CHECK_CSOUND) && ctx->V == 3 && ctx->cs_min <= 0.) ctx->brk = 1;
@@ -1086,6 +1086,9 @@ extern "C" int fv_create(fv_ctx **out, const fv_config *cfg) {
                                      {R_DAXE, M_DAXE}, {R_DAYN, M_DAYN}};
   for (auto &p : rm)
     if (!ring_from(ctx, p.r, ctx->mesh.a[p.m].data())) return bail("mesh metric depends on j");
+  for (int id : {R_CXYX, R_CZXZ, R_CZYZ})  // k_rhs leaves their terms out
+    for (int i = 0; i < ctx->NI; i++)
+      if (ctx->ring_h[(size_t)id * ctx->NI + i] != 0.0) return bail("commutator coefficients besides c_yxy");
   for (int j = 0; j < ctx->NJ; j++) {
     ctx->col_h[(size_t)C_RDYS * ctx->NJ + j] = ctx->mesh.a[M_RDYS][(size_t)j * ctx->NI];
     ctx->col_h[(size_t)C_RDYN * ctx->NJ + j] = ctx->mesh.a[M_RDYN][(size_t)j * ctx->NI];
@@ -1152,12 +1155,11 @@ extern "C" int fv_create(fv_ctx **out, const fv_config *cfg) {
   g.twoomega = 2 * c.omega;
   g.dtype = c.dtype;
   g.stages = ctx->tab.m;
-  g.tile_x = 64;
-  if (const char *e = std::getenv("FV_RHS_TILE")) g.tile_x = std::atoi(e) == 32 ? 32 : 64;
+  g.rows = strip_rows((long)strip_cols(c.inum) * c.jnum, c.dtype);
+  // FV_RHS_TILE=32: strips of half the rows
+  if (const char *e = std::getenv("FV_RHS_TILE")) g.rows = std::atoi(e) == 32 ? std::max(1, g.rows / 2) : g.rows;
   ctx->nb_rhs = rhs_blocks(g);
-  Geom g32 = g;  // partials sized for the finest tiling, which batches may choose
-  g32.tile_x = 32;
-  const int nb_part = std::max(ctx->nb_rhs, rhs_blocks(g32));
+  const int nb_part = strip_cols(c.inum) * strip_blocks(c.jnum, 1) + 1;  // the finest tiling, which batches may choose
   ok = ok && dalloc(&ctx->part_r, sizeof(double) * 2 * nb_part) &&
        dalloc(&ctx->part_c, sizeof(double) * 2 * nb_part) && dalloc(&ctx->d_red, sizeof(double) * 2);
   ok = ok && hipMalloc((void **)&ctx->d_ctl, sizeof(Ctl)) == hipSuccess &&
@@ -1301,7 +1303,7 @@ extern "C" int fv_device_bytes(const fv_config *c, double *bytes) {
   const double NI = c->inum + 4.0, NJ = c->jnum + 4.0, P = std::ceil(NI / 16.0) * 16.0;
   const double V = c->physics == EULER ? 4.0 : 3.0, es = c->dtype == 1 ? 4.0 : 8.0;
   const double state = es * V * NJ * P;  // one state buffer, ghost cells and row padding included
-  const double nb32 = std::ceil(c->inum / 32.0) * std::ceil(c->jnum / (double)TY_TILE);
+  const double nbp = (double)strip_cols(c->inum) * strip_blocks(c->jnum, 1) + 1.0;
   double b = state * (NBUF + (t.m - 1) + 2 + 1);      // states, stage rhs, coeff(1) pair, pvar
   b += 3.0 * 8.0 * 2.0 * V * (NI + NJ);                // boundary fluxes (two copies), last-stage rows
   if (c->fargo == 1)                                    // FARGO type 1: velocities, second ring arrays
@@ -1311,7 +1313,7 @@ extern "C" int fv_device_bytes(const fv_config *c, double *bytes) {
     b += 8.0 * (V - 1.0) * NJ * P + 16.0 * std::ceil(NI / 64.0) * std::ceil(NJ / 8.0);
   if (c->vismodel >= 2)                                 // viscosity, e_phi/r, r^2; Euler ALPHA: sound speeds
     b += (c->vismodel == 2 && V == 4 ? 6.0 : 4.0) * 8.0 * NJ * P;
-  b += 2.0 * 2.0 * 8.0 * nb32;                         // CFL and error partials
+  b += 2.0 * 2.0 * 8.0 * nbp;                          // CFL and error partials
   b += 8.0 * (R_COUNT * NI + C_COUNT * NJ);             // metric arrays
   if (c->dtype == 1) b += 4.0 * (R_COUNT * NI + C_COUNT * NJ);
   b += sizeof(Ctl) + 16.0;
@@ -1501,8 +1503,9 @@ extern "C" int fv_step(fv_ctx *ctx, int *done) {
 extern "C" int fv_step_noalloc(fv_ctx *ctx, int *done) {
   if (!ctx) return -1;
   if (ctx->prof) return fail(ctx, "fv_step_noalloc: kernel profiling (fv_profile) creates events; disable it");
-  if (ctx->nb_rhs > SCRATCH_MAX_BLOCKS)
-    return fail(ctx, "fv_step_noalloc: " + std::to_string(ctx->nb_rhs) + " workgroups per RHS launch exceed the " +
+  const long tiles = (long)strip_cols(ctx->c.inum) * ((ctx->c.jnum + 7) / 8);  // of 64 x 8 cells
+  if (tiles > SCRATCH_MAX_BLOCKS || ctx->nb_rhs + 1 > SCRATCH_MAX_BLOCKS)
+    return fail(ctx, "fv_step_noalloc: " + std::to_string(tiles) + " tiles of 64 x 8 cells exceed the " +
                          std::to_string(SCRATCH_MAX_BLOCKS) + " the static scratch holds (use fv_step)");
   int cur = -1;
   HIPCHK(hipGetDevice(&cur));
@@ -1691,10 +1694,9 @@ extern "C" const char *fv_last_error(const fv_ctx *ctx) { return ctx ? ctx->err.
 // the single-context code above.
 
 namespace {
-constexpr int NCAND = 4;     // RHS tilings: 64 row-major, 64 XCD-chunked, 32 row-major, 32 XCD-chunked
+constexpr int NCAND = 4;     // RHS tilings: tall strips row-major, XCD-chunked, strips of half the rows row-major, XCD-chunked
 constexpr int XCDS = 8;      // MI355X: workgroup b of a launch is dispatched to XCD b mod 8
 constexpr int TUNE_REPS = 2;
-int cand_tx(int c) { return c < 2 ? 64 : 32; }
 }  // namespace
 
 struct fv_batch {
@@ -1776,22 +1778,38 @@ void free_tables(fv_batch *b) {
   b->cap = 0;
 }
 
+// strip rows of tiling c: tall strips by the rule for single meshes over all
+// members, and half of it; a member's block rows have to fit the tile codes
+int cand_rows(const fv_batch *b, int c) {
+  long wave_rows = 0;
+  int least = 1;
+  for (const fv_ctx *x : b->sims) {
+    wave_rows += (long)strip_cols(x->c.inum) * x->c.jnum;
+    while (strip_blocks(x->c.jnum, least) >= (1 << TILE_BY_BITS)) least++;
+  }
+  const int r = strip_rows(wave_rows, b->dtype);
+  return std::max(least, c < 2 ? r : std::max(1, r / 2));
+}
+
 // k_rhs tile list of tiling c over all members
 std::vector<unsigned> rhs_tiles(const fv_batch *b, int c) {
-  const int tx = cand_tx(c);
-  std::vector<unsigned> lin;
+  const int rows = cand_rows(b, c);
+  std::vector<unsigned> lin, aux;
   for (size_t d = 0; d < b->sims.size(); d++) {
     const fv_ctx *x = b->sims[d];
-    const int nbx = (x->c.inum + tx - 1) / tx, nby = (x->c.jnum + TY_TILE - 1) / TY_TILE;
+    const int nbx = strip_cols(x->c.inum), nby = strip_blocks(x->c.jnum, rows);
     for (int by = 0; by < nby; by++)
       for (int bx = 0; bx < nbx; bx++) lin.push_back(tile_code((int)d, bx, by));
+    for (int k = 0; k < rhs_aux_max(x->g, x->V); k++) aux.push_back(tile_code((int)d, k, nby));
   }
-  if (!(c & 1)) return lin;
-  // XCD-chunked: tile t goes to XCD t / Q, at that XCD's slot t % Q
-  const size_t N = lin.size(), Q = (N + XCDS - 1) / XCDS;
-  std::vector<unsigned> out(Q * XCDS, NO_TILE);
-  for (size_t t = 0; t < N; t++) out[(t % Q) * XCDS + t / Q] = lin[t];
-  return out;
+  if (c & 1) {  // XCD-chunked: tile t goes to XCD t / Q, at that XCD's slot t % Q
+    const size_t N = lin.size(), Q = (N + XCDS - 1) / XCDS;
+    std::vector<unsigned> out(Q * XCDS, NO_TILE);
+    for (size_t t = 0; t < N; t++) out[(t % Q) * XCDS + t / Q] = lin[t];
+    lin.swap(out);
+  }
+  lin.insert(lin.end(), aux.begin(), aux.end());  // the auxiliary workgroups, over all XCDs
+  return lin;
 }
 
 // tables and tile lists for the current members; graphs are recaptured
@@ -1860,7 +1878,7 @@ void enqueue_batch_step(fv_batch *b, int p, int c) {
   const unsigned *tl = b->d_tiles + b->cand_off[c];
   for (int q = 0; q < m - 1; q++)  // stages 2..s, the last fused with the combination
     launch_rhs_multi(b->d_rhs + (size_t)(p * m + q) * cap, tl, b->cand_n[c], b->V, b->dtype, b->limiter,
-                     cand_tx(c), b->m, q == m - 2 ? 1 : 0, b->st);
+                     cand_rows(b, c), q == m - 2 ? 1 : 0, q + 1, b->st);
   if (b->remap_n)
     launch_remap_multi(b->d_remap + (size_t)p * cap, b->d_tiles + b->remap_off, b->remap_n, b->V, b->dtype, b->st);
   if (b->acc_n) {  // the step's boundary fluxes, then UpdateGravity
@@ -1868,7 +1886,7 @@ void enqueue_batch_step(fv_batch *b, int p, int c) {
     launch_accrete_multi(b->d_acc + (size_t)p * cap, b->acc_n, b->st);
   }
   launch_rhs_multi(b->d_rhs + (size_t)(p * m + m - 1) * cap, tl, b->cand_n[c], b->V, b->dtype, b->limiter,
-                   cand_tx(c), b->m, 2, b->st);
+                   cand_rows(b, c), 2, 0, b->st);
   launch_control_multi(b->d_cent + (size_t)c * cap, n, b->st);
 }
 
@@ -1913,6 +1931,8 @@ int batch_round(fv_batch *b, const std::vector<int> &want, int K, int c, bool ti
   const int n = (int)b->sims.size(), m = b->m, cap = b->cap;
   b->roles.resize(n);
   int ai = 0;  // entry of the next accreting member
+  int rows_of[NCAND];
+  for (int cc = 0; cc < NCAND; cc++) rows_of[cc] = cand_rows(b, cc);
   for (int d = 0; d < n; d++) {
     fv_ctx *x = b->sims[d];
     Ctl *h = &b->h_ctl[d];
@@ -1948,8 +1968,7 @@ int batch_round(fv_batch *b, const std::vector<int> &want, int K, int c, bool ti
       b->h_remap[(size_t)p * cap + d] = re;
     }
     for (int cc = 0; cc < NCAND; cc++) {
-      const int tx = cand_tx(cc);
-      const int nb = ((x->c.inum + tx - 1) / tx) * ((x->c.jnum + TY_TILE - 1) / TY_TILE);
+      const int nb = strip_cols(x->c.inum) * strip_blocks(x->c.jnum, rows_of[cc]);
       b->h_cent[(size_t)cc * cap + d] = ControlEntry{dc, x->part_c, x->part_r, nb};
     }
     if (x->grav[0]) ai++;
@@ -2030,7 +2049,7 @@ extern "C" int fv_batch_add(fv_batch *b, fv_ctx *x) {
   if (x->batch) return bfail(b, "context already belongs to a batch");
   if ((int)b->sims.size() >= MAX_BATCH) return bfail(b, "batch is full (" + std::to_string(MAX_BATCH) + " members)");
   if (x->c.vismodel) return bfail(b, "viscosity is supported on single contexts, not in batches");
-  const int nbx = (x->c.inum + 31) / 32, nby = (x->c.jnum + TY_TILE - 1) / TY_TILE, rby = remap_rows_blocks(x->c.jnum);
+  const int nbx = (x->c.inum + 31) / 32, nby = (x->c.jnum + 7) / 8, rby = remap_rows_blocks(x->c.jnum);
   if (nbx >= (1 << TILE_BX_BITS) || nby >= (1 << TILE_BY_BITS) || rby >= (1 << TILE_BY_BITS))
     return bfail(b, "mesh too large for a batch tile code");
   if (b->sims.empty()) {

@@ -7,7 +7,6 @@ namespace fv {
 
 constexpr int GH = 2;       // ghost layers per side (mesh/mesh_base.f90:462)
 constexpr int MAXK = 7;     // RK stages (Dormand-Prince has 7)
-constexpr int TILE_X = 64;  // tile width in cells (one wavefront per tile row)
 constexpr int CTL_HIST = 512;  // steps per device-controlled batch
 
 enum Physics { EULER_ISOTHERM = 16, EULER = 17 };
@@ -40,7 +39,7 @@ struct Geom {
   int fargo, gravity, curvilinear;
   int rotframe;         // rotating-frame source: 0 off, 1 centrifugal + Coriolis, 2 Coriolis only
   double twoomega;      // 2*Omega (sources_rotframe.f90:162); centrifugal terms in R_CACX, C_CACY
-  int tile_x;           // k_rhs tile width in cells: 64 or 32
+  int rows;             // k_rhs: rows of a wave's strip (1 .. STRIP_ROWS)
   int stages;           // RK stages of the tableau (picks the kernels' coefficient slots)
   int dtype;            // stored state: 0 FP64 (plain drop-in), 1 FP32 (precision form)
   const double *ring;   // [R_COUNT][NI]
@@ -57,11 +56,13 @@ struct Geom {
 // cannot decide alone (rejection, break, output, stop time) halts the batch
 // and the host redoes that step itself.
 enum HaltReason { H_NONE = 0, H_ERR = 1, H_DTLIMIT = 2, H_FLAGS = 3, H_OUTPUT = 4, H_STOP = 5, H_BATCH = 6 };
-struct Ctl {
+struct CtlHead {
   double time, dt, dt_step, t_out, stoptime, cfl, dtlimit, maxerrold, beta, order;
   double invdt;
   double cvis, invdt_v;  // viscosity (vis = 1): its Courant number and the last step's viscous 1/dt
   int halt, reason, step, nsteps, flags, vis;
+};
+struct Ctl : CtlHead {
   double err_hist[CTL_HIST], dt_hist[CTL_HIST];
 };
 
@@ -132,7 +133,7 @@ struct StageArgsT {
   int bflux;
   double *bks;
   // device-controlled end-of-step evaluation: the step's boundary-flux
-  // accumulation (bfa.out set), by the launch's first threads after their tiles
+  // accumulation (bfa.out set), by auxiliary workgroups of the launch
   BfluxArgs bfa;
   // FARGO type 1: the azimuthal velocity of the real frame as the next
   // CalcBackgroundVelocity sees it, (v - w) + w (timedisc_base.f90:2243-2326),
@@ -196,7 +197,7 @@ enum Flag { F_INVALID = 1, F_RHOMIN = 2, F_PMIN = 4 };
 // Batches of independent meshes: one launch per kernel of the step covers
 // every mesh.  Each launch reads its per-mesh arguments from a table in device
 // memory and maps block b to a tile through a tile list of 32-bit codes
-// (mesh index, tile column, tile row).
+// (mesh index, tile column, tile row; k_rhs: a workgroup's strips).
 struct RhsEntry {
   Geom g;
   StageArgs a;
@@ -249,20 +250,32 @@ void launch_accrete(const AccreteArgs &p, hipStream_t s);
 // arrays (FP64 and, for the precision form, FP32)
 void launch_wsum(const Geom &g, const double *v, double *ring, float *ringf, hipStream_t s,
                  const Ctl *ctl = nullptr);
-// batch launchers: ntiles blocks over the tile list; TX = tile width of the list
-#ifndef FV_RHS_ROWS
-#define FV_RHS_ROWS 8
-#endif
-constexpr int TY_TILE = FV_RHS_ROWS;  // k_rhs tile rows
+// k_rhs: strips of 64 columns x up to STRIP_ROWS rows, one per wave,
+// STRIP_WAVES of them above each other in a workgroup
+constexpr int STRIP_ROWS = 8, STRIP_WAVES = 4;
+__host__ __device__ inline int strip_cols(int inum) { return (inum + 63) / 64; }
+__host__ __device__ inline int strip_blocks(int jnum, int rows) {
+  return (jnum + rows * STRIP_WAVES - 1) / (rows * STRIP_WAVES);
+}
+// auxiliary workgroups of an end-of-step launch: the corner ghost cells, and with the boundary-flux
+// accumulation up to 64 more
+__host__ __device__ inline int rhs_aux_max(const Geom &g, int V) {
+  const int n = (V * 2 * (g.inum + g.jnum) + 255) / 256;
+  return 1 + (n < 64 ? n : 64);
+}
+// rows per strip for launches of `wave_rows` rows of 64 columns in all
+int strip_rows(long wave_rows, int dtype);
 // FARGO remap: rows per thread; a 64 x 4 block covers 64 rings x 4*REMAP_ROWS rows
 #ifndef FV_REMAP_ROWS
 #define FV_REMAP_ROWS 2
 #endif
 constexpr int REMAP_ROWS = FV_REMAP_ROWS;
 __host__ __device__ inline int remap_rows_blocks(int jnum) { return (jnum + 4 * REMAP_ROWS - 1) / (4 * REMAP_ROWS); }
-// mode: 0 RK stage rhs, 1 last stage with the final combination, 2 end-of-step evaluation
+// batch launchers: ntiles blocks over the tile list; rows = strip rows of the list
+// mode: 0 RK stage rhs, 1 last stage with the final combination (nk slopes in
+// their stage sums), 2 end-of-step evaluation
 void launch_rhs_multi(const RhsEntry *tab, const unsigned *tiles, int ntiles, int V, int dtype, int limiter,
-                      int tx, int stages, int mode, hipStream_t s);
+                      int rows, int mode, int nk, hipStream_t s);
 void launch_remap_multi(const RemapEntry *tab, const unsigned *tiles, int ntiles, int V, int dtype, hipStream_t s);
 void launch_control_multi(const ControlEntry *tab, int n, hipStream_t s);
 // batches with point-mass accretion: the step's boundary-flux accumulation

@@ -14,7 +14,7 @@
 //
 // Citations are file:line in the fosite source tree.
 //
-// k_rhs (one launch per right-hand-side evaluation) is fully fused:
+// k_rhs (one launch per right-hand-side evaluation, fv_strip.h) is fully fused:
 //   * the input state of every loaded cell is formed on the fly: the RK stage
 //     state Y - sum a*dt*k (timedisc_rkfehlberg.f90:277-302);
 //   * ghost cells are evaluated on the fly from interior cells with the
@@ -60,10 +60,46 @@ template <typename T>
 __device__ __forceinline__ T fsign(T a, T b) { return copysign(fabs(a), b); }
 template <typename T>
 __device__ __forceinline__ bool bad(T x) { return (x != x) || (x > Real<T>::huge); }
-// division, square root, log, exp: IEEE in FP64; hardware-rate in FP32
-__device__ __forceinline__ double dv(double a, double b) { return a / b; }
+// minimum and maximum as one instruction each: NaN-dropping like fmin2/fmax2
+// with a number as first argument (only the sign of a zero may differ)
+__device__ __forceinline__ double mn(double a, double b) { return __builtin_fmin(a, b); }
+__device__ __forceinline__ float mn(float a, float b) { return __builtin_fminf(a, b); }
+__device__ __forceinline__ double mx(double a, double b) { return __builtin_fmax(a, b); }
+__device__ __forceinline__ float mx(float a, float b) { return __builtin_fmaxf(a, b); }
+// division, square root, log, exp: correctly rounded in FP64; hardware-rate
+// in FP32.
+//
+// The FP64 quotient dv is Newton's iteration on the hardware reciprocal with
+// Markstein's final correction (P. Markstein, IBM J. Res. Dev. 34, 1990): a/b
+// rounds as IEEE division does while the operands, the quotient and the
+// residual a - b*q (2^-53 of a) stay in the normal range.  It leaves out the
+// rescaling of extreme exponents and the special-case fix-up (3 of 11
+// instructions, 12 of about 56 issue cycles); an infinite or zero divisor
+// gives NaN where IEEE gives 0 or Inf, both of which the data checks and the
+// error norm treat alike.  Densities, pressures, sound speeds and wave speeds
+// take it; quotients of differences, which do reach the subnormal range ahead
+// of a signal, take dvx or the guarded forms below.
+__device__ __forceinline__ double dv(double a, double b) {
+  double y = __builtin_amdgcn_rcp(b);
+  y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+  y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+  const double q = a * y;
+  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
 __device__ __forceinline__ float dv(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
-__device__ __forceinline__ double sq(double a) { return sqrt(a); }
+__device__ __forceinline__ double dvx(double a, double b) { return a / b; }
+__device__ __forceinline__ float dvx(float a, float b) { return dv(a, b); }
+// Goldschmidt's iteration on the hardware reciprocal square root with two
+// final corrections (the same source), for a > 2*tiny
+__device__ __forceinline__ double sq(double a) {
+  const double y = __builtin_amdgcn_rsq(a);
+  double s = a * y, h = 0.5 * y;
+  const double r = __builtin_fma(-h, s, 0.5);
+  s = __builtin_fma(s, r, s);
+  h = __builtin_fma(h, r, h);
+  s = __builtin_fma(__builtin_fma(-s, s, a), h, s);
+  return __builtin_fma(__builtin_fma(-s, s, a), h, s);
+}
 __device__ __forceinline__ float sq(float a) { return __builtin_amdgcn_sqrtf(a); }
 __device__ __forceinline__ double lg(double a) { return log(a); }
 __device__ __forceinline__ float lg(float a) { return __logf(a); }
@@ -129,10 +165,17 @@ __device__ __forceinline__ void p2c(const T *p, T *u, T gamma) {
   u[2] = p[0] * p[2];
   if (V == 4) u[3] = dv(p[3], gamma - T(1)) + T(0.5) * p[0] * (p[1] * p[1] + p[2] * p[2]);
 }
-// physics_euler.f90:2682-2689
+// SQRT(MAX(2*TINY, gamma*P/rho)) (physics_euler.f90:2682-2689); FP64: the
+// floor's square root is a constant
 template <typename T>
 __device__ __forceinline__ T sound_speed(T gamma, T rho, T pr) {
-  return sq(fmax2(T(2) * Real<T>::tiny, dv(gamma * pr, rho)));
+  const T x = dv(gamma * pr, rho);
+  if constexpr (sizeof(T) == 8) {
+    const T s = sq(x);
+    return x > T(2) * Real<T>::tiny ? s : T(0x1.6a09e667f3bcdp-511);
+  } else {
+    return sq(fmax2(T(2) * Real<T>::tiny, x));
+  }
 }
 
 // Absorbing boundary in x: characteristic variables from the two edge cells
@@ -140,11 +183,22 @@ __device__ __forceinline__ T sound_speed(T gamma, T rho, T pr) {
 // set to zero, extrapolation into the ghost cells (boundary_absorbing.f90:
 // 114-150).  Isothermal: physics_eulerisotherm.f90:1764-1849, 2027-2085,
 // 2895-2969.  Euler: physics_euler.f90:743-846, 1072-1129 with
-// SetEigenValues, SetCharVars and SetBoundaryData (1d/2d).  i1 is the edge
-// cell, iR the higher-index cell of the pair.
+// SetEigenValues, SetCharVars and SetBoundaryData (1d/2d).
+// Isothermal sound speeds: cs of the edge cell, csf at the west face of the
+// higher-index cell of the pair, cs2 at the edge cell's outer face.
+template <typename C>
+struct AbsorbingSpeeds {
+  C cs, csf, cs2;
+  __device__ __forceinline__ AbsorbingSpeeds(const Geom &g, int east) {
+    const int i1 = east ? GH + g.inum - 1 : GH;
+    cs = rg<C>(g, R_CS, i1);
+    csf = rg<C>(g, R_CSW, east ? i1 : i1 + 1);
+    cs2 = rg<C>(g, east ? R_CSE : R_CSW, i1);
+  }
+};
 template <typename C, int V>
-__device__ __forceinline__ void absorbing_math(const Geom &g, int east, int i1, int iR, C gam, const C *pL,
-                                               const C *pR, C *p) {
+__device__ __forceinline__ void absorbing_math(int east, const AbsorbingSpeeds<C> &as, C gam, const C *pL, const C *pR,
+                                               C *p) {
   const C delta = east ? C(1) : C(-1);
   C p1[V];  // element-wise select keeps both states in registers
 #pragma unroll
@@ -153,9 +207,9 @@ __device__ __forceinline__ void absorbing_math(const Geom &g, int east, int i1, 
     const C rho1 = p1[0], u1 = p1[1], v1 = p1[2], P1 = p1[3];
     const C cs = sound_speed(gam, rho1, P1);
     const C lam0 = u1 - cs, lam1 = u1, lam3 = u1 + cs;
-    const C dlnP = lg(dv(pR[3], pL[3]));
-    const C gammadu_cs = dv(C(2) * gam * (pR[1] - pL[1]), lam3 - lam0);
-    C x0 = dlnP - gammadu_cs, x1 = dlnP - gam * lg(dv(pR[0], pL[0])), x2 = pR[2] - pL[2];
+    const C dlnP = lg(dvx(pR[3], pL[3]));
+    const C gammadu_cs = dvx(C(2) * gam * (pR[1] - pL[1]), lam3 - lam0);
+    C x0 = dlnP - gammadu_cs, x1 = dlnP - gam * lg(dvx(pR[0], pL[0])), x2 = pR[2] - pL[2];
     C x3 = dlnP + gammadu_cs;
     if (east) {
       if (lam0 <= C(0)) x0 = C(0);
@@ -167,19 +221,19 @@ __device__ __forceinline__ void absorbing_math(const Geom &g, int east, int i1, 
       if (lam3 >= C(0)) x3 = C(0);
     }
     const C dlp = C(0.5) * (x3 + x0);
-    const C rho2 = rho1 * ex(dv(delta, gam) * (dlp - x1));
+    const C rho2 = rho1 * ex(dvx(delta, gam) * (dlp - x1));
     const C P2 = P1 * ex(delta * dlp);
     const C cs2 = sound_speed(gam, rho1 + rho2, P1 + P2);
     p[0] = rho2;
-    p[1] = u1 + dv(C(0.5) * delta * cs2, gam) * (x3 - x0);
+    p[1] = u1 + dvx(C(0.5) * delta * cs2, gam) * (x3 - x0);
     p[2] = v1 + delta * x2;
     p[3] = P2;
   } else {
-    const C cs = rg<C>(g, R_CS, i1), u1 = p1[1];
+    const C cs = as.cs, u1 = p1[1];
     const C lam0 = u1 - cs, lam1 = u1, lam2 = u1 + cs;
-    const C csf = rg<C>(g, R_CSW, iR);
-    const C dlnrho = lg(dv(pR[0], pL[0]));
-    const C ducs = dv(pR[1] - pL[1], csf);
+    const C csf = as.csf;
+    const C dlnrho = lg(dvx(pR[0], pL[0]));
+    const C ducs = dvx(pR[1] - pL[1], csf);
     C x0 = dlnrho - ducs, x1 = pR[2] - pL[2], x2 = dlnrho + ducs;
     if (east) {
       if (lam0 <= C(0)) x0 = C(0);
@@ -190,7 +244,7 @@ __device__ __forceinline__ void absorbing_math(const Geom &g, int east, int i1, 
       if (lam1 >= C(0)) x1 = C(0);
       if (lam2 >= C(0)) x2 = C(0);
     }
-    const C cs2 = rg<C>(g, east ? R_CSE : R_CSW, i1);
+    const C cs2 = as.cs2;
     p[0] = p1[0] * ex(delta * C(0.5) * (x2 + x0));
     p[1] = u1 + delta * C(0.5) * cs2 * (x2 - x0);
     p[2] = p1[2] + delta * x1;
@@ -214,8 +268,9 @@ __device__ __forceinline__ void frame_sub(T *u, T w) {
 
 // ------------------------------------------------------------ input state
 // KM: coefficient slots of the tableau (3 for up to three stages, else MAXK);
-// loops over stages are unrolled to KM with run-time guards on nk
-template <typename T, int V, int KM>
+// loops over stages are unrolled to KM with run-time guards on nk, or with
+// EXACT over exactly KM slopes
+template <typename T, int V, int KM, bool EXACT = false>
 struct In {
   const Geom &g;
   const StageArgsT<T> &a;
@@ -228,9 +283,9 @@ struct In {
   double c[sizeof(T) == 8 ? KA : 1];
   float ch[sizeof(T) == 4 ? KA : 1];
 
-  __forceinline__ __device__ In(const Geom &g_, const StageArgsT<T> &a_, bool chk_) : g(g_), a(a_), chk(chk_) {
-    dt = a.ctl ? a.ctl->dt : a.dt;  // device-controlled: this step's dt
-    nk = a.nk;
+  __forceinline__ __device__ In(const Geom &g_, const StageArgsT<T> &a_, bool chk_, double dt_)
+      : g(g_), a(a_), dt(dt_), chk(chk_) {
+    nk = EXACT ? KM : a.nk;
     gam = (T)g.gamma;
 #pragma unroll
     for (int q = 0; q < KM; q++) {
@@ -322,10 +377,20 @@ struct In {
   // frame change, CenterBoundary and PMIN (real frame), pr = pvar at that
   // point, uc = cvar handed to the fluxes
   __forceinline__ __device__ void transform(int i, const T *s, T *ur, T *pr, T *uc) const {
+    transform_at(rg<T>(g, R_W, i), s, ur, pr, uc);
+  }
+  __forceinline__ __device__ void transform_at(T w, const T *s, T *ur, T *pr, T *uc) const {
+    to_prim(w, s, ur, pr);
+    comoving(w, s, ur, pr, uc);
+  }
+  // real frame: cvar and pvar right after CenterBoundary's conversion
+  __forceinline__ __device__ void to_prim(T w, const T *s, T *ur, T *pr) const {
 #pragma unroll
     for (int l = 0; l < V; l++) ur[l] = s[l];
-    if (a.add_bg) frame_add<T, V>(ur, rg<T>(g, R_W, i));
+    if (a.add_bg) frame_add<T, V>(ur, w);
     c2p<T, V>(ur, pr, gam);
+  }
+  __forceinline__ __device__ void comoving(T w, const T *s, T *ur, T *pr, T *uc) const {
     if (V == 4 && a.pmin_clamp) {
       pr[3] = fmax2(pr[3], (T)g.pmin);
       p2c<T, V>(pr, ur, gam);
@@ -336,24 +401,24 @@ struct In {
       // FP32 (isothermal only): m' + rho*w - rho*w would cancel to a few
       // bits of the residual momentum m'; the stored residual is what the
       // subtraction means
-      if (a.sub_bg) uc[2] = a.add_bg ? s[2] : ur[2] - ur[0] * rg<T>(g, R_W, i);
+      if (a.sub_bg) uc[2] = a.add_bg ? s[2] : ur[2] - ur[0] * w;
     } else {
-      if (a.sub_bg) frame_sub<T, V>(uc, rg<T>(g, R_W, i));
+      if (a.sub_bg) frame_sub<T, V>(uc, w);
     }
   }
 
   // PRIMITIVE reconstruction: the pvar handed to the reconstruction, after
   // SubtractBackgroundVelocityY (physics_eulerisotherm.f90:1373-1413) of the
   // real-frame pvar p (as transform returns it); s is the stage state
-  __forceinline__ __device__ void prim_comoving(int i, const T *s, const T *p, T *po) const {
+  __forceinline__ __device__ void prim_comoving(T w, const T *s, const T *p, T *po) const {
 #pragma unroll
     for (int l = 0; l < V; l++) po[l] = p[l];
     if constexpr (sizeof(T) == 4) {
       // FP32: (v' + w) - w would keep a few bits of the residual velocity v';
       // the stored residual is what the subtraction means
-      if (a.sub_bg) po[2] = a.add_bg ? dv(s[2], s[0]) : p[2] - rg<T>(g, R_W, i);
+      if (a.sub_bg) po[2] = a.add_bg ? dv(s[2], s[0]) : p[2] - w;
     } else {
-      if (a.sub_bg) po[2] = p[2] - rg<T>(g, R_W, i);
+      if (a.sub_bg) po[2] = p[2] - w;
     }
   }
 
@@ -373,7 +438,7 @@ struct In {
     T pL[V], pR[V];
     prim_interior(iL, j, pL);
     prim_interior(iR, j, pR);
-    absorbing_math<T, V>(g, east, i1, iR, gam, pL, pR, p);
+    absorbing_math<T, V>(east, AbsorbingSpeeds<T>(g, east), gam, pL, pR, p);
   }
 
   // x-ghost (side, layer 1..2) at interior row j
@@ -427,6 +492,9 @@ struct In {
   // final ghost state: PMIN round trip, prim->cons, data check, frame change
   __forceinline__ __device__ void ghost_final(int i, int j, T *u, T *p, int &flags) const {
     ghost_prim(i, j, p);
+    ghost_from_prim(rg<T>(g, R_W, i), p, u, flags);
+  }
+  __forceinline__ __device__ void ghost_from_prim(T w, T *p, T *u, int &flags) const {
     if (V == 4 && a.pmin_clamp) p[3] = fmax2(p[3], (T)g.pmin);
     p2c<T, V>(p, u, gam);
     if (chk) {
@@ -435,7 +503,6 @@ struct In {
         if (bad(u[l]) || bad(p[l])) flags |= F_INVALID;
     }
     if (a.sub_bg) {
-      const T w = rg<T>(g, R_W, i);
       p[2] = p[2] - w;
       frame_sub<T, V>(u, w);
     }
@@ -445,10 +512,14 @@ struct In {
 // CFL contribution of one cell (timedisc_base.f90:869-872 with
 // physics_eulerisotherm.f90:530-552); u, v = pvar after the frame change back
 template <typename T>
+__device__ __forceinline__ T cell_invdt(T dlx, T dly, T u, T v, T cs) {
+  const T mnx = mn(T(0), u - cs), mxx = mx(T(0), u + cs);
+  const T mny = mn(T(0), v - cs), mxy = mx(T(0), v + cs);
+  return dv(mx(mxx, -mnx), dlx) + dv(mx(mxy, -mny), dly);
+}
+template <typename T>
 __device__ __forceinline__ T cell_invdt(const Geom &g, int i, T u, T v, T cs) {
-  const T mnx = fmin2(T(0), u - cs), mxx = fmax2(T(0), u + cs);
-  const T mny = fmin2(T(0), v - cs), mxy = fmax2(T(0), v + cs);
-  return dv(fmax2(mxx, -mnx), rg<T>(g, R_DLX, i)) + dv(fmax2(mxy, -mny), rg<T>(g, R_DLY, i));
+  return cell_invdt<T>(rg<T>(g, R_DLX, i), rg<T>(g, R_DLY, i), u, v, cs);
 }
 
 // ------------------------------------------------------------ reductions
@@ -504,16 +575,16 @@ static __device__ int blk_or(int v, int *red) {
 // ----------------------------------------------------------- reconstruction
 // limiters, reconstruction_linear.f90:645-733
 // LIM = 0: limiter chosen at run time from g.limiter
+// a1, a2: differences to the lower and the higher neighbour um, up
 template <typename T, int LIM>
-__device__ __forceinline__ T slope(const Geom &g, T um, T u0, T up) {
-  const T a1 = u0 - um, a2 = up - u0;
+__device__ __forceinline__ T limited(const Geom &g, T a1, T a2, T um, T up) {
   const T one = T(1), zero = T(0), tiny = Real<T>::tiny;
   switch (LIM ? LIM : g.limiter) {
     case MINMOD:
       return (fsign(one, a1) * fsign(one, a2) > zero) ? fsign(fmin2(fabs(a1), fabs(a2)), a1) : zero;
     case MONOCENT: {
       const T th = (T)g.theta;
-      const T b1 = th * (u0 - um), b2 = th * (up - u0), b3 = T(0.5) * (up - um);
+      const T b1 = th * a1, b2 = th * a2, b3 = T(0.5) * (up - um);
       if ((fsign(one, b1) * fsign(one, b2) > zero) && (fsign(one, b2) * fsign(one, b3) > zero))
         return fsign(fmin2(fmin2(fabs(b1), fabs(b2)), fabs(b3)), b1);
       return zero;
@@ -526,14 +597,45 @@ __device__ __forceinline__ T slope(const Geom &g, T um, T u0, T up) {
                  : zero;
     }
     case OSPRE:
-      return dv(T(1.5) * a1 * a2 * (a1 + a2), a1 * (a1 + T(0.5) * a2) + a2 * (a2 + T(0.5) * a1) + tiny);
+      return dvx(T(1.5) * a1 * a2 * (a1 + a2), a1 * (a1 + T(0.5) * a2) + a2 * (a2 + T(0.5) * a1) + tiny);
     case VANLEER: {
       const T b1 = fabs(a1), b2 = fabs(a2);
-      return dv(a1 * b2 + a2 * b1, b1 + b2 + tiny);
+      return dvx(a1 * b2 + a2 * b1, b1 + b2 + tiny);
     }
     default:
       return T(0.5) * (a1 + a2);
   }
+}
+
+// V limited slopes at once.  Van Leer in FP64 divides with dv, which is exact
+// while no numerator has bits below the subnormal limit; the return value is
+// the least binary exponent of the non-zero numerators (frexp's), and below
+// SLOPE_EXACT the caller takes slopes_exact.
+constexpr int SLOPE_EXACT = -960;
+template <typename T, int V, int LIM>
+__device__ __forceinline__ int slopes(const Geom &g, const T *a1, const T *a2, const T *um, const T *up, T *s) {
+  int t = 0;
+#pragma unroll
+  for (int l = 0; l < V; l++) {
+    if constexpr (LIM == VANLEER && sizeof(T) == 8) {
+      const T b1 = fabs(a1[l]), b2 = fabs(a2[l]), num = a1[l] * b2 + a2[l] * b1;
+      t = min(t, __builtin_amdgcn_frexp_exp(num));
+      s[l] = dv(num, b1 + b2 + Real<T>::tiny);
+    } else {
+      s[l] = limited<T, LIM>(g, a1[l], a2[l], um[l], up[l]);
+    }
+  }
+  return t;
+}
+template <typename T, int V, int LIM>
+__device__ __forceinline__ void slopes_exact(const Geom &g, const T *a1, const T *a2, const T *um, const T *up, T *s) {
+#pragma unroll
+  for (int l = 0; l < V; l++) s[l] = limited<T, LIM>(g, a1[l], a2[l], um[l], up[l]);
+}
+// whether some lane needs the exact form (compile-time false where none can)
+template <typename T, int LIM>
+__device__ __forceinline__ bool any_exact(int t) {
+  return LIM == VANLEER && sizeof(T) == 8 && __any(t < SLOPE_EXACT);
 }
 
 // KT flux across one interface from the two face states (fluxes_kt.f90:126-176,
@@ -550,8 +652,8 @@ __device__ __forceinline__ void kt_core(const Geom &g, int d, const T *UL, const
     csR = sound_speed(gam, pr[0], pr[3]);
   }
   const T vL = pl[un], vR = pr[un];
-  const T amin = fmin2(fmin2(zero, fmin2(zero, vR - csR)), fmin2(zero, vL - csL));
-  const T amax = fmax2(fmax2(zero, fmax2(zero, vR + csR)), fmax2(zero, vL + csL));
+  const T amin = mn(mn(zero, vR - csR), vL - csL);
+  const T amax = mx(mx(zero, vR + csR), vL + csL);
   T fL[V], fR[V];
   fL[0] = pl[0] * vL;
   fR[0] = pr[0] * vR;
@@ -594,20 +696,20 @@ __device__ __forceinline__ void kt_flux_p(const Geom &g, int d, const T *PL, con
 // ------------------------------------------------------------ step control
 // PI controller (timedisc_base.f90:759-814), used on the device only to stop
 // a batch when the step could fall under dtlimit; the host redoes such steps
-static __device__ double pi_dtnew(const Ctl *c, double maxerr, double dtold) {
+static __device__ double pi_dtnew(const CtlHead *c, double maxerr, double dtold) {
   double dttmp = maxerr > 0. ? 0.9 * dtold * exp(-log(maxerr) / c->order) : 4. * dtold;
   double dtnew = c->maxerrold > 0. ? dttmp * exp(-c->beta * log(c->maxerrold / maxerr)) : dttmp;
   if (maxerr < 1.0 && 4. * dtold < dtnew) dtnew = 4. * dtold;
   return dtnew;
 }
-static __device__ void halt(Ctl *c, int reason) {
+static __device__ void halt(CtlHead *c, int reason) {
   c->halt = 1;
   c->reason = reason;
 }
 // A lower bound of pi_dtnew for an accepted step (0 <= err < 1) without
 // exp/log: err^(-1/order) >= 1, and (maxerrold/err)^(-beta) >= min(1,
 // err/maxerrold) for 0 <= beta <= 1; other beta take the exact form
-static __device__ double pi_dtnew_lower(const Ctl *c, double err, double dtold) {
+static __device__ double pi_dtnew_lower(const CtlHead *c, double err, double dtold) {
   if (!(c->beta >= 0.0 && c->beta <= 1.0 && c->order > 0.0)) return pi_dtnew(c, err, dtold);
   const double f = (c->maxerrold > 0. && err < c->maxerrold) ? err / c->maxerrold : 1.0;
   return 0.9 * dtold * f;
@@ -615,10 +717,7 @@ static __device__ double pi_dtnew_lower(const Ctl *c, double err, double dtold) 
 // after SolveODE: accept when the embedded error is finite and < 1
 // (timedisc_base.f90:686-713, AcceptSolution 911-959); halt when the next
 // step could fall under dtlimit (the host redoes such a step exactly)
-static __device__ void control_accept(Ctl *c, double err) {
-  const int s = c->step;
-  c->err_hist[s] = err;
-  c->dt_hist[s] = c->dt;
+static __device__ void control_accept(CtlHead *c, double err) {
   if (!(err < 1.0)) return halt(c, H_ERR);  // NaN, Inf or a rejection
   if (pi_dtnew_lower(c, err, c->dt) < c->dtlimit * (1.0 + 1.0e-6)) return halt(c, H_DTLIMIT);
   c->maxerrold = err;
@@ -629,7 +728,7 @@ static __device__ void control_accept(Ctl *c, double err) {
 // after the end-of-step RHS: data checks, output test, next CFL step,
 // stop-time test and output-time clipping (fosite.f90:383-462,
 // io/fileio_base.f90:604-620)
-static __device__ void control_next(Ctl *c, double invdt, int flags, double invdt_v) {
+static __device__ void control_next(CtlHead *c, double invdt, int flags, double invdt_v) {
   if (flags) return halt(c, H_FLAGS);
   const double t = c->time;
   if (fabs(c->t_out - t) <= 1.0E-5 * c->t_out) return halt(c, H_OUTPUT);
@@ -651,47 +750,54 @@ static __device__ void control_next(Ctl *c, double invdt, int flags, double invd
 }
 
 // ------------------------------------------------ boundary-flux accounting
-// Element e of the boundary rows (west/east rows of every field first, then
-// south/north): its new bxflux(j,side,l) / byflux(i,side,l) after one step
-// (timedisc_rkfehlberg.f90:216-259), and in *bi its index in the layout.
-__device__ __forceinline__ double bflux_elem(const BfluxArgs &b, double dt, int e, long *bi) {
-  const int nx = b.V * 2 * b.jnum;
-  int l, side, gx;
-  if (e < nx) {  // west / east: ghost column IMIN-1 / IMAX+1 of row j
-    l = e / (2 * b.jnum);
-    side = (e / b.jnum) & 1;
-    const int j = GH + e % b.jnum;
-    *bi = (long)(l * 2 + side) * b.NJ + j;
-    gx = j * b.P + (side ? GH + b.inum : GH - 1);
-  } else {       // south / north: ghost row JMIN-1 / JMAX+1 of column i
-    const int f = e - nx;
-    l = f / (2 * b.inum);
-    side = (f / b.inum) & 1;
-    const int i = GH + f % b.inum;
-    *bi = 2L * b.V * b.NJ + (long)(l * 2 + side) * b.NI + i;
-    gx = (side ? GH + b.jnum : GH - 1) * b.P + i;
+// One element of the boundary rows (west/east rows of every field first, then
+// south/north): loaded, then its new bxflux(j,side,l) / byflux(i,side,l) after
+// one step (timedisc_rkfehlberg.f90:216-259) stored.
+struct BfluxElem {
+  long bi;  // its index in the layout
+  double kq[MAXK], in, ks;
+  __device__ __forceinline__ void load(const BfluxArgs &b, int e) {
+    const int nx = b.V * 2 * b.jnum;
+    int l, side, gx;
+    if (e < nx) {  // west / east: ghost column IMIN-1 / IMAX+1 of row j
+      l = e / (2 * b.jnum);
+      side = (e / b.jnum) & 1;
+      const int j = GH + e % b.jnum;
+      bi = (long)(l * 2 + side) * b.NJ + j;
+      gx = j * b.P + (side ? GH + b.inum : GH - 1);
+    } else {       // south / north: ghost row JMIN-1 / JMAX+1 of column i
+      const int f = e - nx;
+      l = f / (2 * b.inum);
+      side = (f / b.inum) & 1;
+      const int i = GH + f % b.inum;
+      bi = 2L * b.V * b.NJ + (long)(l * 2 + side) * b.NI + i;
+      gx = (side ? GH + b.jnum : GH - 1) * b.P + i;
+    }
+    const long kx = (long)l * b.FS + gx;
+#pragma unroll
+    for (int q = 0; q < MAXK; q++)  // all loads first
+      if (q < b.nk)
+        kq[q] = b.dtype == 1 ? (double)static_cast<const float *>(b.k[q])[kx] : static_cast<const double *>(b.k[q])[kx];
+    in = b.in[bi];
+    ks = b.ks[bi];
   }
-  double kq[MAXK];
-  const long kx = (long)l * b.FS + gx;
+  __device__ __forceinline__ void store(const BfluxArgs &b, double dt) const {
+    double acc = in;
 #pragma unroll
-  for (int q = 0; q < MAXK; q++)  // all loads first
-    if (q < b.nk)
-      kq[q] = b.dtype == 1 ? (double)static_cast<const float *>(b.k[q])[kx] : static_cast<const double *>(b.k[q])[kx];
-  double acc = b.in[*bi];
-  const double ks = b.ks[*bi];
-#pragma unroll
-  for (int q = 0; q < MAXK; q++)
-    if (q < b.nk) acc = acc - (dt * b.bh[q]) * kq[q];
-  return acc - (dt * b.bh[b.nk]) * ks;
-}
+    for (int q = 0; q < MAXK; q++)
+      if (q < b.nk) acc = acc - (dt * b.bh[q]) * kq[q];
+    b.out[bi] = acc - (dt * b.bh[b.nk]) * ks;
+  }
+};
 // the whole accumulation: threads t, t+nt, ... of the caller each take one
 // boundary row element
+__device__ __forceinline__ int bflux_elems(const BfluxArgs &b) { return b.V * 2 * (b.jnum + b.inum); }
 __device__ __forceinline__ void bflux_accumulate(const BfluxArgs &b, double dt, int t, int nt) {
-  const int n = b.V * 2 * (b.jnum + b.inum);
+  const int n = bflux_elems(b);
   for (int e = t; e < n; e += nt) {
-    long bi;
-    const double v = bflux_elem(b, dt, e, &bi);
-    b.out[bi] = v;
+    BfluxElem x;
+    x.load(b, e);
+    x.store(b, dt);
   }
 }
 
@@ -767,628 +873,192 @@ __device__ __forceinline__ void accrete_update(const AccreteArgs &p, double sum,
 // Workgroup b of a launch is dispatched to XCD b mod 8.  A 1-D grid of
 // 8*Q blocks (Q = ceil(tiles/8)) whose block b runs tile (b mod 8)*Q + b/8
 // gives every XCD a contiguous, row-major run of tiles, so tiles that share
-// halo rows share that XCD's L2.  Returns false for the padding blocks.
+// halo rows share that XCD's L2.  Padding blocks get a tile >= n.
 constexpr int XCDS = 8;
-__device__ __forceinline__ bool xcd_tile(int b, int nbx, int nby, int &bx, int &by) {
-  const int n = nbx * nby, q = (n + XCDS - 1) / XCDS, t = (b % XCDS) * q + b / XCDS;
-  if (t >= n) return false;
-  bx = t % nbx;
-  by = t / nbx;
-  return true;
-}
-inline int xcd_grid(int nbx, int nby) { return ((nbx * nby + XCDS - 1) / XCDS) * XCDS; }
+__device__ __forceinline__ int xcd_tile(int b, int n) { return (b % XCDS) * ((n + XCDS - 1) / XCDS) + b / XCDS; }
+__host__ __device__ inline int xcd_grid(int n) { return ((n + XCDS - 1) / XCDS) * XCDS; }
 
-// -------------------------------------------------------------- fused RHS
-// Tile: TX x TY_RHS output cells (TX = 64 or 32), one thread each.  The
-// footprint (2-cell halo, corners excluded) is staged in LDS as the state the
-// fluxes see; threads with an extra job cover the halo cells and the faces
-// and fluxes one cell beyond the tile.  Phases, separated by barriers:
-//   1 stage state + transform of the own and one extra footprint cell (ghost
-//     cells on boundary tiles), sources, data checks and CFL of the own cell
-//   2 limited slopes and face states: own cell; rows -1 and TY; columns -1, TX
-//   3 KT interface fluxes: own east and north interfaces; west of column 0,
-//     south of row 0
-//   4 rhs assembly, or the final RK combination in the last stage; stores
-// Faces live in their own LDS region; the fluxes reuse the footprint region,
-// which is dead after phase 2, so three barriers separate the four phases.
-// Output-aligned tiles keep every lane of the flux phases busy and divide
-// power-of-two meshes exactly.
-//
-// Occupancy: a CU has 160 KB of LDS, allocated in 512-byte granules.  The
-// FP64 isothermal stage tiles (64 x 8, V = 3) take 54444 bytes, 107
-// granules, so two tiles share a CU (4 waves per SIMD); the launch bounds
-// compute that from the layout.  The ghost-cell CFL and flag arrays only
-// exist in the end-of-step mode.
-constexpr int TY_RHS = TY_TILE;
+// -------------------------------------------------------------- RHS pieces
 // launch modes of the RHS kernel
 enum RhsMode { M_STAGE = 0, M_LAST = 1, M_END = 2 };
-// LDS bytes of one tile (the layout rhs_tile declares)
-template <typename T, int V, int TX>
-constexpr int rhs_lds_words() {
-  constexpr int TY = TY_RHS, SX = TX + 4, SY = TY + 4;
-  constexpr int N_UC = V * SY * SX, N_FLUX = V * TY * (TX + 1) + V * (TY + 1) * TX;
-  constexpr int N_FACE = V * TY * (TX + 1) + V * TY + V * (TY + 1) * TX + V * TX;
-  return (N_UC > N_FLUX ? N_UC : N_FLUX) + N_FACE;
-}
-// LDS bytes of one tile, rounded to the 512-byte allocation granule
-template <typename T, int V, int TX>
-constexpr int rhs_lds_bytes() {
-  return ((int)sizeof(T) * rhs_lds_words<T, V, TX>() + 12 * TY_RHS + 511) / 512 * 512;
-}
-// waves per SIMD the launch bounds ask for: the FP64 stage kernels of up to
-// three stages fit 80 VGPRs without spilling, so they take as many waves as
-// the tiles' LDS lets share a CU (160 KB), at most 6; everything else 4
-template <typename T, int V, int TX, int KM, int MODE>
-constexpr int rhs_waves_per_simd() {
-#ifdef FV_RHS_WAVES_PER_SIMD
-  return FV_RHS_WAVES_PER_SIMD;
-#else
-  if (!(sizeof(T) == 8 && V == 3 && KM <= 3 && MODE != M_END)) return 4;
-  constexpr int w = (163840 / rhs_lds_bytes<T, V, TX>()) * (TX * TY_RHS / 64) / 4;
-  return w < 4 ? 4 : (w > 6 ? 6 : w);
-#endif
+template <typename T>
+__host__ __device__ inline int rhs_aux(const Geom &g, const StageArgsT<T> &a) {
+  return a.bfa.out ? rhs_aux_max(g, a.bfa.V) : 1;
 }
 template <typename T>
 inline int rhs_mode(const StageArgsT<T> &a) { return a.ynew ? M_LAST : (a.nk == 0 ? M_END : M_STAGE); }
 
-// one TX x TY tile (bx, by) of a mesh tiled nbx x nby
-template <typename T, int V, int LIM, int TX, int KM, int MODE>
-__device__ __forceinline__ void rhs_tile(const Geom &g, const StageArgsT<T> &a, int bx, int by, int nbx,
-                                         int nby) {
-  // what this launch does, fixed at compile time (the run-time flags of the
-  // arguments still apply within it): RK stage rhs, last stage with the
-  // final combination, or the end-of-step evaluation (no stage sum; CFL,
-  // data checks, new state, FARGO type-1 velocities, boundary fluxes)
-  constexpr bool kEnd = MODE == M_END, kLast = MODE == M_LAST;
-  constexpr int KE = kEnd ? 0 : KM;
-  const bool want_cfl = kEnd && a.want_cfl, want_check = kEnd && a.want_check;
-  T *const yout = kEnd ? a.yout : nullptr;
-  T *const pout = kEnd ? a.pout : nullptr;
-  double *const vout = kEnd ? a.vout : nullptr;
-  T *const ynew = kLast ? a.ynew : nullptr;
-  constexpr int TY = TY_RHS, SX = TX + 4, SY = TY + 4;
-  // the threads with an extra footprint cell cover rows -2, -1, TY, TY+1 and
-  // columns -2, -1, TX, TX+1
-  static_assert(TX * TY >= 4 * TX + 4 * TY, "tile too small for its halo jobs");
-  constexpr int N_UC = V * SY * SX;
-  constexpr int XW = V * TY * (TX + 1), XE = V * TY, YS = V * (TY + 1) * TX, YN = V * TX;
-  constexpr int N_FACE = XW + XE + YS + YN;
-  constexpr int FX = V * TY * (TX + 1), FY = V * (TY + 1) * TX;
-  constexpr int N_FLUX = FX + FY;
-  // region A: footprint state (phases 1-2), then fluxes (phases 3-4);
-  // region B: face states (phases 2-3)
-  constexpr int NA = N_UC > N_FLUX ? N_UC : N_FLUX;
-  __shared__ T lds[rhs_lds_words<T, V, TX>()];
-  static_assert(NA + N_FACE == rhs_lds_words<T, V, TX>(), "LDS layout");
-  __shared__ double redd[TY];
-  __shared__ int redi[TY];
-  // CFL term and check flags of the ghost cells a thread evaluated (kept in
-  // LDS rather than registers across the interior path)
-  __shared__ T gcfl[kEnd ? TX * TY : 1];
-  __shared__ int gflg[kEnd ? TX * TY : 1];
-  // footprint state, tile-relative row r in [-2, TY+1], column c in [-2, TX+1]
-  auto UC = [&](int l, int r, int c) -> T & { return lds[(l * SY + r + 2) * SX + c + 2]; };
-  // faces: W of columns 0..TX, E of column -1, S of rows 0..TY, N of row -1
-  T *fb = lds + NA;
-  auto FW = [&](int l, int r, int c) -> T & { return fb[(l * TY + r) * (TX + 1) + c]; };
-  auto FE1 = [&](int l, int r) -> T & { return fb[XW + l * TY + r]; };
-  auto FS = [&](int l, int r, int c) -> T & { return fb[XW + XE + (l * (TY + 1) + r) * TX + c]; };
-  auto FN1 = [&](int l, int c) -> T & { return fb[XW + XE + YS + l * TX + c]; };
-  // fluxes: x interface c-1/2 (c = 0..TX) of row r; y interface r-1/2 (r = 0..TY) of column c
-  auto FLX = [&](int l, int r, int c) -> T & { return lds[(l * TY + r) * (TX + 1) + c]; };
-  auto FLY = [&](int l, int r, int c) -> T & { return lds[FX + (l * (TY + 1) + r) * TX + c]; };
-
-  if (a.ctl && a.ctl->halt) return;
-  // PRIMITIVE reconstruction: the footprint and the face states hold pvar
-  // (only the run-time-limiter instantiation carries this path)
-  const bool prim_rec = LIM == 0 && g.recon_prim;
-  const In<T, V, KE> in(g, a, want_check);
-  const int tx = threadIdx.x, ty = threadIdx.y, t = tx + TX * ty;
-  const int i0 = GH + bx * TX, j0 = GH + by * TY;
-  const int imin = GH, jmin = GH, imax = GH + g.inum - 1, jmax = GH + g.jnum - 1;
-  const int i = i0 + tx, j = j0 + ty;
-  const bool out = i <= imax && j <= jmax;  // own cell is an interior cell
-  const T zero = T(0);
-
-  // ---- phase 1: footprint state into LDS
-  // extra footprint cell: rows -2,-1,TY,TY+1 of the own column (t < 4*TX),
-  // then columns -2,-1,TX,TX+1 of rows 0..TY-1 (next 4*TY threads)
-  int er = 0, ec = 0;
-  bool has_e = false;
-  if (t < 4 * TX) {
-    er = ty < 2 ? ty - 2 : TY + ty - 2;
-    ec = tx;
-    has_e = true;
-  } else if (t < 4 * TX + 4 * TY) {
-    const int k = t - 4 * TX, q = k / TY;
-    ec = q < 2 ? q - 2 : TX + q - 2;
-    er = k % TY;
-    has_e = true;
-  }
-  const int ei = i0 + ec, ej = j0 + er;
-  const bool e_in = has_e && ei >= imin && ei <= imax && ej >= jmin && ej <= jmax;
-  // ghost cells or cells beyond the mesh (boundary tiles only) first, so that
-  // no value of the interior path is live across this register-hungry code.
-  // Every non-corner ghost cell of the mesh lies in some tile's footprint, so
-  // the ghost part of the data checks and of the CFL reduction (ghosts
-  // included, timedisc_base.f90:869-872) and the ghost cells of the new state
-  // are produced here; a cell seen by two tiles contributes identical values.
-  const bool own_g = !out, e_g = has_e && !e_in;
-  if (own_g || e_g) {
-    T ginv = -Real<T>::huge;
-    int gf = 0;
-#pragma unroll
-    for (int p = 0; p < 2; p++) {
-      if (!(p ? e_g : own_g)) continue;
-      const int ii = p ? ei : i, jj = p ? ej : j;
-      const bool xin = ii >= imin && ii <= imax, yin = jj >= jmin && jj <= jmax;
-      T u[V], pp[V];
-      if ((xin || yin) && ii >= 0 && jj >= 0 && ii < g.NI && jj < g.NJ) {
-        in.ghost_final(ii, jj, u, pp, gf);
-        if (want_cfl) {
-          const T cs = (V == 4) ? sound_speed(in.gam, pp[0], pp[3]) : rg<T>(g, R_CS, ii);
-          ginv = fmax2(ginv, cell_invdt(g, ii, pp[1], pp[2], cs));
-        }
-        if (yout) {
-          const unsigned ix = (unsigned)jj * (unsigned)g.P + (unsigned)ii;
-#pragma unroll
-          for (int l = 0; l < V; l++) (yout + l * g.FS)[ix] = u[l];
-        }
-        if (pout) {
-          const unsigned ix = (unsigned)jj * (unsigned)g.P + (unsigned)ii;
-#pragma unroll
-          for (int l = 0; l < V; l++) (pout + l * g.FS)[ix] = pp[l];
-        }
-        if (vout && yin) {  // x-ghost ring of an interior row: (v - w) + w
-          const T w = rg<T>(g, R_W, ii), vc = a.sub_bg ? pp[2] : pp[2] - w;
-          vout[(unsigned)jj * (unsigned)g.P + (unsigned)ii] = (double)(vc + w);
-        }
-      } else {
-#pragma unroll
-        for (int l = 0; l < V; l++) u[l] = pp[l] = zero;  // corner or beyond the mesh: never needed
-      }
-#pragma unroll
-      for (int l = 0; l < V; l++) UC(l, p ? er : ty, p ? ec : tx) = prim_rec ? pp[l] : u[l];
-    }
-    if constexpr (kEnd) {
-      gcfl[t] = ginv;
-      gflg[t] = gf;
+// Source terms of the cells of one ring.  Of the commutator coefficients only
+// c_yxy differs from zero on the supported meshes (fv_create checks it).
+template <typename T, int V>
+struct SourceRing {
+  T cs, cyxy, w, dw, dlx, dly, ax, ay, cac;
+  double wd, cyd, accd, cacd;  // FP32: the radial balance in FP64
+  __forceinline__ __device__ SourceRing(const Geom &g, const StageArgsT<T> &a, int i) {
+    const T *acc = sizeof(T) == 4 ? reinterpret_cast<const T *>(a.accf) : reinterpret_cast<const T *>(a.acc);
+    cs = rg<T>(g, R_CS, i);
+    cyxy = rg<T>(g, R_CYXY, i);
+    w = rg<T>(g, R_W, i);
+    dw = rg<T>(g, R_W, i + 1) - rg<T>(g, R_W, i - 1);
+    dlx = rg<T>(g, R_DLX, i);
+    dly = rg<T>(g, R_DLY, i);
+    ax = ay = T(0);
+    if (g.gravity) ax = acc[(unsigned)i], ay = acc[(unsigned)(g.NI + i)];
+    cac = rg<T>(g, R_CACX, i);
+    if constexpr (sizeof(T) == 4) {
+      wd = ring(g, R_W, i);
+      cyd = ring(g, R_CYXY, i);
+      accd = g.gravity ? a.acc[i] : 0.0;
+      cacd = ring(g, R_CACX, i);
     }
   }
-
-  T ur[V], pr[V];
-  T vres = zero;  // FP32: azimuthal velocity of the stored state (residual in the FARGO frame)
-  T ucons[V];     // PRIMITIVE reconstruction: the own cell's cvar for the new state (the footprint holds pvar)
-  {
-    T so[V], se[V], uo[V], ue[V], re[V], pe[V];
-    in.interior2(out, i, j, so, e_in, ei, ej, se);
-    if (out) {
-      in.transform(i, so, ur, pr, uo);
-      if constexpr (sizeof(T) == 4) vres = dv(so[2], so[0]);
-      if (vout) {  // pvar after SubtractBackgroundVelocityY, then + w again
-        const T w = rg<T>(g, R_W, i);
-        vout[(unsigned)j * (unsigned)g.P + (unsigned)i] = (double)((pr[2] - w) + w);
-      }
-      if (pout) {  // pvar after SubtractBackgroundVelocityY
-        const unsigned ix = (unsigned)j * (unsigned)g.P + (unsigned)i;
+  // of the cell in row j: stage state s, real-frame cvar ur and pvar pr; geo
+  // and ext are the reference's geometrical and external sources
+  __forceinline__ __device__ void sources(const Geom &g, const StageArgsT<T> &a, int j, const T *s, const T *ur,
+                                          const T *pr, T *geo, T *ext) const {
+    const T zero = T(0);
 #pragma unroll
-        for (int l = 0; l < V; l++) (pout + l * g.FS)[ix] = (l == 2 && a.sub_bg) ? pr[2] - rg<T>(g, R_W, i) : pr[l];
-      }
-      if (prim_rec) {
-#pragma unroll
-        for (int l = 0; l < V; l++) ucons[l] = uo[l];
-        in.prim_comoving(i, so, pr, uo);
-      }
-#pragma unroll
-      for (int l = 0; l < V; l++) UC(l, ty, tx) = uo[l];
-    }
-    if (e_in) {
-      in.transform(ei, se, re, pe, ue);
-      if (prim_rec) in.prim_comoving(ei, se, pe, ue);
-#pragma unroll
-      for (int l = 0; l < V; l++) UC(l, er, ec) = ue[l];
-    }
-  }
-  // sources, data checks and CFL of the own interior cell
-  T geo[V], ext[V];
-  T invdt = -Real<T>::huge;
-  int flags = 0;
-#pragma unroll
-  for (int l = 0; l < V; l++) geo[l] = ext[l] = zero;
-  if (out) {
+    for (int l = 0; l < V; l++) geo[l] = ext[l] = zero;
     // geometrical sources (physics_eulerisotherm.f90:689-832, elementals 3069-3088;
-    // physics_euler.f90:1706-1846); zero on cartesian meshes
-    if (g.curvilinear) {
-      const T cxyx = rg<T>(g, R_CXYX, i), cyxy = rg<T>(g, R_CYXY, i);
-      const T czxz = rg<T>(g, R_CZXZ, i), czyz = rg<T>(g, R_CZYZ, i);
-      const T vx = pr[1], vy = pr[2], vz = zero, mx = ur[1], my = ur[2], mz = zero;
-      T P;
-      if (V == 4) {
-        P = pr[3];
-      } else {
-        const T cs = rg<T>(g, R_CS, i);
-        P = pr[0] * (cs * cs);
-      }
+    // physics_euler.f90:1706-1846); zero (c_yxy = 0) on cartesian meshes
+    {
+      const T P = V == 4 ? pr[3] : pr[0] * (cs * cs);
       if constexpr (sizeof(T) == 4) {
         // FP32: the radial momentum source is the small difference of the
         // centrifugal force and gravity (relative size ~(cs/vK)^2 on a disk);
         // both are formed in FP64 from the stored state, with the rotating
         // frame velocity added exactly, and only their sum is rounded
-        const double vyd = a.add_bg ? (double)vres + ring(g, R_W, i) : (double)vy;
+        const T vres = dv(s[2], s[0]);  // azimuthal velocity of the stored state (residual in the FARGO frame)
+        const double vyd = a.add_bg ? (double)vres + wd : (double)pr[2];
         const double rho = (double)ur[0], myd = rho * vyd;
-        const double cyd = ring(g, R_CYXY, i);
-        double s1 = myd * (cyd * vyd - ring(g, R_CXYX, i) * (double)vx) + (cyd + ring(g, R_CZXZ, i)) * (double)P;
-        if (g.gravity) s1 = s1 + rho * a.acc[i];
-        if (g.rotframe) {  // the rotating frame's radial acceleration joins the balance
-          const double ax = g.rotframe == 2 ? g.twoomega * vyd : ring(g, R_CACX, i) + g.twoomega * vyd;
-          s1 = s1 + rho * ax;
+        double s1 = myd * (cyd * vyd) + cyd * (double)P;
+        if (g.gravity) s1 = s1 + rho * accd;
+        if (g.rotframe && g.curvilinear) {  // the rotating frame's radial acceleration joins the balance
+          const double axd = g.rotframe == 2 ? g.twoomega * vyd : cacd + g.twoomega * vyd;
+          s1 = s1 + rho * axd;
         }
         geo[1] = (T)s1;
       } else {
-        geo[1] = my * (cyxy * vy - cxyx * vx) + mz * (czxz * vz - zero * vx) + (cyxy + czxz) * P;
+        geo[1] = ur[2] * (cyxy * pr[2]) + cyxy * P;
       }
-      geo[2] = mz * (czyz * vz - zero * vy) + mx * (cxyx * vx - cyxy * vy) + (cxyx + czyz) * P;
+      geo[2] = ur[1] * -(cyxy * pr[2]);
     }
     // FARGO source (physics_eulerisotherm.f90:1531-1586); Euler also takes
     // -v_y*(that + GetGeometricalSourceY(vz = P = mz = 0)) from the energy
     // (physics_euler.f90:2368-2400, elemental physics_eulerisotherm.f90:
     // 3080-3088), with the real-frame velocities
     if (g.fargo) {
-      T tmp = dv(ur[1] * T(0.5) * (rg<T>(g, R_W, i + 1) - rg<T>(g, R_W, i - 1)), rg<T>(g, R_DLX, i));
+      // FP64: the numerator scaled up, so that the quotient of a tiny radial
+      // momentum rounds as IEEE division does
+      const T m = ur[1] * T(0.5) * dw;
+      T tmp = sizeof(T) == 8 ? dv(m * T(0x1p200), dlx) * T(0x1p-200) : dv(m, dlx);
       geo[2] = geo[2] - tmp;
       if constexpr (V == 4) {
-        const T vx = pr[1], vy = pr[2], mx = ur[1];
-        T cxyx = zero, cyxy = zero, czyz = zero;
-        if (g.curvilinear) cxyx = rg<T>(g, R_CXYX, i), cyxy = rg<T>(g, R_CYXY, i), czyz = rg<T>(g, R_CZYZ, i);
-        tmp = tmp + (zero * (czyz * zero - zero * vy) + mx * (cxyx * vx - cyxy * vy) + (cxyx + czyz) * zero);
-        geo[3] = geo[3] - vy * tmp;
+        tmp = tmp + ur[1] * -(cyxy * pr[2]);
+        geo[3] = geo[3] - pr[2] * tmp;
       }
     }
     // point-mass gravity through the source list (sources_generic.f90:220-261,
     // sources_gravity.f90:164-199, physics_eulerisotherm.f90:1201-1226,
     // physics_euler.f90:1849-1885)
-    if (g.gravity) {
-      const T *acc = sizeof(T) == 4 ? reinterpret_cast<const T *>(a.accf) : reinterpret_cast<const T *>(a.acc);
-      const T ax = acc[(unsigned)i], ay = acc[(unsigned)(g.NI + i)];
-      // FP32 curvilinear: already part of the FP64 radial balance above
-      if (sizeof(T) == 8 || !g.curvilinear) ext[1] = zero + ur[0] * ax;
-      ext[2] = zero + ur[0] * ay;
-      if (V == 4) ext[3] = zero + (ur[1] * ax + ur[2] * ay);
-    }
+    // (FP32: the radial part is in the FP64 balance above; without gravity
+    // the accelerations are zero)
+    if (sizeof(T) == 8) ext[1] = ur[0] * ax;
+    ext[2] = ur[0] * ay;
+    if (V == 4) ext[3] = ur[1] * ax + ur[2] * ay;
     // rotating frame, after gravity in the source list (sources_generic.f90:
     // 133-199, 236-241; sources_rotframe.f90:226-234): centrifugal plus
     // Coriolis acceleration of the real-frame velocities, through the same
     // ExternalSources as gravity
     if (g.rotframe) {
       const T tw = (T)g.twoomega, vx = pr[1], vy = pr[2];
-      T ax, ay;
+      T rx, ry;
       if (g.rotframe == 2) {
-        ax = tw * vy;
-        ay = -(tw * vx);
+        rx = tw * vy;
+        ry = -(tw * vx);
       } else {
-        ax = rg<T>(g, R_CACX, i) + tw * vy;
-        ay = cl<T>(g, C_CACY, j) - tw * vx;
+        rx = cac + tw * vy;
+        ry = cl<T>(g, C_CACY, j) - tw * vx;
       }
       // FP32 curvilinear: the radial part is in the FP64 radial balance above
-      if (sizeof(T) == 8 || !g.curvilinear) ext[1] = ext[1] + ur[0] * ax;
-      ext[2] = ext[2] + ur[0] * ay;
-      if (V == 4) ext[3] = ext[3] + (ur[1] * ax + ur[2] * ay);
-    }
-    // CheckData (timedisc_base.f90:1666-1742) and CFL (timedisc_base.f90:818-909)
-    if (want_check) {
-      if (pr[0] < (T)g.rhomin) flags |= F_RHOMIN;
-      if (V == 4 && pr[3] < (T)g.pmin) flags |= F_PMIN;
-#pragma unroll
-      for (int l = 0; l < V; l++)
-        if (bad(pr[l]) || bad(ur[l])) flags |= F_INVALID;
-    }
-    if (want_cfl) {
-      const T vy = a.sub_bg ? pr[2] - rg<T>(g, R_W, i) : pr[2];
-      const T cs = (V == 4) ? sound_speed(in.gam, pr[0], pr[3]) : rg<T>(g, R_CS, i);
-      invdt = cell_invdt(g, i, pr[1], vy, cs);
+      if (sizeof(T) == 8 || !g.curvilinear) ext[1] = ext[1] + ur[0] * rx;
+      ext[2] = ext[2] + ur[0] * ry;
+      if (V == 4) ext[3] = ext[3] + (ur[1] * rx + ur[2] * ry);
     }
   }
-  __syncthreads();
+};
 
-  // ---- phase 2: limited slopes and face states (reconstruction_linear.f90)
-  const int ir = i < g.NI - 1 ? i : g.NI - 2;  // ring index, kept inside the mesh arrays
-  const int jr = j < g.NJ ? j : g.NJ - 1;
-  const T invdx = (T)g.invdx, invdy = (T)g.invdy;
-  T uc[V], fe[V], fn[V];
-  {
-    const T dw = rg<T>(g, R_RDXW, ir), de = rg<T>(g, R_RDXE, ir);
-    const T ds = cl<T>(g, C_RDYS, jr), dn = cl<T>(g, C_RDYN, jr);
-#pragma unroll
-    for (int l = 0; l < V; l++) {
-      uc[l] = UC(l, ty, tx);
-      const T sx = invdx * slope<T, LIM>(g, UC(l, ty, tx - 1), uc[l], UC(l, ty, tx + 1));
-      FW(l, ty, tx) = uc[l] + sx * dw;
-      fe[l] = uc[l] + sx * de;
-      const T sy = invdy * slope<T, LIM>(g, UC(l, ty - 1, tx), uc[l], UC(l, ty + 1, tx));
-      FS(l, ty, tx) = uc[l] + sy * ds;
-      fn[l] = uc[l] + sy * dn;
-    }
+// The last stage's final combination of one cell with the embedded error
+// (timedisc_rkfehlberg.f90:199-266, timedisc_base.f90:1012-1053): the sums over
+// k_1 .. k_{s-1} are formed when the cell's inputs arrive, the term of this
+// stage's rhs is added when it is known.  FP64: the reference's operation
+// order; FP32: compensated sums, error norm in FP64.
+template <typename T, int V, int NK>
+struct Combination {
+  T h[V], lo[V];               // FP64: both embedded solutions; FP32: compensated sum
+  T e[sizeof(T) == 4 ? V : 1];  // FP32: difference of the two, summed directly (no cancellation)
+  // FP32: weights b_h*dt as hi/lo pairs, and (b_h - b_l)*dt for the error
+  static __device__ __forceinline__ void weights(const StageArgsT<T> &a, double dt, int q, float &bhh, float &bhl,
+                                                 float &bde) {
+    const double bh = a.bh[q] * dt;
+    bhh = (float)bh;
+    bhl = (float)(bh - (double)bhh);
+    bde = (float)((a.bh[q] - a.bl[q]) * dt);
   }
-  // extra faces: N of row -1 and S of row TY (t < 2*TX); E of column -1 and
-  // W of column TX (next 2*TY threads)
-  if (t < 2 * TX) {
-    const int xk = t / TX;  // 0: row -1 (N face), 1: row TY (S face)
-    const int xr = xk ? TY : -1, xc = tx;
-    const int jj = j0 + xr, jc = jj < g.NJ ? jj : g.NJ - 1;
-    const T off = xk ? cl<T>(g, C_RDYS, jc) : cl<T>(g, C_RDYN, jc);
-#pragma unroll
-    for (int l = 0; l < V; l++) {
-      const T c0 = UC(l, xr, xc);
-      const T f = c0 + invdy * slope<T, LIM>(g, UC(l, xr - 1, xc), c0, UC(l, xr + 1, xc)) * off;
-      if (xk)
-        FS(l, TY, xc) = f;
-      else
-        FN1(l, xc) = f;
-    }
-  } else if (t < 2 * TX + 2 * TY) {
-    const int k = t - 2 * TX;
-    const int xk = k / TY;  // 0: column -1 (E face), 1: column TX (W face)
-    const int xr = k % TY, xc = xk ? TX : -1;
-    const int ii = i0 + xc, ic = ii < g.NI ? ii : g.NI - 1;
-    const T off = xk ? rg<T>(g, R_RDXW, ic) : rg<T>(g, R_RDXE, ic);
-#pragma unroll
-    for (int l = 0; l < V; l++) {
-      const T c0 = UC(l, xr, xc);
-      const T f = c0 + invdx * slope<T, LIM>(g, UC(l, xr, xc - 1), c0, UC(l, xr, xc + 1)) * off;
-      if (xk)
-        FW(l, xr, TX) = f;
-      else
-        FE1(l, xr) = f;
-    }
-  }
-  __syncthreads();
-
-  // ---- phase 3: KT interface fluxes (fluxes_kt.f90:126-176)
-  auto kt = [&](int d, const T *L, const T *R, T csL, T csR, T dA, T *F) {
-    if (prim_rec)
-      kt_flux_p<T, V>(g, d, L, R, csL, csR, dA, F);
-    else
-      kt_flux<T, V>(g, d, L, R, csL, csR, dA, F);
-  };
-  T xf[V], yf[V];
-  {
-    T r2[V], n2[V];
-#pragma unroll
-    for (int l = 0; l < V; l++) {
-      r2[l] = FW(l, ty, tx + 1);
-      n2[l] = FS(l, ty + 1, tx);
-    }
-    kt(0, fe, r2, rg<T>(g, R_CSE, ir), rg<T>(g, R_CSW, ir + 1), rg<T>(g, R_DAXW, ir + 1), xf);
-    kt(1, fn, n2, rg<T>(g, R_CSN, ir), rg<T>(g, R_CSS, ir), rg<T>(g, R_DAYS, ir), yf);
-#pragma unroll
-    for (int l = 0; l < V; l++) {
-      FLX(l, ty, tx + 1) = xf[l];
-      FLY(l, ty + 1, tx) = yf[l];
-    }
-  }
-  // extra fluxes: south interface of row 0 (t < TX), west interface of
-  // column 0 (threads 2*TX .. 2*TX+TY-1)
-  if (t < TX) {
-    T s1[V], n1[V], ef[V];
-#pragma unroll
-    for (int l = 0; l < V; l++) {
-      n1[l] = FN1(l, tx);
-      s1[l] = FS(l, 0, tx);
-    }
-    kt(1, n1, s1, rg<T>(g, R_CSN, ir), rg<T>(g, R_CSS, ir), rg<T>(g, R_DAYS, ir), ef);
-#pragma unroll
-    for (int l = 0; l < V; l++) FLY(l, 0, tx) = ef[l];
-  } else if (t >= 2 * TX && t < 2 * TX + TY) {
-    const int fr = t - 2 * TX;
-    T e1[V], w1[V], ef[V];
-#pragma unroll
-    for (int l = 0; l < V; l++) {
-      e1[l] = FE1(l, fr);
-      w1[l] = FW(l, fr, 0);
-    }
-    kt(0, e1, w1, rg<T>(g, R_CSE, i0 - 1), rg<T>(g, R_CSW, i0), rg<T>(g, R_DAXW, i0), ef);
-#pragma unroll
-    for (int l = 0; l < V; l++) FLX(l, fr, 0) = ef[l];
-  }
-  __syncthreads();
-
-  // ---- phase 4: rhs assembly (timedisc_base.f90:1254-1271)
-  double err = -DBL_MAX;
-  if (out) {
-    const T dydzdV = rg<T>(g, R_DYDZDV, i), dzdxdV = rg<T>(g, R_DZDXDV, i);
-    const T dxdydV = rg<T>(g, R_DXDYDV, i);
-    const unsigned ix = (unsigned)j * (unsigned)g.P + (unsigned)i;
-    T rhs[V];
-    // the viscous source joins the source list's sum last (sources_generic.f90:
-    // 236-241); it has no density component
+  __device__ __forceinline__ void add(const StageArgsT<T> &a, double dt, int q, const T *k) {
     if constexpr (sizeof(T) == 8) {
-      if (a.vsrc) {
-#pragma unroll
-        for (int l = 1; l < V; l++) ext[l] = ext[l] + (a.vsrc + (l - 1) * g.FS)[ix];
-      }
-    }
-#pragma unroll
-    for (int l = 0; l < V; l++) {
-      const T xw = FLX(l, ty, tx), ys = FLY(l, ty, tx);
-      rhs[l] = dydzdV * (xf[l] - xw) + dzdxdV * (yf[l] - ys) + dxdydV * (zero - zero) - geo[l] - ext[l];
-      if (yout) (yout + l * g.FS)[ix] = prim_rec ? ucons[l] : uc[l];
-    }
-    // boundary rows: the fluxes through the mesh boundary at the boundary
-    // cells' outer interfaces, Mesh%dy*Mesh%dz*xflux (W), -Mesh%dy*Mesh%dz*xflux
-    // (E) and likewise in y (timedisc_base.f90:1224-1252), stored at the ghost
-    // position next to the cell (the last stage: into bks).  bxs/bys: the x
-    // and y side of a boundary cell (0 W/S, 1 E/N, -1 none).
-    const int bxs = !a.bflux ? -1 : i == imin ? 0 : i == imax ? 1 : -1;
-    const int bys = !a.bflux ? -1 : j == jmin ? 0 : j == jmax ? 1 : -1;
-    const unsigned gxx = (unsigned)j * (unsigned)g.P + (unsigned)(bxs == 0 ? imin - 1 : imax + 1);
-    const unsigned gxy = (unsigned)(bys == 0 ? jmin - 1 : jmax + 1) * (unsigned)g.P + (unsigned)i;
-    const long bix = (long)bxs * g.NJ + j, biy = 2L * V * g.NJ + (long)bys * g.NI + i;
-    T kbx[V], kby[V];
-    if (bxs >= 0 || bys >= 0) {
-      const T ax = (T)g.bdydz, ay = (T)g.bdzdx;
+      const T cl = a.bl[q] * dt, ch = a.bh[q] * dt;
 #pragma unroll
       for (int l = 0; l < V; l++) {
-        kbx[l] = bxs == 0 ? ax * FLX(l, ty, tx) : -(ax * xf[l]);
-        kby[l] = bys == 0 ? ay * FLY(l, ty, tx) : -(ay * yf[l]);
-        if (!ynew) {
-          if (bxs >= 0) (a.kout + l * g.FS)[gxx] = kbx[l];
-          if (bys >= 0) (a.kout + l * g.FS)[gxy] = kby[l];
-        }
-      }
-    }
-    if (ynew) {
-      // final combination with this stage's rhs as k_s, and the error of the
-      // embedded solution (FP64: same operation order as the reference;
-      // FP32: compensated sums, error norm in FP64)
-      T y[V], kq[KM][V];
-#pragma unroll
-      for (int l = 0; l < V; l++) y[l] = (a.Y + l * g.FS)[ix];
-#pragma unroll
-      for (int q = 0; q < KM; q++)
-        if (q < in.nk) {
-#pragma unroll
-          for (int l = 0; l < V; l++) kq[q][l] = (a.k[q] + l * g.FS)[ix];
-        }
-      // FP32: weights b_h*dt as hi/lo pairs, and (b_h - b_l)*dt for the error
-      float bhh[KM], bhl[KM], bde[KM];
-      if constexpr (sizeof(T) == 4) {
-#pragma unroll
-        for (int q = 0; q < KM; q++) {
-          const double bh = a.bh[q] * in.dt;
-          bhh[q] = (float)bh;
-          bhl[q] = (float)(bh - (double)bhh[q]);
-          bde[q] = (float)((a.bh[q] - a.bl[q]) * in.dt);
-        }
-      }
-#pragma unroll
-      for (int l = 0; l < V; l++) {
-        // k_1 .. k_{s-1} from memory, then this stage's rhs as k_s (every
-        // coefficient index is a compile-time constant)
-        double yh, dif;
-        if constexpr (sizeof(T) == 8) {
-          T h = y[l], w = y[l];
-#pragma unroll
-          for (int q = 0; q < KM; q++)
-            if (q <= in.nk) {
-              const T kk = q < in.nk ? kq[q][l] : rhs[l];
-              w = w - (T)(a.bl[q] * in.dt) * kk;
-              h = h - (T)(a.bh[q] * in.dt) * kk;
-            }
-          (ynew + l * g.FS)[ix] = h;
-          yh = (double)h;
-          dif = yh - (double)w;
-        } else {
-          // compensated accumulation of the new state; the difference of the
-          // two embedded solutions summed directly (no cancellation)
-          Acc h((float)y[l]);
-          float e = 0.f;
-#pragma unroll
-          for (int q = 0; q < KM; q++)
-            if (q <= in.nk) {
-              const float kk = (float)(q < in.nk ? kq[q][l] : rhs[l]);
-              h.sub(bhh[q], bhl[q], kk);
-              e = fmaf(bde[q], kk, e);
-            }
-          (ynew + l * g.FS)[ix] = (T)h.value();
-          yh = h.wide();
-          dif = (double)e;
-        }
-        err = fmax2(err, fabs(dif) / (a.tol_rel * fabs(yh) + a.tol_abs[l]));
-      }
-      // this stage's boundary rows for the boundary-flux accumulation
-#pragma unroll
-      for (int l = 0; l < V; l++) {
-        if (bxs >= 0) a.bks[bix + 2L * l * g.NJ] = (double)kbx[l];
-        if (bys >= 0) a.bks[biy + 2L * l * g.NI] = (double)kby[l];
+        lo[l] = lo[l] - cl * k[l];
+        h[l] = h[l] - ch * k[l];
       }
     } else {
+      float bhh, bhl, bde;
+      weights(a, dt, q, bhh, bhl, bde);
 #pragma unroll
-      for (int l = 0; l < V; l++) (a.kout + l * g.FS)[ix] = rhs[l];
-    }
-  }
-  if (ynew) {
-    double m = err;
-    int unused = 0;
-    blk_max_or0(m, unused, redd, redi);
-    if (t == 0) {
-      const int b = bx + by * nbx;
-      a.part_c[2 * b] = m;
-      a.part_c[2 * b + 1] = 0.0;
-    }
-  }
-
-  if (!(want_cfl || want_check)) return;
-  if (own_g || e_g) {  // ghost cells evaluated in phase 1
-    if constexpr (kEnd) {
-      invdt = fmax2(invdt, gcfl[t]);
-      flags |= gflg[t];
-    }
-  }
-  // ---- the corner ghost cells (in no footprint) of the corner tiles:
-  // data checks, CFL and the new state (SetCornerEdges, boundary_generic.f90:434-517)
-  if (t < 16) {
-    const bool west = bx == 0, east = bx == nbx - 1;
-    const bool south = by == 0, north = by == nby - 1;
-    const int c = t / 4, ga = 1 + (t & 1), gb = 1 + ((t >> 1) & 1);
-    const int ce = c & 1, cn = c >> 1;
-    if ((ce ? east : west) && (cn ? north : south)) {
-      const int gi = ce ? imax + ga : imin - ga, gj = cn ? jmax + gb : jmin - gb;
-      T u[V], p[V];
-      in.ghost_final(gi, gj, u, p, flags);
-      if (want_cfl) {
-        const T cs = (V == 4) ? sound_speed(in.gam, p[0], p[3]) : rg<T>(g, R_CS, gi);
-        invdt = fmax2(invdt, cell_invdt(g, gi, p[1], p[2], cs));
-      }
-      if (yout) {
-        const unsigned ix = (unsigned)gj * (unsigned)g.P + (unsigned)gi;
-#pragma unroll
-        for (int l = 0; l < V; l++) (yout + l * g.FS)[ix] = u[l];
-      }
-      if (pout) {
-        const unsigned ix = (unsigned)gj * (unsigned)g.P + (unsigned)gi;
-#pragma unroll
-        for (int l = 0; l < V; l++) (pout + l * g.FS)[ix] = p[l];
+      for (int l = 0; l < V; l++) {
+        Acc c(h[l]);
+        c.lo = lo[l];
+        c.sub(bhh, bhl, k[l]);
+        h[l] = c.hi;
+        lo[l] = c.lo;
+        e[l] = fmaf(bde, k[l], e[l]);
       }
     }
   }
-  // CFL partials in FP64 (the maximum of FP32 values is exact)
-  double m = invdt == -Real<T>::huge ? -DBL_MAX : (double)invdt;
-  int f = flags;
-  if (ynew) __syncthreads();  // the reduction scratch is in use above
-  blk_max_or0(m, f, redd, redi);
-  if (t == 0) {
-    const int b = bx + by * nbx;
-    a.part[2 * b] = m;
-    a.part[2 * b + 1] = (double)f;
+  __device__ __forceinline__ void begin(const StageArgsT<T> &a, double dt, const T *y, const T (*k)[V]) {
+#pragma unroll
+    for (int l = 0; l < V; l++) {
+      h[l] = y[l];
+      lo[l] = sizeof(T) == 8 ? y[l] : T(0);
+      if constexpr (sizeof(T) == 4) e[l] = T(0);
+    }
+#pragma unroll
+    for (int q = 0; q < NK; q++) add(a, dt, q, k[q]);
   }
-  // the step's boundary-flux accumulation (device-controlled steps), after
-  // this tile's work so that it adds no register pressure to it
-  if (kEnd && a.bfa.out) {
-    const int nt = TX * TY;
-    bflux_accumulate(a.bfa, in.dt, (bx + by * nbx) * nt + t, nbx * nby * nt);
+  // stores the new state and returns the cell's error
+  __device__ __forceinline__ double finish(const Geom &g, const StageArgsT<T> &a, double dt, unsigned ix,
+                                           const T *rhs) {
+    double err = -DBL_MAX;
+    add(a, dt, NK, rhs);
+#pragma unroll
+    for (int l = 0; l < V; l++) {
+      double yh, dif;
+      if constexpr (sizeof(T) == 8) {
+        (a.ynew + l * g.FS)[ix] = h[l];
+        yh = h[l];
+        dif = h[l] - lo[l];
+      } else {
+        (a.ynew + l * g.FS)[ix] = h[l] + lo[l];
+        yh = (double)h[l] + (double)lo[l];
+        dif = (double)e[l];
+      }
+      err = fmax2(err, fabs(dif) / (a.tol_rel * fabs(yh) + a.tol_abs[l]));
+    }
+    return err;
   }
-}
-
-template <typename T, int V, int LIM, int TX, int KM, int MODE>
-__global__ __launch_bounds__(TX *TY_RHS, (rhs_waves_per_simd<T, V, TX, KM, MODE>())) void k_rhs(Geom g, StageArgsT<T> a) {
-  const int nbx = (g.inum + TX - 1) / TX, nby = (g.jnum + TY_RHS - 1) / TY_RHS;
-  int bx, by;
-  if (!xcd_tile(blockIdx.x, nbx, nby, bx, by)) return;
-  rhs_tile<T, V, LIM, TX, KM, MODE>(g, a, bx, by, nbx, nby);
-}
-
-// Many meshes in one launch: block b runs the tile tiles[b] (TileCode) of
-// the mesh whose Geom and arguments of this launch are tab[disk].
-template <typename T, int V, int LIM, int TX, int KM, int MODE>
-__global__ __launch_bounds__(TX *TY_RHS, (rhs_waves_per_simd<T, V, TX, KM, MODE>())) void k_rhs_multi(
-    const RhsEntry *__restrict__ tab, const unsigned *__restrict__ tiles) {
-  const unsigned e = tiles[blockIdx.x];
-  if (e == NO_TILE) return;
-  const RhsEntry &E = tab[tile_disk(e)];
-  const StageArgsT<T> &a = reinterpret_cast<const StageArgsT<T> &>(E.a);
-  const int nbx = (E.g.inum + TX - 1) / TX, nby = (E.g.jnum + TY_RHS - 1) / TY_RHS;
-  rhs_tile<T, V, LIM, TX, KM, MODE>(E.g, a, tile_bx(e), tile_by(e), nbx, nby);
-}
+};
 
 // ------------------------------------------------------------ FARGO remap
 // FargoAdvectionY (timedisc_base.f90:1935-2069) of one interior cell from
@@ -1489,9 +1159,8 @@ __device__ __forceinline__ void remap_block(const Geom &g, const RemapArgsT<T> &
 
 template <typename T, int V>
 __global__ __launch_bounds__(256) void k_remap(Geom g, RemapArgsT<T> a) {
-  int bx, by;
-  if (!xcd_tile(blockIdx.x, (g.inum + 63) / 64, remap_rows_blocks(g.jnum), bx, by)) return;
-  remap_block<T, V>(g, a, bx, by);
+  const int nbx = (g.inum + 63) / 64, n = nbx * remap_rows_blocks(g.jnum), t = xcd_tile(blockIdx.x, n);
+  if (t < n) remap_block<T, V>(g, a, t % nbx, t / nbx);
 }
 template <typename T, int V>
 __global__ __launch_bounds__(256) void k_remap_multi(const RemapEntry *__restrict__ tab,
@@ -1618,7 +1287,7 @@ __global__ __launch_bounds__(VT_X *VT_Y, FV_VISC_WAVES_PER_SIMD) void k_visc(Geo
   __shared__ double Pown[V == 4 ? VT_Y : 1][V == 4 ? VT_X : 1];  // Euler: pressure of the own cells
   __shared__ double red[VT_X * VT_Y / 64];
   if (a.ctl && a.ctl->halt) return;
-  const In<double, V, KM> in(g, a, false);
+  const In<double, V, KM> in(g, a, false, a.ctl ? a.ctl->dt : a.dt);  // device-controlled: this step's dt
   const int tx = threadIdx.x, ty = threadIdx.y, t = tx + VT_X * ty;
   const int i0 = blockIdx.x * VT_X, j0 = blockIdx.y * VT_Y;
   const int imin = GH, imax = GH + g.inum - 1, jmin = GH, jmax = GH + g.jnum - 1;
@@ -1777,16 +1446,17 @@ __global__ __launch_bounds__(256) void k_visc_cfl(Geom g, VisArgs va, const doub
 
 // typed launchers, explicitly instantiated in fv_inst_*.hip (one translation
 // unit per element type and kernel family, compiled in parallel)
-template <typename T, int KM>
-void rhs_single(const Geom &g, const StageArgsT<T> &a, int V, hipStream_t s);
+template <typename T, int V>
+void rhs_single(const Geom &g, const StageArgsT<T> &a, hipStream_t s);
 template <typename T>
 void remap_single(const Geom &g, const RemapArgsT<T> &a, int V, hipStream_t s);
 template <typename T>
 void frame_single(const Geom &g, const void *src, void *dst, int sign, int V, const Ctl *ctl, const void *w2,
                   hipStream_t s);
-template <typename T, int KM>
-void rhs_multi(const RhsEntry *tab, const unsigned *tiles, int n, int V, int limiter, int tx, int mode, hipStream_t s);
-// coefficient slots the kernels are compiled for, by tableau size
+template <typename T, int V>
+void rhs_multi(const RhsEntry *tab, const unsigned *tiles, int n, int limiter, int rows, int mode, int nk,
+               hipStream_t s);
+// coefficient slots k_visc is compiled for, by tableau size
 constexpr int KM_SMALL = 3;
 inline int km_for(int stages) { return stages <= KM_SMALL ? KM_SMALL : MAXK; }
 template <typename T>

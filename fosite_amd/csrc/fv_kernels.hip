@@ -15,18 +15,36 @@ __device__ __forceinline__ void control_block(Ctl *ctl, const double *part_c, co
                                               const double *part_v = nullptr, int nbv = 0) {
   __shared__ double rede[4], redm[4], redv[4];
   __shared__ int redi[4];
-  if (ctl->halt) return;
+  // the whole header first: one memory latency beside the partials', and the
+  // decisions below then run on registers
+  CtlHead h = *ctl;
   double e = -DBL_MAX, m = -DBL_MAX, v = -DBL_MAX;
   int f = 0;
-#pragma unroll 4
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) {
-    e = fmax2(e, part_c[2 * b]);
-    m = fmax2(m, part_r[2 * b]);
-    f |= (int)part_r[2 * b + 1];
+  constexpr int Q = 4;  // partials per thread and pass, all loaded before the first is used
+  for (int b0 = threadIdx.x; b0 < nb; b0 += Q * 256) {
+    double pe[Q], pm[Q], pf[Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++) {  // (beyond the end: the last one again)
+      const int b = min(b0 + q * 256, nb - 1);
+      pe[q] = part_c[2 * b];
+      pm[q] = part_r[2 * b];
+      pf[q] = part_r[2 * b + 1];
+    }
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+      e = fmax2(e, pe[q]);
+      m = fmax2(m, pm[q]);
+      f |= (int)pf[q];
+    }
+  }
+  if (threadIdx.x == 0) {  // the corner cells' partial
+    m = fmax2(m, part_r[2 * nb]);
+    f |= (int)part_r[2 * nb + 1];
   }
   if (part_v) {
     for (int b = threadIdx.x; b < nbv; b += blockDim.x) v = fmax2(v, part_v[2 * b]);
   }
+  if (h.halt) return;
   // one barrier: wave results to LDS, thread 0 combines
   e = wave_max(e);
   m = wave_max(m);
@@ -49,8 +67,11 @@ __device__ __forceinline__ void control_block(Ctl *ctl, const double *part_c, co
       v = fmax2(v, redv[k]);
       f |= redi[k];
     }
-    control_accept(ctl, e);
-    if (!ctl->halt) control_next(ctl, m, f, v);
+    ctl->err_hist[h.step] = e;
+    ctl->dt_hist[h.step] = h.dt;
+    control_accept(&h, e);
+    if (!h.halt) control_next(&h, m, f, v);
+    *static_cast<CtlHead *>(ctl) = h;
   }
 }
 __global__ __launch_bounds__(256) void k_control(Ctl *ctl, const double *part_c, const double *part_r, int nb,
@@ -258,17 +279,27 @@ hipError_t scratch_address(int dev, double **out) {
 static_assert(sizeof(StageArgsT<float>) == sizeof(StageArgsT<double>), "StageArgs layout");
 static_assert(sizeof(RemapArgsT<float>) == sizeof(RemapArgsT<double>), "RemapArgs layout");
 
-int rhs_blocks(const Geom &g) { return ((g.inum + g.tile_x - 1) / g.tile_x) * ((g.jnum + TY_RHS - 1) / TY_RHS); }
+// partials of a last stage; an end-of-step evaluation has one more (the corner cells)
+int rhs_blocks(const Geom &g) { return strip_cols(g.inum) * strip_blocks(g.jnum, g.rows); }
+// The fewest rows that still give no more waves than the chip's SIMDs hold well
+// (256 CUs of 4; one FP64 or two FP32 waves each): fewer rows leave a wave a
+// shorter serial march, more rows read and transform fewer halo rows (rows + 4
+// per strip).  us per 512x1024 step at 2, 4 and 8 rows: 100, 85, 79 in FP64,
+// 63, 56, 61 in FP32.
+int strip_rows(long wave_rows, int dtype) {
+  const long waves = dtype == 1 ? 2048 : 1024, r = (wave_rows + waves - 1) / waves;
+  return r < 1 ? 1 : r > STRIP_ROWS ? STRIP_ROWS : (int)r;
+}
 
 void launch_rhs(const Geom &g, const StageArgs &a, int V, hipStream_t s) {
   if (g.dtype == 1) {
     StageArgsT<float> af;
     std::memcpy(&af, &a, sizeof(af));
-    if (km_for(g.stages) == KM_SMALL) rhs_single<float, KM_SMALL>(g, af, V, s);
-    else rhs_single<float, MAXK>(g, af, V, s);
+    if (V == 3) rhs_single<float, 3>(g, af, s);
+    else rhs_single<float, 4>(g, af, s);
   } else {
-    if (km_for(g.stages) == KM_SMALL) rhs_single<double, KM_SMALL>(g, a, V, s);
-    else rhs_single<double, MAXK>(g, a, V, s);
+    if (V == 3) rhs_single<double, 3>(g, a, s);
+    else rhs_single<double, 4>(g, a, s);
   }
 }
 void launch_remap(const Geom &g, const RemapArgs &a, int V, hipStream_t s) {
@@ -293,14 +324,13 @@ void launch_control(Ctl *ctl, const double *part_c, const double *part_r, int nb
 }
 int visc_blocks(const Geom &g) { return ((g.NI + VT_X - 1) / VT_X) * ((g.NJ + VT_Y - 1) / VT_Y); }
 void launch_rhs_multi(const RhsEntry *tab, const unsigned *tiles, int ntiles, int V, int dtype, int limiter,
-                      int tx, int stages, int mode, hipStream_t s) {
-  const bool small = km_for(stages) == KM_SMALL;
+                      int rows, int mode, int nk, hipStream_t s) {
   if (dtype == 1) {
-    if (small) rhs_multi<float, KM_SMALL>(tab, tiles, ntiles, V, limiter, tx, mode, s);
-    else rhs_multi<float, MAXK>(tab, tiles, ntiles, V, limiter, tx, mode, s);
+    if (V == 3) rhs_multi<float, 3>(tab, tiles, ntiles, limiter, rows, mode, nk, s);
+    else rhs_multi<float, 4>(tab, tiles, ntiles, limiter, rows, mode, nk, s);
   } else {
-    if (small) rhs_multi<double, KM_SMALL>(tab, tiles, ntiles, V, limiter, tx, mode, s);
-    else rhs_multi<double, MAXK>(tab, tiles, ntiles, V, limiter, tx, mode, s);
+    if (V == 3) rhs_multi<double, 3>(tab, tiles, ntiles, limiter, rows, mode, nk, s);
+    else rhs_multi<double, 4>(tab, tiles, ntiles, limiter, rows, mode, nk, s);
   }
 }
 void launch_remap_multi(const RemapEntry *tab, const unsigned *tiles, int ntiles, int V, int dtype, hipStream_t s) {

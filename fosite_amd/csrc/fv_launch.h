@@ -1,45 +1,69 @@
 // fv_launch.h -- launch templates of the kernels in fv_kernels.h: the
-// compile-time variants (limiter, tile width, field count) each launch picks.
+// compile-time variants (limiter, slopes, mode, field count) each launch picks.
 #pragma once
-#include "fv_kernels.h"
+#include "fv_strip.h"
 
 namespace fv {
 
-template <typename T, int V, int LIM, int TX, int KM>
-static void rhs_lim(const Geom &g, const StageArgsT<T> &a, hipStream_t s) {
-  const dim3 grid(xcd_grid((g.inum + TX - 1) / TX, (g.jnum + TY_RHS - 1) / TY_RHS)), block(TX, TY_RHS);
-  switch (rhs_mode(a)) {
-    case M_STAGE: hipLaunchKernelGGL((k_rhs<T, V, LIM, TX, KM, M_STAGE>), grid, block, 0, s, g, a); break;
-    case M_LAST: hipLaunchKernelGGL((k_rhs<T, V, LIM, TX, KM, M_LAST>), grid, block, 0, s, g, a); break;
-    default: hipLaunchKernelGGL((k_rhs<T, V, LIM, TX, KM, M_END>), grid, block, 0, s, g, a); break;
+// f(integral constant NK): the number of slopes in a launch's stage sum, for
+// the tableaux of 3, 5, 6 and 7 stages
+template <int N>
+struct Slots {
+  static constexpr int value = N;
+};
+template <class F>
+static void with_stage_slopes(int nk, F f) {
+  switch (nk) {
+    case 1: f(Slots<1>()); break;
+    case 2: f(Slots<2>()); break;
+    case 3: f(Slots<3>()); break;
+    case 4: f(Slots<4>()); break;
+    default: f(Slots<5>()); break;
   }
 }
-template <typename T, int V, int TX, int KM>
-static void rhs_v(const Geom &g, const StageArgsT<T> &a, hipStream_t s) {
+template <class F>
+static void with_last_slopes(int nk, F f) {
+  switch (nk) {
+    case 2: f(Slots<2>()); break;
+    case 4: f(Slots<4>()); break;
+    case 5: f(Slots<5>()); break;
+    default: f(Slots<6>()); break;
+  }
+}
+template <typename T, int V, int LIM>
+static void rhs_lim(const Geom &g, const StageArgsT<T> &a, hipStream_t s) {
+  const int mode = rhs_mode(a), n = strip_cols(g.inum) * strip_blocks(g.jnum, g.rows);
+  const dim3 grid(xcd_grid(n) + (mode == M_END ? rhs_aux(g, a) : 0)), block(64 * SWAVES);
+  switch (mode) {
+    case M_STAGE:
+      with_stage_slopes(a.nk, [&](auto n) {
+        hipLaunchKernelGGL((k_rhs<T, V, LIM, decltype(n)::value, M_STAGE>), grid, block, 0, s, g, a);
+      });
+      break;
+    case M_LAST:
+      with_last_slopes(a.nk, [&](auto n) {
+        hipLaunchKernelGGL((k_rhs<T, V, LIM, decltype(n)::value, M_LAST>), grid, block, 0, s, g, a);
+      });
+      break;
+    default: hipLaunchKernelGGL((k_rhs<T, V, LIM, 0, M_END>), grid, block, 0, s, g, a); break;
+  }
+}
+template <typename T, int V>
+void rhs_single(const Geom &g, const StageArgsT<T> &a, hipStream_t s) {
   // compile-time limiters for the common choices, run-time switch otherwise
   // (and for PRIMITIVE reconstruction, which only that instantiation carries)
   if (g.recon_prim)
-    rhs_lim<T, V, 0, TX, KM>(g, a, s);
+    rhs_lim<T, V, 0>(g, a, s);
   else if (g.limiter == VANLEER)
-    rhs_lim<T, V, VANLEER, TX, KM>(g, a, s);
+    rhs_lim<T, V, VANLEER>(g, a, s);
   else if (g.limiter == MINMOD)
-    rhs_lim<T, V, MINMOD, TX, KM>(g, a, s);
+    rhs_lim<T, V, MINMOD>(g, a, s);
   else
-    rhs_lim<T, V, 0, TX, KM>(g, a, s);
-}
-template <typename T, int KM>
-void rhs_single(const Geom &g, const StageArgsT<T> &a, int V, hipStream_t s) {
-  if (V == 3) {
-    if (g.tile_x == 32) rhs_v<T, 3, 32, KM>(g, a, s);
-    else rhs_v<T, 3, 64, KM>(g, a, s);
-  } else {
-    if (g.tile_x == 32) rhs_v<T, 4, 32, KM>(g, a, s);
-    else rhs_v<T, 4, 64, KM>(g, a, s);
-  }
+    rhs_lim<T, V, 0>(g, a, s);
 }
 template <typename T>
 void remap_single(const Geom &g, const RemapArgsT<T> &a, int V, hipStream_t s) {
-  const dim3 grid(xcd_grid((g.inum + 63) / 64, remap_rows_blocks(g.jnum))), block(64, 4);
+  const dim3 grid(xcd_grid((g.inum + 63) / 64 * remap_rows_blocks(g.jnum))), block(64, 4);
   if (V == 3)
     hipLaunchKernelGGL((k_remap<T, 3>), grid, block, 0, s, g, a);
   else
@@ -59,31 +83,35 @@ void frame_single(const Geom &g, const void *src, void *dst, int sign, int V, co
 
 // batches: van Leer compiled in, every other limiter (and mixed limiters) by
 // the run-time switch
-template <typename T, int V, int LIM, int TX, int KM>
-static void rhs_multi_lim(const RhsEntry *tab, const unsigned *tiles, int n, int mode, hipStream_t s) {
-  const dim3 block(TX, TY_RHS);
+template <typename T, int V, int LIM>
+static void rhs_multi_lim(const RhsEntry *tab, const unsigned *tiles, int n, int rows, int mode, int nk,
+                          hipStream_t s) {
+  const dim3 block(64 * SWAVES);
   switch (mode) {
-    case M_STAGE: hipLaunchKernelGGL((k_rhs_multi<T, V, LIM, TX, KM, M_STAGE>), dim3(n), block, 0, s, tab, tiles); break;
-    case M_LAST: hipLaunchKernelGGL((k_rhs_multi<T, V, LIM, TX, KM, M_LAST>), dim3(n), block, 0, s, tab, tiles); break;
-    default: hipLaunchKernelGGL((k_rhs_multi<T, V, LIM, TX, KM, M_END>), dim3(n), block, 0, s, tab, tiles); break;
+    case M_STAGE:
+      with_stage_slopes(nk, [&](auto k) {
+        hipLaunchKernelGGL((k_rhs_multi<T, V, LIM, decltype(k)::value, M_STAGE>), dim3(n), block, 0, s, tab, tiles,
+                           rows);
+      });
+      break;
+    case M_LAST:
+      with_last_slopes(nk, [&](auto k) {
+        hipLaunchKernelGGL((k_rhs_multi<T, V, LIM, decltype(k)::value, M_LAST>), dim3(n), block, 0, s, tab, tiles,
+                           rows);
+      });
+      break;
+    default:
+      hipLaunchKernelGGL((k_rhs_multi<T, V, LIM, 0, M_END>), dim3(n), block, 0, s, tab, tiles, rows);
+      break;
   }
 }
-template <typename T, int V, int TX, int KM>
-static void rhs_multi_v(const RhsEntry *tab, const unsigned *tiles, int n, int limiter, int mode, hipStream_t s) {
+template <typename T, int V>
+void rhs_multi(const RhsEntry *tab, const unsigned *tiles, int n, int limiter, int rows, int mode, int nk,
+               hipStream_t s) {
   if (limiter == VANLEER)
-    rhs_multi_lim<T, V, VANLEER, TX, KM>(tab, tiles, n, mode, s);
+    rhs_multi_lim<T, V, VANLEER>(tab, tiles, n, rows, mode, nk, s);
   else
-    rhs_multi_lim<T, V, 0, TX, KM>(tab, tiles, n, mode, s);
-}
-template <typename T, int KM>
-void rhs_multi(const RhsEntry *tab, const unsigned *tiles, int n, int V, int limiter, int tx, int mode, hipStream_t s) {
-  if (V == 3) {
-    if (tx == 32) rhs_multi_v<T, 3, 32, KM>(tab, tiles, n, limiter, mode, s);
-    else rhs_multi_v<T, 3, 64, KM>(tab, tiles, n, limiter, mode, s);
-  } else {
-    if (tx == 32) rhs_multi_v<T, 4, 32, KM>(tab, tiles, n, limiter, mode, s);
-    else rhs_multi_v<T, 4, 64, KM>(tab, tiles, n, limiter, mode, s);
-  }
+    rhs_multi_lim<T, V, 0>(tab, tiles, n, rows, mode, nk, s);
 }
 template <typename T>
 void remap_multi(const RemapEntry *tab, const unsigned *tiles, int n, int V, hipStream_t s) {

@@ -1,0 +1,603 @@
+// fv_strip.h -- the right-hand-side kernel of the finite-volume step: one
+// wavefront per strip of 64 columns, marching along y.
+#pragma once
+#include "fv_kernels.h"
+
+namespace fv {
+
+// A wave owns SW output columns (one lane each) and up to SR rows, and walks
+// its rows from the southern halo to the northern one:
+//   * the loads of a row are issued one row ahead of its arithmetic;
+//   * along y everything lives in registers: the state of three rows, the
+//     north face and the south flux of the row before;
+//   * along x neighbours exchange through DPP wave shifts; the three columns
+//     at either edge (halo cells, x ghost cells, the faces and the flux one
+//     interface beyond the strip) are evaluated for all rows at once by the
+//     64 lanes before the march and wait in LDS;
+//   * y ghost rows are interior rows read at their boundary rule's source row
+//     and taken through the ghost cells' conversions.
+// No wave waits for another before the workgroup's final reduction.
+//
+// What bounds it: VALU issue.  A row of 64 cells takes about 390 vector
+// instructions (isothermal van Leer stage), 12 of them quarter-rate
+// reciprocals; one wave alone issues an FP64 instruction every 6 to 7 cycles
+// (two waves on a SIMD: every 4.6 to 4.8).  Before this, one 512-thread
+// workgroup per 64 x 8 tile exchanged the footprint, the faces and the fluxes
+// through LDS in four phases between barriers, with 668 instructions per row:
+// us per launch (stage, last stage, end of step; HIP events), before -> now
+//   512x1024 isothermal FP64        27.0  32.8  32.4  ->  20.7  24.6  23.4
+//   512x1024 isothermal FP32        18.8  23.9  23.1  ->  14.8  18.0  16.0
+//   1024x2048 isothermal FP64       83    107   96    ->  54    71    57
+//   1024x2048 Euler FP64, 7 stages  201   345   123   ->  114   196   95
+// Strips of 64 columns keep power-of-two meshes free of idle lanes; a strip of
+// 60 columns whose outer lanes are the halo needs no edge work but a ninth
+// strip at 512 columns.
+constexpr int SW = 64, SR = STRIP_ROWS, SWAVES = STRIP_WAVES;
+// LDS values of a strip's row: state of column -1, state and west face of the
+// column behind lane 63, flux through the first west interface, states of the
+// columns ce and ce+1 behind a strip of ce < 64 columns, and the y face offsets
+// of the row above
+template <int V>
+constexpr int HX = 6 * V + 2;
+
+// value of the lane before / after; the first / last lane takes `edge`
+template <int CTRL>
+__device__ __forceinline__ int dpp_shift(int edge, int v) {
+  return __builtin_amdgcn_update_dpp(edge, v, CTRL, 0xf, 0xf, false);
+}
+template <int CTRL, typename T>
+__device__ __forceinline__ T dpp_shift(T edge, T v) {
+  if constexpr (sizeof(T) == 8) {
+    const int2 e = __builtin_bit_cast(int2, edge), x = __builtin_bit_cast(int2, v);
+    return __builtin_bit_cast(T, make_int2(dpp_shift<CTRL>(e.x, x.x), dpp_shift<CTRL>(e.y, x.y)));
+  } else {
+    return __builtin_bit_cast(T, dpp_shift<CTRL>(__builtin_bit_cast(int, edge), __builtin_bit_cast(int, v)));
+  }
+}
+template <typename T>
+__device__ __forceinline__ T lane_prev(T edge, T v) { return dpp_shift<0x138, T>(edge, v); }  // wave_shr:1
+template <typename T>
+__device__ __forceinline__ T lane_next(T edge, T v) { return dpp_shift<0x130, T>(edge, v); }  // wave_shl:1
+
+// orders the edge lanes' LDS writes before the wave's reads of them
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// one row of a strip's inputs: the state and the NK slopes of the stage sum
+template <typename T, int V, int NK>
+struct RowIn {
+  T y[V], k[NK > 0 ? NK : 1][V];
+};
+
+// what a wave's rows leave for the workgroup's reduction
+struct StripOut {
+  double err, invdt;
+  int flags, halted;
+};
+
+template <typename T, int V, int LIM, int NK, int MODE>
+__device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T> &a, int bx, int j0, int nr, T *hx) {
+  constexpr bool kEnd = MODE == M_END, kLast = MODE == M_LAST;
+  using Row = RowIn<T, V, NK>;
+  using Comb = Combination<T, V, NK>;
+  // the last stage's sums over k_1 .. k_{s-1}: formed when a row arrives and
+  // kept through the march, or for few slopes (FP64) from a second read of the row
+  // when it is finished, which leaves registers for a second wave per SIMD
+  constexpr bool kReread = kLast && sizeof(T) == 8 && NK <= 2;
+  const bool want_cfl = kEnd && a.want_cfl, want_check = kEnd && a.want_check;
+  T *const yout = kEnd ? a.yout : nullptr;
+  T *const pout = kEnd ? a.pout : nullptr;
+  double *const vout = kEnd ? a.vout : nullptr;
+  const bool prim_rec = LIM == 0 && g.recon_prim;
+  const int lane = threadIdx.x & 63;
+  const int imin = GH, jmin = GH, imax = GH + g.inum - 1, jmax = GH + g.jnum - 1;
+  const int i0 = GH + bx * SW;
+  const int ce = min(SW, imax + 1 - i0);          // columns of this strip
+  const bool act = lane < ce;
+  const int i = act ? i0 + lane : imax;           // lanes beyond the mesh repeat its last column
+  const int iw = min(i0 + lane, imax + 1);        // (column ce's west face is needed)
+  const T zero = T(0);
+  const T invdx = (T)g.invdx, invdy = (T)g.invdy;
+  T cfl = -Real<T>::huge;
+  int flags = 0;
+
+  // rows are wave-uniform: row pointers stay in scalar registers
+  const int js_s = g.bc[2] == PERIODIC ? g.jnum : 0, js_n = g.bc[3] == PERIODIC ? g.jnum : 0;
+  auto source_row = [&](int j) {
+    if (j < jmin) return js_s ? j + js_s : jmin;
+    if (j > jmax) return js_n ? j - js_n : jmax;
+    return j;
+  };
+  // (byte offsets from scalar row pointers)
+  const unsigned lo = (unsigned)i * sizeof(T);
+  auto at = [&](const T *row) { return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(row) + lo); };
+  auto load_at = [&](int j, Row &R) {
+    const long base = (long)source_row(j) * g.P;
+#pragma unroll
+    for (int l = 0; l < V; l++) R.y[l] = at(a.Y + l * g.FS + base);
+#pragma unroll
+    for (int q = 0; q < NK; q++)
+#pragma unroll
+      for (int l = 0; l < V; l++) R.k[q][l] = at(a.k[q] + l * g.FS + base);
+  };
+  // Everything the strip needs before its march is loaded here, ahead of the
+  // first wait: one memory latency instead of a chain of them.  That includes
+  // the step's halt flag and dt (host-controlled launches read a dummy).
+  constexpr int PRE = NK * V <= 8 ? 4 : 1;
+  Row pre[4], re;
+#pragma unroll
+  for (int q = 0; q < PRE; q++) load_at(j0 - 2 + q, pre[q]);
+  // edge columns of all rows: lane = slot * SR + row, slots = columns -2, -1,
+  // 0, 1 and ce-1, ce, ce+1, ce-2; x ghost cells load the interior cell that
+  // their boundary rule starts from
+  const int er = lane % SR, eq = lane / SR;
+  const bool on = er < nr;
+  const int ii = i0 + (eq < 4 ? eq - 2 : eq == 7 ? ce - 2 : ce - 5 + eq), jj = on ? j0 + er : j0;
+  const bool xg = ii < imin || ii > imax;
+  const int east = ii > imax, bcx = east ? g.bc[1] : g.bc[0];
+  const int is = !xg ? ii : bcx == PERIODIC ? (east ? ii - g.inum : ii + g.inum) : east ? imax : imin;
+  {
+    const long ix = cidx(g, is, jj);
+#pragma unroll
+    for (int l = 0; l < V; l++) re.y[l] = (a.Y + l * g.FS)[ix];
+#pragma unroll
+    for (int q = 0; q < NK; q++)
+#pragma unroll
+      for (int l = 0; l < V; l++) re.k[q][l] = (a.k[q] + l * g.FS)[ix];
+  }
+  const AbsorbingSpeeds<T> as(g, east);
+  const T e_ws = rg<T>(g, R_W, is), e_w = rg<T>(g, R_W, ii), e_off = rg<T>(g, eq == 1 ? R_RDXE : R_RDXW, ii);
+  const T e_ds = cl<T>(g, C_RDYS, jj + 1), e_dn = cl<T>(g, C_RDYN, jj + 1);
+  const T e_csE = rg<T>(g, R_CSE, i0 - 1), e_csW = rg<T>(g, R_CSW, i0), e_dA = rg<T>(g, R_DAXW, i0);
+  const T dn1 = cl<T>(g, C_RDYN, j0 - 1), ds0 = cl<T>(g, C_RDYS, j0), dn0 = cl<T>(g, C_RDYN, j0);
+  // per-ring quantities of the lane's column
+  const T w = rg<T>(g, R_W, i);
+  const T dxw = rg<T>(g, R_RDXW, iw), dxe = rg<T>(g, R_RDXE, i);
+  const T csE = rg<T>(g, R_CSE, i), csWn = rg<T>(g, R_CSW, i + 1), csN = rg<T>(g, R_CSN, i), csS = rg<T>(g, R_CSS, i);
+  const T dAxn = rg<T>(g, R_DAXW, i + 1), dAy = rg<T>(g, R_DAYS, i);
+  const T dydzdV = rg<T>(g, R_DYDZDV, i), dzdxdV = rg<T>(g, R_DZDXDV, i);
+  const SourceRing<T, V> sr(g, a, i);
+  const int halt = *(a.ctl ? &a.ctl->halt : reinterpret_cast<const int *>(g.ring));
+  const double ctl_dt = *(a.ctl ? &a.ctl->dt : g.ring);
+  asm volatile("" ::: "memory");  // keeps the loads above this branch
+  if (a.ctl && halt) return {0.0, 0.0, 0, 1};
+  const In<T, V, NK, true> in(g, a, want_check, a.ctl ? ctl_dt : a.dt);
+
+  // ---- edge columns
+  {
+    T u[V], p[V], s[V], ur[V];
+    in.stage_sum(re.y, re.k, s);
+    in.to_prim(e_ws, s, ur, p);
+    T pl[V], pr[V];
+    if (bx == 0 || i0 + ce + 1 >= imax) {  // the two edge cells of an absorbing boundary
+      // (column imax is slot 4, or slot 5 where the next strip has one column)
+      const int sR = east ? 4 + imax - (i0 + ce - 1) : 3, sL = east ? (sR == 4 ? 7 : sR - 1) : 2;
+#pragma unroll
+      for (int l = 0; l < V; l++) pl[l] = __shfl(p[l], sL * SR + er, 64), pr[l] = __shfl(p[l], sR * SR + er, 64);
+    }
+    if (on && xg) {  // x ghost cells: also their part of the new state, the data checks and the CFL maximum
+      if (bcx == ABSORBING) absorbing_math<T, V>(east, as, in.gam, pl, pr, p);
+      in.ghost_from_prim(e_w, p, u, flags);
+      if (want_cfl) {
+        const T cs = (V == 4) ? sound_speed(in.gam, p[0], p[3]) : rg<T>(g, R_CS, ii);
+        cfl = fmax2(cfl, cell_invdt(g, ii, p[1], p[2], cs));
+      }
+      const unsigned ix = (unsigned)jj * (unsigned)g.P + (unsigned)ii;
+      if (yout) {
+#pragma unroll
+        for (int l = 0; l < V; l++) (yout + l * g.FS)[ix] = u[l];
+      }
+      if (pout) {
+#pragma unroll
+        for (int l = 0; l < V; l++) (pout + l * g.FS)[ix] = p[l];
+      }
+      if (vout) {  // (v - w) + w
+        const T vc = a.sub_bg ? p[2] : p[2] - e_w;
+        vout[ix] = (double)(vc + e_w);
+      }
+      if (prim_rec) {
+#pragma unroll
+        for (int l = 0; l < V; l++) u[l] = p[l];
+      }
+    } else {
+      in.comoving(e_w, s, ur, p, u);
+      if (prim_rec) in.prim_comoving(e_w, s, p, u);
+    }
+    T f[V], fr[V], fx[V], um[V], up[V], a1[V], a2[V], sl[V];
+#pragma unroll
+    for (int l = 0; l < V; l++) {
+      um[l] = __shfl(u[l], lane - SR, 64);
+      up[l] = __shfl(u[l], lane + SR, 64);
+      a1[l] = u[l] - um[l];
+      a2[l] = up[l] - u[l];
+    }
+    if (any_exact<T, LIM>(slopes<T, V, LIM>(g, a1, a2, um, up, sl))) slopes_exact<T, V, LIM>(g, a1, a2, um, up, sl);
+#pragma unroll
+    for (int l = 0; l < V; l++) {
+      f[l] = u[l] + invdx * sl[l] * e_off;
+      fr[l] = __shfl(f[l], lane + SR, 64);
+    }
+    if (prim_rec)
+      kt_flux_p<T, V>(g, 0, f, fr, e_csE, e_csW, e_dA, fx);
+    else
+      kt_flux<T, V>(g, 0, f, fr, e_csE, e_csW, e_dA, fx);
+    T *h = hx + er * HX<V>;
+    if (on && eq == 1) {
+#pragma unroll
+      for (int l = 0; l < V; l++) h[l] = u[l], h[3 * V + l] = fx[l];
+      h[6 * V] = e_ds;
+      h[6 * V + 1] = e_dn;
+    }
+    if (on && eq == 5) {
+#pragma unroll
+      for (int l = 0; l < V; l++) h[4 * V + l] = u[l], h[2 * V + l] = f[l];
+    }
+    if (on && eq == 6) {
+#pragma unroll
+      for (int l = 0; l < V; l++) h[5 * V + l] = u[l];
+    }
+    if (on && eq == (ce == SW ? 5 : 6)) {
+#pragma unroll
+      for (int l = 0; l < V; l++) h[V + l] = u[l];
+    }
+  }
+  wave_sync();
+
+  auto kt = [&](int d, const T *L, const T *R, T csL, T csR, T dA, T *F) {
+    if (prim_rec)
+      kt_flux_p<T, V>(g, d, L, R, csL, csR, dA, F);
+    else
+      kt_flux<T, V>(g, d, L, R, csL, csR, dA, F);
+  };
+
+  // state of row j0 + r from its loaded values, and for own rows the sources,
+  // the CFL term, the data checks, the new state and the combination's sums
+  auto enter = [&](int r, const Row &R, T *u, T *geo, T *ext, Comb &cb) {
+    const int j = j0 + r;
+    T s[V], ur[V], p[V];
+    in.stage_sum(R.y, R.k, s);
+    const unsigned ix = (unsigned)j * (unsigned)g.P + (unsigned)i;
+    if (j < jmin || j > jmax) {  // y ghost row
+      if (a.add_bg) frame_add<T, V>(s, w);
+      c2p<T, V>(s, p, in.gam);
+      in.ghost_from_prim(w, p, u, flags);
+      if (want_cfl) {
+        const T cs = (V == 4) ? sound_speed(in.gam, p[0], p[3]) : sr.cs;
+        cfl = fmax2(cfl, cell_invdt(sr.dlx, sr.dly, p[1], p[2], cs));
+      }
+      if (act && yout) {
+#pragma unroll
+        for (int l = 0; l < V; l++) (yout + l * g.FS)[ix] = u[l];
+      }
+      if (act && pout) {
+#pragma unroll
+        for (int l = 0; l < V; l++) (pout + l * g.FS)[ix] = p[l];
+      }
+      if (prim_rec) {
+#pragma unroll
+        for (int l = 0; l < V; l++) u[l] = p[l];
+      }
+      return;
+    }
+    in.transform_at(w, s, ur, p, u);
+    const bool own = r >= 0 && r < nr;
+    if (kEnd && own && act) {
+      if (yout) {
+#pragma unroll
+        for (int l = 0; l < V; l++) (yout + l * g.FS)[ix] = u[l];
+      }
+      if (vout) vout[ix] = (double)((p[2] - w) + w);  // pvar after SubtractBackgroundVelocityY, then + w again
+      if (pout) {
+#pragma unroll
+        for (int l = 0; l < V; l++) (pout + l * g.FS)[ix] = (l == 2 && a.sub_bg) ? p[2] - w : p[l];
+      }
+    }
+    if (prim_rec) in.prim_comoving(w, s, p, u);
+    if constexpr (kLast && !kReread) {
+      if (own) cb.begin(a, in.dt, R.y, R.k);
+    }
+    sr.sources(g, a, j, s, ur, p, geo, ext);
+    if (own) {
+      // CheckData (timedisc_base.f90:1666-1742) and CFL (timedisc_base.f90:818-909)
+      if (want_check) {
+        if (p[0] < (T)g.rhomin) flags |= F_RHOMIN;
+        if (V == 4 && p[3] < (T)g.pmin) flags |= F_PMIN;
+#pragma unroll
+        for (int l = 0; l < V; l++)
+          if (bad(p[l]) || bad(ur[l])) flags |= F_INVALID;
+      }
+      if (want_cfl) {
+        const T vy = a.sub_bg ? p[2] - w : p[2];
+        const T cs = (V == 4) ? sound_speed(in.gam, p[0], p[3]) : sr.cs;
+        cfl = fmax2(cfl, cell_invdt(sr.dlx, sr.dly, p[1], vy, cs));
+      }
+    }
+  };
+  // south and north faces of a row from its offsets and limited slopes
+  auto yfaces = [&](T ds, T dn, const T *u, const T *sl, T *fs, T *fn) {
+#pragma unroll
+    for (int l = 0; l < V; l++) {
+      const T sy = invdy * sl[l];
+      fs[l] = u[l] + sy * ds;
+      fn[l] = u[l] + sy * dn;
+    }
+  };
+
+  // ---- rows -2 .. 1: states, the faces of rows -1 and 0, the flux between them
+  T uA[V], uB[V], uC[V], dlo[V], fn[V], ys[V];
+  T geoA[V], extA[V], geoB[V], extB[V];
+  Comb cA, cB;
+  Row nx;
+  {
+    T fs[V], fn0[V], g0[V], e0[V], dmi[V], dhi[V], s1[V], s0[V], uD[V];
+    Comb c0;
+    if constexpr (PRE == 4) {
+      load_at(min(j0 + 2, jmax + 2), nx);
+      enter(-2, pre[0], uA, g0, e0, c0);
+      enter(-1, pre[1], uB, g0, e0, c0);
+      enter(0, pre[2], uC, geoA, extA, cA);
+      enter(1, pre[3], uD, geoB, extB, cB);
+    } else {
+      load_at(j0 - 1, nx);
+      enter(-2, pre[0], uA, g0, e0, c0);
+      load_at(j0, pre[0]);
+      enter(-1, nx, uB, g0, e0, c0);
+      load_at(j0 + 1, nx);
+      enter(0, pre[0], uC, geoA, extA, cA);
+      load_at(min(j0 + 2, jmax + 2), pre[0]);
+      enter(1, nx, uD, geoB, extB, cB);
+      nx = pre[0];
+    }
+#pragma unroll
+    for (int l = 0; l < V; l++) dlo[l] = uB[l] - uA[l], dmi[l] = uC[l] - uB[l], dhi[l] = uD[l] - uC[l];
+    const int t = min(slopes<T, V, LIM>(g, dlo, dmi, uA, uC, s1), slopes<T, V, LIM>(g, dmi, dhi, uB, uD, s0));
+    if (any_exact<T, LIM>(t)) {
+      slopes_exact<T, V, LIM>(g, dlo, dmi, uA, uC, s1);
+      slopes_exact<T, V, LIM>(g, dmi, dhi, uB, uD, s0);
+    }
+    yfaces(ds0, dn1, uB, s1, fs, fn0);  // (only the north face of row -1 is used)
+    yfaces(ds0, dn0, uC, s0, fs, fn);
+    kt(1, fn0, fs, csN, csS, dAy, ys);
+#pragma unroll
+    for (int l = 0; l < V; l++) uA[l] = uC[l], uB[l] = uD[l], dlo[l] = dhi[l];  // rows 0 and 1 next
+  }
+  // ---- march: row rr is finished when the row two above it has arrived
+  double err = -DBL_MAX;
+  for (int rr = 0; rr < nr; rr++) {
+    const int j = j0 + rr;
+    const Row cur = nx;
+    Row mine;
+    if constexpr (kReread) load_at(j, mine);
+    load_at(min(j + 3, jmax + 2), nx);
+    T uw[V], ue[V], fwe[V], fxw[V];
+    const T *h = hx + rr * HX<V>;
+#pragma unroll
+    for (int l = 0; l < V; l++) uw[l] = h[l], ue[l] = h[V + l], fwe[l] = h[2 * V + l], fxw[l] = h[3 * V + l];
+    const T ds = h[6 * V], dn = h[6 * V + 1];
+    if (ce < SW) {  // the two lanes behind a narrow strip hold the columns there
+#pragma unroll
+      for (int l = 0; l < V; l++) uA[l] = lane == ce ? h[4 * V + l] : lane == ce + 1 ? h[5 * V + l] : uA[l];
+    }
+    // the row two above; x slopes of row rr, y slopes of the row above it
+    T geoC[V], extC[V];
+    Comb cC;
+    enter(rr + 2, cur, uC, geoC, extC, cC);
+    T um[V], up[V], a1[V], a2[V], dhi[V], sx[V], sy[V];
+#pragma unroll
+    for (int l = 0; l < V; l++) {
+      um[l] = lane_prev(uw[l], uA[l]);
+      up[l] = lane_next(ue[l], uA[l]);
+      a1[l] = uA[l] - um[l];
+      a2[l] = up[l] - uA[l];
+      dhi[l] = uC[l] - uB[l];
+    }
+    const int t = min(slopes<T, V, LIM>(g, a1, a2, um, up, sx), slopes<T, V, LIM>(g, dlo, dhi, uA, uC, sy));
+    if (any_exact<T, LIM>(t)) {
+      slopes_exact<T, V, LIM>(g, a1, a2, um, up, sx);
+      slopes_exact<T, V, LIM>(g, dlo, dhi, uA, uC, sy);
+    }
+    // faces and fluxes
+    T xf[V], xw[V], fe[V], fr[V], fs[V], fnn[V], yf[V];
+#pragma unroll
+    for (int l = 0; l < V; l++) {
+      const T s = invdx * sx[l], fw = uA[l] + s * dxw;
+      fe[l] = uA[l] + s * dxe;
+      fr[l] = lane_next(fwe[l], fw);
+      dlo[l] = dhi[l];
+    }
+    yfaces(ds, dn, uB, sy, fs, fnn);
+    kt(0, fe, fr, csE, csWn, dAxn, xf);
+    kt(1, fn, fs, csN, csS, dAy, yf);
+#pragma unroll
+    for (int l = 0; l < V; l++) xw[l] = lane_prev(fxw[l], xf[l]);
+
+    // rhs assembly (timedisc_base.f90:1254-1271)
+    if (act) {
+      const unsigned ix = (unsigned)j * (unsigned)g.P + (unsigned)i;
+      T rhs[V];
+      // the viscous source joins the source list's sum last (sources_generic.f90:
+      // 236-241); it has no density component
+      if constexpr (sizeof(T) == 8) {
+        if (a.vsrc) {
+#pragma unroll
+          for (int l = 1; l < V; l++) extA[l] = extA[l] + (a.vsrc + (l - 1) * g.FS)[ix];
+        }
+      }
+#pragma unroll
+      for (int l = 0; l < V; l++) {
+        const T d = dydzdV * (xf[l] - xw[l]) + dzdxdV * (yf[l] - ys[l]);
+        rhs[l] = l == 0 ? d : d - geoA[l] - extA[l];
+      }
+      // boundary rows: the fluxes through the mesh boundary at the boundary
+      // cells' outer interfaces, Mesh%dy*Mesh%dz*xflux (W), -Mesh%dy*Mesh%dz*xflux
+      // (E) and likewise in y (timedisc_base.f90:1224-1252), stored at the ghost
+      // position next to the cell (the last stage: into bks).  bxs/bys: the x
+      // and y side of a boundary cell (0 W/S, 1 E/N, -1 none).
+      const int bxs = !a.bflux ? -1 : i == imin ? 0 : i == imax ? 1 : -1;
+      const int bys = !a.bflux ? -1 : j == jmin ? 0 : j == jmax ? 1 : -1;
+      if (bxs >= 0) {
+        const unsigned gx = (unsigned)j * (unsigned)g.P + (unsigned)(bxs == 0 ? imin - 1 : imax + 1);
+        const long bi = (long)bxs * g.NJ + j;
+#pragma unroll
+        for (int l = 0; l < V; l++) {
+          const T b = bxs == 0 ? (T)g.bdydz * xw[l] : -((T)g.bdydz * xf[l]);
+          if constexpr (kLast)
+            a.bks[bi + 2L * l * g.NJ] = (double)b;
+          else
+            (a.kout + l * g.FS)[gx] = b;
+        }
+      }
+      if (bys >= 0) {
+        const unsigned gy = (unsigned)(bys == 0 ? jmin - 1 : jmax + 1) * (unsigned)g.P + (unsigned)i;
+        const long bi = 2L * V * g.NJ + (long)bys * g.NI + i;
+#pragma unroll
+        for (int l = 0; l < V; l++) {
+          const T b = bys == 0 ? (T)g.bdzdx * ys[l] : -((T)g.bdzdx * yf[l]);
+          if constexpr (kLast)
+            a.bks[bi + 2L * l * g.NI] = (double)b;
+          else
+            (a.kout + l * g.FS)[gy] = b;
+        }
+      }
+      if constexpr (kReread) cA.begin(a, in.dt, mine.y, mine.k);
+      if constexpr (kLast)
+        err = fmax2(err, cA.finish(g, a, in.dt, ix, rhs));
+      else {
+#pragma unroll
+        for (int l = 0; l < V; l++) (a.kout + l * g.FS)[ix] = rhs[l];
+      }
+    }
+#pragma unroll
+    for (int l = 0; l < V; l++) {
+      uA[l] = uB[l];
+      uB[l] = uC[l];
+      fn[l] = fnn[l];
+      ys[l] = yf[l];
+      geoA[l] = geoB[l];
+      extA[l] = extB[l];
+      geoB[l] = geoC[l];
+      extB[l] = extC[l];
+    }
+    cA = cB;
+    cB = cC;
+  }
+
+  // CFL partials in FP64 (the maximum of FP32 values is exact)
+  return {err, cfl == -Real<T>::huge ? -DBL_MAX : (double)cfl, flags, 0};
+}
+
+// The end-of-step evaluation's auxiliary workgroups (k = 0 .. rhs_aux() - 1),
+// beside the strips so that no strip's wave waits for their remote loads:
+// k = 0 evaluates the corner ghost cells, which are in no strip (data checks,
+// CFL and the new state, SetCornerEdges, boundary_generic.f90:434-517); the
+// others make the step's boundary-flux accumulation (device-controlled steps).
+template <typename T, int V>
+__device__ __forceinline__ void rhs_aux_block(const Geom &g, const StageArgsT<T> &a, int k, int naux, int b) {
+  if (a.ctl && a.ctl->halt) return;
+  const double dt = a.ctl ? a.ctl->dt : a.dt;
+  const int t = threadIdx.x;
+  if (k > 0) {
+    if (a.bfa.out) bflux_accumulate(a.bfa, dt, (k - 1) * 64 * SWAVES + t, (naux - 1) * 64 * SWAVES);
+    return;
+  }
+  if (t >= 64 || !(a.want_cfl || a.want_check)) return;
+  T cfl = -Real<T>::huge;
+  int flags = 0;
+  if (t < 16) {
+    const int ga = 1 + (t & 1), gb = 1 + ((t >> 1) & 1), cE = (t >> 2) & 1, cN = t >> 3;
+    const int gi = cE ? GH + g.inum - 1 + ga : GH - ga, gj = cN ? GH + g.jnum - 1 + gb : GH - gb;
+    const In<T, V, 0, true> in(g, a, a.want_check, dt);
+    T u[V], p[V];
+    in.ghost_final(gi, gj, u, p, flags);
+    if (a.want_cfl) {
+      const T cs = (V == 4) ? sound_speed(in.gam, p[0], p[3]) : rg<T>(g, R_CS, gi);
+      cfl = cell_invdt(g, gi, p[1], p[2], cs);
+    }
+    const unsigned ix = (unsigned)gj * (unsigned)g.P + (unsigned)gi;
+    if (a.yout) {
+#pragma unroll
+      for (int l = 0; l < V; l++) (a.yout + l * g.FS)[ix] = u[l];
+    }
+    if (a.pout) {
+#pragma unroll
+      for (int l = 0; l < V; l++) (a.pout + l * g.FS)[ix] = p[l];
+    }
+  }
+  const double m = wave_max(cfl == -Real<T>::huge ? -DBL_MAX : (double)cfl);
+  const int f = wave_or(flags);
+  if (t == 0) {
+    a.part[2 * b] = m;
+    a.part[2 * b + 1] = (double)f;
+  }
+}
+
+// one workgroup: SWAVES strips of `rows` rows above each other
+template <typename T, int V, int LIM, int NK, int MODE>
+__device__ __forceinline__ void rhs_block(const Geom &g, const StageArgsT<T> &a, int rows, int bx, int by, int b) {
+  __shared__ T hx[SWAVES][SR * HX<V>];
+  __shared__ double redd[SWAVES];
+  __shared__ int redi[SWAVES];
+  const int t = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int j0 = GH + (by * SWAVES + wv) * rows, nr = min(rows, GH + g.jnum - j0);
+  StripOut o{-DBL_MAX, -DBL_MAX, 0, 0};
+  if (nr > 0)
+    o = rhs_strip<T, V, LIM, NK, MODE>(g, a, bx, j0, nr, hx[wv]);
+  else
+    o.halted = a.ctl && a.ctl->halt;
+  if (o.halted) return;
+  if constexpr (MODE == M_LAST) {
+    int unused = 0;
+    blk_max_or0(o.err, unused, redd, redi);
+    if (t == 0) {
+      a.part_c[2 * b] = o.err;
+      a.part_c[2 * b + 1] = 0.0;
+    }
+  }
+  if constexpr (MODE == M_END) {
+    if (!(a.want_cfl || a.want_check)) return;
+    blk_max_or0(o.invdt, o.flags, redd, redi);
+    if (t == 0) {
+      a.part[2 * b] = o.invdt;
+      a.part[2 * b + 1] = (double)o.flags;
+    }
+  }
+}
+
+// waves per SIMD the registers allow: the FP64 last stages keep three rows of
+// partial sums beside the march's window
+template <typename T, int V, int NK, int MODE>
+constexpr int strip_occupancy() {
+  return sizeof(T) == 8 && (MODE == M_LAST ? V * NK > 6 : V * NK > 12) ? 1 : 2;
+}
+template <typename T, int V, int LIM, int NK, int MODE>
+__global__ __launch_bounds__(64 * SWAVES, (strip_occupancy<T, V, NK, MODE>())) void k_rhs(Geom g, StageArgsT<T> a) {
+  const int nbx = strip_cols(g.inum), n = nbx * strip_blocks(g.jnum, g.rows), grid = xcd_grid(n);
+  const int t = xcd_tile(blockIdx.x, n), k = (int)blockIdx.x - grid;
+  if (k >= 0) {  // behind the strips' workgroups, so that the XCDs' shares of those stay even
+    if constexpr (MODE == M_END) rhs_aux_block<T, V>(g, a, k, gridDim.x - grid, n);
+  } else if (t < n) {
+    rhs_block<T, V, LIM, NK, MODE>(g, a, g.rows, t % nbx, t / nbx, t);
+  }
+}
+
+// Many meshes in one launch: block b runs the strips tiles[b] (TileCode) of
+// the mesh whose Geom and arguments of this launch are tab[disk]; the row
+// behind a mesh's last one holds its auxiliary workgroups.
+template <typename T, int V, int LIM, int NK, int MODE>
+__global__ __launch_bounds__(64 * SWAVES, (strip_occupancy<T, V, NK, MODE>())) void k_rhs_multi(
+    const RhsEntry *__restrict__ tab, const unsigned *__restrict__ tiles, int rows) {
+  const unsigned e = tiles[blockIdx.x];
+  if (e == NO_TILE) return;
+  const RhsEntry &E = tab[tile_disk(e)];
+  const StageArgsT<T> &a = reinterpret_cast<const StageArgsT<T> &>(E.a);
+  const int nbx = strip_cols(E.g.inum), nby = strip_blocks(E.g.jnum, rows), bx = tile_bx(e), by = tile_by(e);
+  if (by < nby)
+    rhs_block<T, V, LIM, NK, MODE>(E.g, a, rows, bx, by, bx + by * nbx);
+  else if (MODE == M_END)
+    rhs_aux_block<T, V>(E.g, a, bx, rhs_aux_max(E.g, V), nbx * nby);
+}
+
+}  // namespace fv

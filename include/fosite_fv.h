@@ -245,10 +245,11 @@ int fv_kernel_stats(const fv_ctx *ctx, int kernel, int *launches, double *ms, do
  * members take their steps on the host path).  A context belongs to at most one batch; fv_destroy
  * removes it from its batch.
  *
- * Tilings of the RHS kernels: 0 = 64-wide tiles in row-major order, 1 =
- * 64-wide tiles in XCD-chunked order (block b of the launch runs on XCD
- * b mod 8; each XCD gets a contiguous run of tiles, so neighbouring tiles
- * share that XCD's L2), 2 and 3 = the same with 32-wide tiles.  Every tiling
+ * Tilings of the RHS kernels, strips of 64 columns x up to 8 rows per wave: 0 =
+ * tall strips in row-major order, 1 = tall strips in XCD-chunked order (block b
+ * of the launch runs on XCD b mod 8; each XCD gets a contiguous run of strips,
+ * so neighbouring strips share that XCD's L2), 2 and 3 = the same with strips of
+ * half the rows.  Every tiling
  * gives the same bits.  With autotune, the first device steps of
  * fv_batch_run are timed under each tiling in turn (2 steps per trial, 2
  * trials per tiling), and the fastest is kept. */
