@@ -273,11 +273,6 @@ void prof_collect(fv_ctx *ctx) {
 double cells(const fv_ctx *ctx) { return (double)ctx->c.inum * ctx->c.jnum; }
 size_t elem_bytes(const fv_ctx *ctx) { return ctx->c.dtype == 1 ? sizeof(float) : sizeof(double); }
 double word_bytes(const fv_ctx *ctx) { return (double)elem_bytes(ctx) * ctx->V * cells(ctx); }
-// address of field l of a state buffer (element type by dtype)
-char *field(const fv_ctx *ctx, double *buf, int l) {
-  return reinterpret_cast<char *>(buf) + (size_t)l * ctx->FS * elem_bytes(ctx);
-}
-
 // reduce the per-block partials and fetch {max, flags} to the host
 int reduce(fv_ctx *ctx, const double *part, int n, double *mx, int *flags) {
   launch_reduce(part, n, ctx->d_red, ctx->st);
@@ -1351,23 +1346,28 @@ extern "C" int fv_set_background_velocity(fv_ctx *ctx, const double *w) {
   return upload_geom(ctx);
 }
 
-// the conservative state of all cells into buffer 0 (rounded to FP32 in the
-// precision form); the stored state then starts in the real frame
-static int upload_state(fv_ctx *ctx, const double *cv_in) {
+// the host's state of all cells into buffer 0 (rounded to FP32 in the
+// precision form), through the other state buffers; the stored state then
+// starts in the real frame
+static int upload_state(fv_ctx *ctx, const double *in, bool prim) {
   const int V = ctx->V;
   const size_t N = (size_t)ctx->NI * ctx->NJ;
-  ctx->cvar = ctx->cold = 0;
-  const size_t es = elem_bytes(ctx);
-  std::vector<float> cf;
-  const void *src = cv_in;
-  if (ctx->c.dtype == 1) {  // precision form: conserved variables from FP64, stored rounded
-    cf.assign(cv_in, cv_in + V * N);
-    src = cf.data();
+  // FP64: the V fields fit one buffer; FP32: one field in 1.5 (isothermal) or
+  // two (Euler) of a buffer
+  const int per = ctx->c.dtype == 1 ? (V == 4 ? 2 : 1) : V;
+  LoadArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.prim = prim;
+  for (int l = 0; l < V; l += per) {
+    const int n = std::min(per, V - l);
+    double *d = ctx->buf[1 + l / per];
+    HIPCHK(hipMemcpyAsync(d, in + l * N, sizeof(double) * n * N, hipMemcpyHostToDevice, ctx->st));
+    for (int q = 0; q < n; q++) a.in[l + q] = d + q * N;
   }
-  for (int l = 0; l < V; l++)
-    HIPCHK(hipMemcpy2DAsync(field(ctx, ctx->buf[0], l), es * ctx->P, static_cast<const char *>(src) + l * N * es,
-                            es * ctx->NI, es * ctx->NI, ctx->NJ, hipMemcpyHostToDevice, ctx->st));
+  launch_load(ctx->g, a, ctx->buf[0], V, ctx->st);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(ctx->st));
+  ctx->cvar = ctx->cold = 0;
   ctx->fl_pvar = ctx->fl_cvar = 0;
   ctx->have_state = true;
   ctx->pvalid = false;
@@ -1376,23 +1376,12 @@ static int upload_state(fv_ctx *ctx, const double *cv_in) {
 
 extern "C" int fv_set_pvar(fv_ctx *ctx, const double *pvar) {
   if (!ctx || !pvar) return -1;
-  const int V = ctx->V;
-  const size_t N = (size_t)ctx->NI * ctx->NJ;
-  std::vector<double> cv(V * N);
-  const double g = ctx->c.gamma;
-  for (size_t k = 0; k < N; k++) {  // Prim2Cons2d, all cells
-    const double rho = pvar[k], u = pvar[N + k], v = pvar[2 * N + k];
-    cv[k] = rho;
-    cv[N + k] = rho * u;
-    cv[2 * N + k] = rho * v;
-    if (V == 4) cv[3 * N + k] = pvar[3 * N + k] / (g - 1.) + 0.5 * rho * (u * u + v * v);
-  }
-  return upload_state(ctx, cv.data());
+  return upload_state(ctx, pvar, true);  // Prim2Cons2d, all cells
 }
 
 extern "C" int fv_set_cvar(fv_ctx *ctx, const double *cvar) {
   if (!ctx || !cvar) return -1;
-  return upload_state(ctx, cvar);
+  return upload_state(ctx, cvar, false);
 }
 
 extern "C" int fv_first_rhs(fv_ctx *ctx, int *brk) {
@@ -1551,48 +1540,25 @@ extern "C" int fv_get_state(fv_ctx *ctx, double *cvar, double *pvar) {
   if (!ctx) return -1;
   const int V = ctx->V;
   const size_t N = (size_t)ctx->NI * ctx->NJ;
-  std::vector<double> cv(V * N);
-  std::vector<float> cf(ctx->c.dtype == 1 ? V * N : 0);
-  const size_t es = elem_bytes(ctx);
-  char *dst = ctx->c.dtype == 1 ? reinterpret_cast<char *>(cf.data()) : reinterpret_cast<char *>(cv.data());
-  HIPCHK(hipStreamSynchronize(ctx->st));
-  for (int l = 0; l < V; l++)
-    HIPCHK(hipMemcpy2DAsync(dst + l * N * es, es * ctx->NI, field(ctx, ctx->buf[ctx->cvar], l), es * ctx->P,
-                            es * ctx->NI, ctx->NJ, hipMemcpyDeviceToHost, ctx->st));
-  HIPCHK(hipStreamSynchronize(ctx->st));
-  if (ctx->c.dtype == 1) std::copy(cf.begin(), cf.end(), cv.begin());
-  if (cvar) std::memcpy(cvar, cv.data(), sizeof(double) * V * N);
-  if (pvar && ctx->pvalid) {
-    // Timedisc%pvar of the last ComputeRHS, in the frame of the state: after
-    // an output-time AddBackgroundVelocityY (physics_eulerisotherm.f90:
-    // 1263-1303) the same + w as the reference applies to its pvar
-    std::vector<double> pv(V * N);
-    std::vector<float> pf(ctx->c.dtype == 1 ? V * N : 0);
-    char *pd = ctx->c.dtype == 1 ? reinterpret_cast<char *>(pf.data()) : reinterpret_cast<char *>(pv.data());
-    for (int l = 0; l < V; l++)
-      HIPCHK(hipMemcpy2DAsync(pd + l * N * es, es * ctx->NI, field(ctx, ctx->pbuf, l), es * ctx->P, es * ctx->NI,
-                              ctx->NJ, hipMemcpyDeviceToHost, ctx->st));
-    std::vector<double> w(ctx->NI, 0.0);
-    const bool addw = ctx->c.fargo && ctx->pflag && !ctx->fl_pvar;
-    if (addw)
-      HIPCHK(hipMemcpyAsync(w.data(), ring_tab(ctx, ctx->wcur) + (size_t)R_W * ctx->NI, sizeof(double) * ctx->NI,
-                            hipMemcpyDeviceToHost, ctx->st));
-    HIPCHK(hipStreamSynchronize(ctx->st));
-    if (ctx->c.dtype == 1) std::copy(pf.begin(), pf.end(), pv.begin());
-    if (addw)
-      for (int j = 0; j < ctx->NJ; j++)
-        for (int i = 0; i < ctx->NI; i++) pv[2 * N + (size_t)j * ctx->NI + i] += w[i];
-    std::memcpy(pvar, pv.data(), sizeof(double) * V * N);
-  } else if (pvar) {  // before FirstStep: Convert2Primitive of the state
-    const double g = ctx->c.gamma;
-    for (size_t k = 0; k < N; k++) {  // Cons2Prim2d
-      const double rho = cv[k], inv = 1. / rho, mu = cv[N + k], mv = cv[2 * N + k];
-      pvar[k] = rho;
-      pvar[N + k] = mu * inv;
-      pvar[2 * N + k] = mv * inv;
-      if (V == 4) pvar[3 * N + k] = (g - 1.) * (cv[3 * N + k] - 0.5 * inv * (mu * mu + mv * mv));
-    }
+  // packed into the two state buffers that hold neither cvar nor cold
+  const int a = pick_free(ctx, ctx->cvar, ctx->cold, -1), b = pick_free(ctx, ctx->cvar, ctx->cold, a);
+  // Timedisc%pvar of the last ComputeRHS, in the frame of the state: after an
+  // output-time AddBackgroundVelocityY (physics_eulerisotherm.f90:1263-1303)
+  // the same + w as the reference applies to its pvar.  Before FirstStep and
+  // after device-controlled steps: Convert2Primitive of the state.
+  const void *p = ctx->pvalid ? ctx->pbuf : nullptr;
+  const int addw = ctx->c.fargo && ctx->pflag && !ctx->fl_pvar;
+  // FP64: all fields at once; FP32: a buffer holds one field in FP64
+  const bool whole = ctx->c.dtype != 1;
+  for (int l = 0; l < (whole ? 1 : V); l++) {
+    launch_readout(ctx->g, ctx->buf[ctx->cvar], p, cvar ? ctx->buf[a] : nullptr, pvar ? ctx->buf[b] : nullptr,
+                   whole ? -1 : l, addw, V, ctx->st);
+    HIPCHK(hipGetLastError());
+    const size_t n = sizeof(double) * N * (whole ? V : 1);
+    if (cvar) HIPCHK(hipMemcpyAsync(cvar + l * N, ctx->buf[a], n, hipMemcpyDeviceToHost, ctx->st));
+    if (pvar) HIPCHK(hipMemcpyAsync(pvar + l * N, ctx->buf[b], n, hipMemcpyDeviceToHost, ctx->st));
   }
+  HIPCHK(hipStreamSynchronize(ctx->st));
   return 0;
 }
 

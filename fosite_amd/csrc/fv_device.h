@@ -231,6 +231,18 @@ void launch_remap(const Geom &g, const RemapArgs &a, int V, hipStream_t s);
 void launch_frame(const Geom &g, const void *src, void *dst, int sign, int V, hipStream_t s,
                   const Ctl *ctl = nullptr, const void *w2 = nullptr);
 void launch_reduce(const double *part, int n, double *out, hipStream_t s);
+// Host arrays of the C ABI ([V][NJ][NI], FP64) to and from state buffers.
+// k_readout: the conserved state u into oc and the primitive one into op (each
+// may be null): the stored pvar p (v + w when add_w), or Convert2Primitive of u
+// where p is null; field >= 0: that field only (oc and op then hold one field).
+void launch_readout(const Geom &g, const void *u, const void *p, double *oc, double *op, int field, int add_w, int V,
+                    hipStream_t s);
+// k_load: the V fields in[l] into the state u, prim: through Convert2Conservative
+struct LoadArgs {
+  const double *in[4];
+  int prim;
+};
+void launch_load(const Geom &g, const LoadArgs &a, void *u, int V, hipStream_t s);
 // CalcTimestep partials (max per block) from a stored pvar, v + w when add_w
 void launch_cfl_pvar(const Geom &g, const void *pv, int add_w, double *part, int nblocks, int V, hipStream_t s);
 // viscous source of the evaluation a into v.src (FP64)

@@ -245,6 +245,81 @@ void launch_visc_cfl(const Geom &g, const VisArgs &v, const double *pv, int add_
   else hipLaunchKernelGGL((k_visc_cfl<4>), dim3(nblocks), dim3(256), 0, s, g, v, pv, add_w, part);
 }
 
+// ------------------------------------------------ host arrays of the C ABI
+// The state's rows are padded to the pitch P and may be FP32; the host's
+// arrays are [V][NJ][NI] in FP64.  Packing on the device leaves one contiguous
+// copy per array: copies of pitched rows into pageable memory run at about 1 GB/s.
+// us for cvar and pvar, before -> now: 25600 -> 2100 at 512x1024 (isothermal,
+// 25 MB), 1950 -> 110 at 64x64 (Euler).
+template <typename T, int V>
+__global__ __launch_bounds__(256) void k_readout(Geom g, const T *__restrict__ u, const T *__restrict__ p, double *oc,
+                                                 double *op, int field, int add_w) {
+  const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y;
+  if (i >= g.NI || j >= g.NJ) return;
+  const long ix = cidx(g, i, j), k = (long)j * g.NI + i, N = (long)g.NI * g.NJ;
+  double c[V];
+#pragma unroll
+  for (int l = 0; l < V; l++) c[l] = (double)u[l * g.FS + ix];
+  double q[V];
+  if (op && p) {
+#pragma unroll
+    for (int l = 0; l < V; l++) q[l] = (double)p[l * g.FS + ix];
+    if (add_w) q[2] = q[2] + ring(g, R_W, i);
+  } else {  // Cons2Prim2d
+    const double inv = dvx(1.0, c[0]);
+    q[0] = c[0];
+    q[1] = c[1] * inv;
+    q[2] = c[2] * inv;
+    if constexpr (V == 4) q[3] = (g.gamma - 1.0) * (c[3] - 0.5 * inv * (c[1] * c[1] + c[2] * c[2]));
+  }
+#pragma unroll
+  for (int l = 0; l < V; l++) {
+    if (field >= 0 && l != field) continue;
+    const long o = field >= 0 ? k : l * N + k;
+    if (oc) oc[o] = c[l];
+    if (op) op[o] = q[l];
+  }
+}
+template <typename T, int V>
+__global__ __launch_bounds__(256) void k_load(Geom g, LoadArgs a, T *u) {
+  const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y;
+  if (i >= g.NI || j >= g.NJ) return;
+  const long ix = cidx(g, i, j), k = (long)j * g.NI + i;
+  double p[V], c[V];
+#pragma unroll
+  for (int l = 0; l < V; l++) c[l] = p[l] = a.in[l][k];
+  if (a.prim) {  // Prim2Cons2d
+    c[1] = p[0] * p[1];
+    c[2] = p[0] * p[2];
+    if constexpr (V == 4) c[3] = dvx(p[3], g.gamma - 1.0) + 0.5 * p[0] * (p[1] * p[1] + p[2] * p[2]);
+  }
+#pragma unroll
+  for (int l = 0; l < V; l++) u[l * g.FS + ix] = (T)c[l];
+}
+template <typename T>
+static void readout(const Geom &g, const void *u, const void *p, double *oc, double *op, int field, int add_w, int V,
+                    hipStream_t s) {
+  const dim3 grid((g.NI + 63) / 64, (g.NJ + 3) / 4), block(64, 4);
+  const T *tu = static_cast<const T *>(u), *tp = static_cast<const T *>(p);
+  if (V == 3) hipLaunchKernelGGL((k_readout<T, 3>), grid, block, 0, s, g, tu, tp, oc, op, field, add_w);
+  else hipLaunchKernelGGL((k_readout<T, 4>), grid, block, 0, s, g, tu, tp, oc, op, field, add_w);
+}
+void launch_readout(const Geom &g, const void *u, const void *p, double *oc, double *op, int field, int add_w, int V,
+                    hipStream_t s) {
+  if (g.dtype == 1) readout<float>(g, u, p, oc, op, field, add_w, V, s);
+  else readout<double>(g, u, p, oc, op, field, add_w, V, s);
+}
+void launch_load(const Geom &g, const LoadArgs &a, void *u, int V, hipStream_t s) {
+  const dim3 grid((g.NI + 63) / 64, (g.NJ + 3) / 4), block(64, 4);
+  if (g.dtype == 1) {
+    if (V == 3) hipLaunchKernelGGL((k_load<float, 3>), grid, block, 0, s, g, a, (float *)u);
+    else hipLaunchKernelGGL((k_load<float, 4>), grid, block, 0, s, g, a, (float *)u);
+  } else {
+    if (V == 3) hipLaunchKernelGGL((k_load<double, 3>), grid, block, 0, s, g, a, (double *)u);
+    else hipLaunchKernelGGL((k_load<double, 4>), grid, block, 0, s, g, a, (double *)u);
+  }
+}
+
 // ------------------------------------------------- static reduction scratch
 // The array's name is only meaningful in device code; host code uses the
 // address hipGetSymbolAddress returns for each device (each device holds its
