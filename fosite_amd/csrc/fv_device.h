@@ -264,7 +264,7 @@ void launch_wsum(const Geom &g, const double *v, double *ring, float *ringf, hip
                  const Ctl *ctl = nullptr);
 // k_rhs: strips of 64 columns x up to STRIP_ROWS rows, one per wave,
 // STRIP_WAVES of them above each other in a workgroup
-constexpr int STRIP_ROWS = 8, STRIP_WAVES = 4;
+constexpr int STRIP_ROWS = 16, STRIP_WAVES = 4;
 __host__ __device__ inline int strip_cols(int inum) { return (inum + 63) / 64; }
 __host__ __device__ inline int strip_blocks(int jnum, int rows) {
   return (jnum + rows * STRIP_WAVES - 1) / (rows * STRIP_WAVES);

@@ -59,7 +59,7 @@ __device__ __forceinline__ T fmax2(T a, T b) { return (b > a) ? b : a; }
 template <typename T>
 __device__ __forceinline__ T fsign(T a, T b) { return copysign(fabs(a), b); }
 template <typename T>
-__device__ __forceinline__ bool bad(T x) { return (x != x) || (x > Real<T>::huge); }
+__device__ __forceinline__ bool bad(T x) { return !(x <= Real<T>::huge); }  // NaN or +Inf, one compare
 // minimum and maximum as one instruction each: NaN-dropping like fmin2/fmax2
 // with a number as first argument (only the sign of a zero may differ)
 __device__ __forceinline__ double mn(double a, double b) { return __builtin_fmin(a, b); }

@@ -359,8 +359,10 @@ int rhs_blocks(const Geom &g) { return strip_cols(g.inum) * strip_blocks(g.jnum,
 // The fewest rows that still give no more waves than the chip's SIMDs hold well
 // (256 CUs of 4; one FP64 or two FP32 waves each): fewer rows leave a wave a
 // shorter serial march, more rows read and transform fewer halo rows (rows + 4
-// per strip).  us per 512x1024 step at 2, 4 and 8 rows: 100, 85, 79 in FP64,
-// 63, 56, 61 in FP32.
+// per strip).  us per step at 4, 8, 16 and 32 rows:
+//   512x1024 isothermal          FP64 78  78 113   -   FP32  55  60  88   -
+//   1024x2048 isothermal         FP64  - 213 203 215   FP32   - 126 128 158
+//   1024x2048 Euler, 7 stages    FP64  - 802 724 736   FP32   - 435 407 482
 int strip_rows(long wave_rows, int dtype) {
   const long waves = dtype == 1 ? 2048 : 1024, r = (wave_rows + waves - 1) / waves;
   return r < 1 ? 1 : r > STRIP_ROWS ? STRIP_ROWS : (int)r;

@@ -30,23 +30,30 @@ static void with_last_slopes(int nk, F f) {
     default: f(Slots<6>()); break;
   }
 }
-template <typename T, int V, int LIM>
-static void rhs_lim(const Geom &g, const StageArgsT<T> &a, hipStream_t s) {
+template <typename T, int V, int LIM, int RMAX>
+static void rhs_rows(const Geom &g, const StageArgsT<T> &a, hipStream_t s) {
   const int mode = rhs_mode(a), n = strip_cols(g.inum) * strip_blocks(g.jnum, g.rows);
   const dim3 grid(xcd_grid(n) + (mode == M_END ? rhs_aux(g, a) : 0)), block(64 * SWAVES);
   switch (mode) {
     case M_STAGE:
       with_stage_slopes(a.nk, [&](auto n) {
-        hipLaunchKernelGGL((k_rhs<T, V, LIM, decltype(n)::value, M_STAGE>), grid, block, 0, s, g, a);
+        hipLaunchKernelGGL((k_rhs<T, V, LIM, decltype(n)::value, M_STAGE, RMAX>), grid, block, 0, s, g, a);
       });
       break;
     case M_LAST:
       with_last_slopes(a.nk, [&](auto n) {
-        hipLaunchKernelGGL((k_rhs<T, V, LIM, decltype(n)::value, M_LAST>), grid, block, 0, s, g, a);
+        hipLaunchKernelGGL((k_rhs<T, V, LIM, decltype(n)::value, M_LAST, RMAX>), grid, block, 0, s, g, a);
       });
       break;
-    default: hipLaunchKernelGGL((k_rhs<T, V, LIM, 0, M_END>), grid, block, 0, s, g, a); break;
+    default: hipLaunchKernelGGL((k_rhs<T, V, LIM, 0, M_END, RMAX>), grid, block, 0, s, g, a); break;
   }
+}
+// strips of more than ER rows take a second pass over their edge columns, which
+// shorter ones leave out of their code (1.5 us of a 512x1024 step)
+template <typename T, int V, int LIM>
+static void rhs_lim(const Geom &g, const StageArgsT<T> &a, hipStream_t s) {
+  if (g.rows > ER) rhs_rows<T, V, LIM, STRIP_ROWS>(g, a, s);
+  else rhs_rows<T, V, LIM, ER>(g, a, s);
 }
 template <typename T, int V>
 void rhs_single(const Geom &g, const StageArgsT<T> &a, hipStream_t s) {
@@ -83,27 +90,33 @@ void frame_single(const Geom &g, const void *src, void *dst, int sign, int V, co
 
 // batches: van Leer compiled in, every other limiter (and mixed limiters) by
 // the run-time switch
-template <typename T, int V, int LIM>
-static void rhs_multi_lim(const RhsEntry *tab, const unsigned *tiles, int n, int rows, int mode, int nk,
+template <typename T, int V, int LIM, int RMAX>
+static void rhs_multi_rows(const RhsEntry *tab, const unsigned *tiles, int n, int rows, int mode, int nk,
                           hipStream_t s) {
   const dim3 block(64 * SWAVES);
   switch (mode) {
     case M_STAGE:
       with_stage_slopes(nk, [&](auto k) {
-        hipLaunchKernelGGL((k_rhs_multi<T, V, LIM, decltype(k)::value, M_STAGE>), dim3(n), block, 0, s, tab, tiles,
+        hipLaunchKernelGGL((k_rhs_multi<T, V, LIM, decltype(k)::value, M_STAGE, RMAX>), dim3(n), block, 0, s, tab, tiles,
                            rows);
       });
       break;
     case M_LAST:
       with_last_slopes(nk, [&](auto k) {
-        hipLaunchKernelGGL((k_rhs_multi<T, V, LIM, decltype(k)::value, M_LAST>), dim3(n), block, 0, s, tab, tiles,
+        hipLaunchKernelGGL((k_rhs_multi<T, V, LIM, decltype(k)::value, M_LAST, RMAX>), dim3(n), block, 0, s, tab, tiles,
                            rows);
       });
       break;
     default:
-      hipLaunchKernelGGL((k_rhs_multi<T, V, LIM, 0, M_END>), dim3(n), block, 0, s, tab, tiles, rows);
+      hipLaunchKernelGGL((k_rhs_multi<T, V, LIM, 0, M_END, RMAX>), dim3(n), block, 0, s, tab, tiles, rows);
       break;
   }
+}
+template <typename T, int V, int LIM>
+static void rhs_multi_lim(const RhsEntry *tab, const unsigned *tiles, int n, int rows, int mode, int nk,
+                          hipStream_t s) {
+  if (rows > ER) rhs_multi_rows<T, V, LIM, STRIP_ROWS>(tab, tiles, n, rows, mode, nk, s);
+  else rhs_multi_rows<T, V, LIM, ER>(tab, tiles, n, rows, mode, nk, s);
 }
 template <typename T, int V>
 void rhs_multi(const RhsEntry *tab, const unsigned *tiles, int n, int limiter, int rows, int mode, int nk,

@@ -5,7 +5,7 @@
 
 namespace fv {
 
-// A wave owns SW output columns (one lane each) and up to SR rows, and walks
+// A wave owns SW output columns (one lane each) and up to RMAX rows, and walks
 // its rows from the southern halo to the northern one:
 //   * the loads of a row are issued one row ahead of its arithmetic;
 //   * along y everything lives in registers: the state of three rows, the
@@ -32,7 +32,7 @@ namespace fv {
 // Strips of 64 columns keep power-of-two meshes free of idle lanes; a strip of
 // 60 columns whose outer lanes are the halo needs no edge work but a ninth
 // strip at 512 columns.
-constexpr int SW = 64, SR = STRIP_ROWS, SWAVES = STRIP_WAVES;
+constexpr int SW = 64, SWAVES = STRIP_WAVES, ER = 8;
 // LDS values of a strip's row: state of column -1, state and west face of the
 // column behind lane 63, flux through the first west interface, states of the
 // columns ce and ce+1 behind a strip of ce < 64 columns, and the y face offsets
@@ -78,15 +78,15 @@ struct StripOut {
   int flags, halted;
 };
 
-template <typename T, int V, int LIM, int NK, int MODE>
+template <typename T, int V, int LIM, int NK, int MODE, int RMAX>
 __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T> &a, int bx, int j0, int nr, T *hx) {
   constexpr bool kEnd = MODE == M_END, kLast = MODE == M_LAST;
   using Row = RowIn<T, V, NK>;
   using Comb = Combination<T, V, NK>;
   // the last stage's sums over k_1 .. k_{s-1}: formed when a row arrives and
-  // kept through the march, or for few slopes (FP64) from a second read of the row
-  // when it is finished, which leaves registers for a second wave per SIMD
-  constexpr bool kReread = kLast && sizeof(T) == 8 && NK <= 2;
+  // kept through the march, or for few slopes from a second read of the row when
+  // it is finished, which leaves registers for more waves per SIMD
+  constexpr bool kReread = kLast && NK <= 2;
   const bool want_cfl = kEnd && a.want_cfl, want_check = kEnd && a.want_check;
   T *const yout = kEnd ? a.yout : nullptr;
   T *const pout = kEnd ? a.pout : nullptr;
@@ -130,16 +130,17 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
   Row pre[4], re;
 #pragma unroll
   for (int q = 0; q < PRE; q++) load_at(j0 - 2 + q, pre[q]);
-  // edge columns of all rows: lane = slot * SR + row, slots = columns -2, -1,
-  // 0, 1 and ce-1, ce, ce+1, ce-2; x ghost cells load the interior cell that
-  // their boundary rule starts from
-  const int er = lane % SR, eq = lane / SR;
-  const bool on = er < nr;
-  const int ii = i0 + (eq < 4 ? eq - 2 : eq == 7 ? ce - 2 : ce - 5 + eq), jj = on ? j0 + er : j0;
+  // edge columns of ER rows at a time: lane = slot * ER + row, slots = columns
+  // -2, -1, 0, 1 and ce-1, ce, ce+1, ce-2; x ghost cells load the interior cell
+  // that their boundary rule starts from
+  const int er = lane % ER, eq = lane / ER;
+  const int ii = i0 + (eq < 4 ? eq - 2 : eq == 7 ? ce - 2 : ce - 5 + eq);
   const bool xg = ii < imin || ii > imax;
   const int east = ii > imax, bcx = east ? g.bc[1] : g.bc[0];
   const int is = !xg ? ii : bcx == PERIODIC ? (east ? ii - g.inum : ii + g.inum) : east ? imax : imin;
-  {
+  T e_ds, e_dn;  // y face offsets of the row above
+  auto load_edge = [&](int e0) {
+    const int jj = min(j0 + e0 + er, j0 + nr - 1);
     const long ix = cidx(g, is, jj);
 #pragma unroll
     for (int l = 0; l < V; l++) re.y[l] = (a.Y + l * g.FS)[ix];
@@ -147,10 +148,12 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
     for (int q = 0; q < NK; q++)
 #pragma unroll
       for (int l = 0; l < V; l++) re.k[q][l] = (a.k[q] + l * g.FS)[ix];
-  }
+    e_ds = cl<T>(g, C_RDYS, jj + 1);
+    e_dn = cl<T>(g, C_RDYN, jj + 1);
+  };
+  load_edge(0);
   const AbsorbingSpeeds<T> as(g, east);
   const T e_ws = rg<T>(g, R_W, is), e_w = rg<T>(g, R_W, ii), e_off = rg<T>(g, eq == 1 ? R_RDXE : R_RDXW, ii);
-  const T e_ds = cl<T>(g, C_RDYS, jj + 1), e_dn = cl<T>(g, C_RDYN, jj + 1);
   const T e_csE = rg<T>(g, R_CSE, i0 - 1), e_csW = rg<T>(g, R_CSW, i0), e_dA = rg<T>(g, R_DAXW, i0);
   const T dn1 = cl<T>(g, C_RDYN, j0 - 1), ds0 = cl<T>(g, C_RDYS, j0), dn0 = cl<T>(g, C_RDYN, j0);
   // per-ring quantities of the lane's column
@@ -167,7 +170,9 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
   const In<T, V, NK, true> in(g, a, want_check, a.ctl ? ctl_dt : a.dt);
 
   // ---- edge columns
-  {
+  for (int e0 = 0;;) {
+    const int jj = j0 + e0 + er;
+    const bool on = e0 + er < nr;
     T u[V], p[V], s[V], ur[V];
     in.stage_sum(re.y, re.k, s);
     in.to_prim(e_ws, s, ur, p);
@@ -176,7 +181,7 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
       // (column imax is slot 4, or slot 5 where the next strip has one column)
       const int sR = east ? 4 + imax - (i0 + ce - 1) : 3, sL = east ? (sR == 4 ? 7 : sR - 1) : 2;
 #pragma unroll
-      for (int l = 0; l < V; l++) pl[l] = __shfl(p[l], sL * SR + er, 64), pr[l] = __shfl(p[l], sR * SR + er, 64);
+      for (int l = 0; l < V; l++) pl[l] = __shfl(p[l], sL * ER + er, 64), pr[l] = __shfl(p[l], sR * ER + er, 64);
     }
     if (on && xg) {  // x ghost cells: also their part of the new state, the data checks and the CFL maximum
       if (bcx == ABSORBING) absorbing_math<T, V>(east, as, in.gam, pl, pr, p);
@@ -209,8 +214,8 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
     T f[V], fr[V], fx[V], um[V], up[V], a1[V], a2[V], sl[V];
 #pragma unroll
     for (int l = 0; l < V; l++) {
-      um[l] = __shfl(u[l], lane - SR, 64);
-      up[l] = __shfl(u[l], lane + SR, 64);
+      um[l] = __shfl(u[l], lane - ER, 64);
+      up[l] = __shfl(u[l], lane + ER, 64);
       a1[l] = u[l] - um[l];
       a2[l] = up[l] - u[l];
     }
@@ -218,13 +223,13 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
 #pragma unroll
     for (int l = 0; l < V; l++) {
       f[l] = u[l] + invdx * sl[l] * e_off;
-      fr[l] = __shfl(f[l], lane + SR, 64);
+      fr[l] = __shfl(f[l], lane + ER, 64);
     }
     if (prim_rec)
       kt_flux_p<T, V>(g, 0, f, fr, e_csE, e_csW, e_dA, fx);
     else
       kt_flux<T, V>(g, 0, f, fr, e_csE, e_csW, e_dA, fx);
-    T *h = hx + er * HX<V>;
+    T *h = hx + (e0 + er) * HX<V>;
     if (on && eq == 1) {
 #pragma unroll
       for (int l = 0; l < V; l++) h[l] = u[l], h[3 * V + l] = fx[l];
@@ -243,6 +248,9 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
 #pragma unroll
       for (int l = 0; l < V; l++) h[V + l] = u[l];
     }
+    if constexpr (RMAX <= ER) break;
+    if ((e0 += ER) >= nr) break;
+    load_edge(e0);
   }
   wave_sync();
 
@@ -303,11 +311,12 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
     if (own) {
       // CheckData (timedisc_base.f90:1666-1742) and CFL (timedisc_base.f90:818-909)
       if (want_check) {
-        if (p[0] < (T)g.rhomin) flags |= F_RHOMIN;
-        if (V == 4 && p[3] < (T)g.pmin) flags |= F_PMIN;
+        flags |= p[0] < (T)g.rhomin ? F_RHOMIN : 0;
+        if (V == 4) flags |= p[3] < (T)g.pmin ? F_PMIN : 0;
+        bool inv = false;
 #pragma unroll
-        for (int l = 0; l < V; l++)
-          if (bad(p[l]) || bad(ur[l])) flags |= F_INVALID;
+        for (int l = 0; l < V; l++) inv = inv | bad(p[l]) | bad(ur[l]);
+        flags |= inv ? F_INVALID : 0;
       }
       if (want_cfl) {
         const T vy = a.sub_bg ? p[2] - w : p[2];
@@ -535,16 +544,16 @@ __device__ __forceinline__ void rhs_aux_block(const Geom &g, const StageArgsT<T>
 }
 
 // one workgroup: SWAVES strips of `rows` rows above each other
-template <typename T, int V, int LIM, int NK, int MODE>
+template <typename T, int V, int LIM, int NK, int MODE, int RMAX>
 __device__ __forceinline__ void rhs_block(const Geom &g, const StageArgsT<T> &a, int rows, int bx, int by, int b) {
-  __shared__ T hx[SWAVES][SR * HX<V>];
+  __shared__ T hx[SWAVES][RMAX * HX<V>];
   __shared__ double redd[SWAVES];
   __shared__ int redi[SWAVES];
   const int t = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int j0 = GH + (by * SWAVES + wv) * rows, nr = min(rows, GH + g.jnum - j0);
   StripOut o{-DBL_MAX, -DBL_MAX, 0, 0};
   if (nr > 0)
-    o = rhs_strip<T, V, LIM, NK, MODE>(g, a, bx, j0, nr, hx[wv]);
+    o = rhs_strip<T, V, LIM, NK, MODE, RMAX>(g, a, bx, j0, nr, hx[wv]);
   else
     o.halted = a.ctl && a.ctl->halt;
   if (o.halted) return;
@@ -572,21 +581,21 @@ template <typename T, int V, int NK, int MODE>
 constexpr int strip_occupancy() {
   return sizeof(T) == 8 && (MODE == M_LAST ? V * NK > 6 : V * NK > 12) ? 1 : 2;
 }
-template <typename T, int V, int LIM, int NK, int MODE>
+template <typename T, int V, int LIM, int NK, int MODE, int RMAX>
 __global__ __launch_bounds__(64 * SWAVES, (strip_occupancy<T, V, NK, MODE>())) void k_rhs(Geom g, StageArgsT<T> a) {
   const int nbx = strip_cols(g.inum), n = nbx * strip_blocks(g.jnum, g.rows), grid = xcd_grid(n);
   const int t = xcd_tile(blockIdx.x, n), k = (int)blockIdx.x - grid;
   if (k >= 0) {  // behind the strips' workgroups, so that the XCDs' shares of those stay even
     if constexpr (MODE == M_END) rhs_aux_block<T, V>(g, a, k, gridDim.x - grid, n);
   } else if (t < n) {
-    rhs_block<T, V, LIM, NK, MODE>(g, a, g.rows, t % nbx, t / nbx, t);
+    rhs_block<T, V, LIM, NK, MODE, RMAX>(g, a, g.rows, t % nbx, t / nbx, t);
   }
 }
 
 // Many meshes in one launch: block b runs the strips tiles[b] (TileCode) of
 // the mesh whose Geom and arguments of this launch are tab[disk]; the row
 // behind a mesh's last one holds its auxiliary workgroups.
-template <typename T, int V, int LIM, int NK, int MODE>
+template <typename T, int V, int LIM, int NK, int MODE, int RMAX>
 __global__ __launch_bounds__(64 * SWAVES, (strip_occupancy<T, V, NK, MODE>())) void k_rhs_multi(
     const RhsEntry *__restrict__ tab, const unsigned *__restrict__ tiles, int rows) {
   const unsigned e = tiles[blockIdx.x];
@@ -595,7 +604,7 @@ __global__ __launch_bounds__(64 * SWAVES, (strip_occupancy<T, V, NK, MODE>())) v
   const StageArgsT<T> &a = reinterpret_cast<const StageArgsT<T> &>(E.a);
   const int nbx = strip_cols(E.g.inum), nby = strip_blocks(E.g.jnum, rows), bx = tile_bx(e), by = tile_by(e);
   if (by < nby)
-    rhs_block<T, V, LIM, NK, MODE>(E.g, a, rows, bx, by, bx + by * nbx);
+    rhs_block<T, V, LIM, NK, MODE, RMAX>(E.g, a, rows, bx, by, bx + by * nbx);
   else if (MODE == M_END)
     rhs_aux_block<T, V>(E.g, a, bx, rhs_aux_max(E.g, V), nbx * nby);
 }

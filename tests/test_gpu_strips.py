@@ -41,8 +41,10 @@ def test_gpu_strip_edges(problem, ni, nj):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nj", [3701, 5001])
 @pytest.mark.parametrize("problem", ["euler_nograd", "disk_fargo"])
-def test_gpu_tall_strips(problem):
-    """Two strips of columns, 3701 rows: eight rows per strip, five in the last."""
-    print("tall strips", problem, flush=True)
-    compare(PROBLEMS[problem](65, 3701), 2)
+def test_gpu_tall_strips(problem, nj):
+    """Two strips of columns; 3701 rows: eight rows per strip, five in the last;
+    5001: ten rows (the edge columns in two passes), one in the last."""
+    print("tall strips", problem, nj, flush=True)
+    compare(PROBLEMS[problem](65, nj), 2)
