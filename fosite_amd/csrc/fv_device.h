@@ -57,7 +57,8 @@ struct Geom {
 // and the host redoes that step itself.
 enum HaltReason { H_NONE = 0, H_ERR = 1, H_DTLIMIT = 2, H_FLAGS = 3, H_OUTPUT = 4, H_STOP = 5, H_BATCH = 6 };
 struct CtlHead {
-  double time, dt, dt_step, t_out, stoptime, cfl, dtlimit, maxerrold, beta, order;
+  double time, dt;  // adjacent: k_remap reads both through &time
+  double dt_step, t_out, stoptime, cfl, dtlimit, maxerrold, beta, order;
   double invdt;
   double cvis, invdt_v;  // viscosity (vis = 1): its Courant number and the last step's viscous 1/dt
   int halt, reason, step, nsteps, flags, vis;

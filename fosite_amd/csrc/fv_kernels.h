@@ -1095,21 +1095,25 @@ __device__ __forceinline__ void ycell(const Geom &g, const T *Y, int i, int jj, 
 // own five.
 template <typename T, int V>
 __device__ __forceinline__ void remap_block(const Geom &g, const RemapArgsT<T> &a, int bx, int by) {
-  if (a.ctl && a.ctl->halt) return;
-  double dts = a.dt_step;
-  if (a.ctl) {  // this%dt as AcceptSolution will set it
-    const double t = a.ctl->time, dt = a.ctl->dt;
-    dts = (t + dt) - t;
-  }
   constexpr int RR = REMAP_ROWS;
   const int i = GH + bx * 64 + threadIdx.x, jb = (by * 4 + threadIdx.y) * RR;
   if (i >= GH + g.inum || jb >= g.jnum) return;
   const int jmin = GH, J = g.jnum;
-  double dd = ring(g, R_W, i) * dts / ring(g, R_DLY, i);
+  // the step control and the ring's values in one memory latency
+  // (host-controlled launches read dummies)
+  const double *h = a.ctl ? &a.ctl->time : g.ring;
+  const double t = h[0], dt = h[1], w = ring(g, R_W, i), dly = ring(g, R_DLY, i);
+  const int halt = *(a.ctl ? &a.ctl->halt : reinterpret_cast<const int *>(g.ring));
+  if (a.ctl && halt) return;
+  const double dts = a.ctl ? (t + dt) - t : a.dt_step;  // this%dt as AcceptSolution will set it
+  double dd = w * dts / dly;
   const double shift = round(dd);
   const T d = (T)(dd - shift);
-  // source row of the first row: jmin + ((jb - shift) mod J); fmod is exact
-  int j0 = jb - (int)fmod(shift, (double)J);
+  // source row of the first row: jmin + ((jb - shift) mod J); shifts of more
+  // than a ring are rare, and the exact fmod is slow
+  int m = fabs(shift) < 2147483648.0 ? (int)shift : (int)fmod(shift, (double)J);
+  if (__any(m >= J || m <= -J)) m %= J;
+  int j0 = jb - m;
   if (j0 < 0) j0 += J;
   if (j0 >= J) j0 -= J;
   const int nr = J - jb < RR ? J - jb : RR;
