@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cfloat>
 #include <cstddef>
 #include <cstdlib>
@@ -179,7 +180,8 @@ struct fv_ctx {
   int batch_steps = 0, batch_halts = 0;
   fv_batch *batch = nullptr;  // batch this context belongs to
   double *part_r = nullptr, *part_c = nullptr;  // per-block partials: CFL/checks, embedded error
-  double *d_red = nullptr, *h_red = nullptr;
+  double *h_red = nullptr;  // pinned: {max, flags, number} of the last reduction
+  double red_no = 0;
   int nb_rhs = 0;
   hipStream_t st = nullptr;
   int dev = 0;  // the device current at fv_create, which holds the state
@@ -273,16 +275,35 @@ void prof_collect(fv_ctx *ctx) {
 double cells(const fv_ctx *ctx) { return (double)ctx->c.inum * ctx->c.jnum; }
 size_t elem_bytes(const fv_ctx *ctx) { return ctx->c.dtype == 1 ? sizeof(float) : sizeof(double); }
 double word_bytes(const fv_ctx *ctx) { return (double)elem_bytes(ctx) * ctx->V * cells(ctx); }
-// reduce the per-block partials and fetch {max, flags} to the host
-int reduce(fv_ctx *ctx, const double *part, int n, double *mx, int *flags) {
-  launch_reduce(part, n, ctx->d_red, ctx->st);
+// Reduction of the per-block partials to {max, flags} in pinned host memory:
+// the kernel writes the result and then the call's number there itself, and
+// the host watches that number.  A copy command and hipStreamSynchronize
+// behind the kernel took about 8 us more for each of a host-controlled step's
+// two waits.  Work queued after the kernel is not waited for.
+int reduce_start(fv_ctx *ctx, const double *part, int n) {
+  launch_reduce(part, n, ctx->h_red, ++ctx->red_no, ctx->st);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(ctx->h_red, ctx->d_red, 2 * sizeof(double), hipMemcpyDeviceToHost, ctx->st));
-  HIPCHK(hipStreamSynchronize(ctx->st));
-  prof_collect(ctx);
-  *mx = ctx->h_red[0];
-  *flags = (int)ctx->h_red[1];
   return 0;
+}
+int reduce_wait(fv_ctx *ctx, double *mx, int *flags) {
+  const volatile double *h = ctx->h_red;
+  // (a failed launch or device never writes the number: the stream's own
+  // synchronisation then returns the error)
+  for (long spin = 0; h[2] != ctx->red_no; spin++)
+    if (spin == 100000 || ctx->prof) {
+      HIPCHK(hipStreamSynchronize(ctx->st));
+      break;
+    }
+  std::atomic_thread_fence(std::memory_order_acquire);
+  if (h[2] != ctx->red_no) return fail(ctx, "reduction result missing", -3);
+  prof_collect(ctx);
+  *mx = h[0];
+  *flags = (int)h[1];
+  return 0;
+}
+int reduce(fv_ctx *ctx, const double *part, int n, double *mx, int *flags) {
+  const int rc = reduce_start(ctx, part, n);
+  return rc ? rc : reduce_wait(ctx, mx, flags);
 }
 
 // gravitational acceleration rings of an evaluation: point-mass state q
@@ -532,14 +553,15 @@ int solve_ode(fv_ctx *ctx, double time, double *dt, double *err) {
     int rc = rhs_stage(ctx, m, *dt, outb, time + ctx->tab.c[m] * *dt);
     if (rc) return rc;
   }
-  launch_bflux(bflux_args(ctx, ctx->k0cur, ctx->bcur, *dt), ctx->st);
+  int rc = reduce_start(ctx, ctx->part_c, ctx->nb_rhs);
+  if (rc) return rc;
+  launch_bflux(bflux_args(ctx, ctx->k0cur, ctx->bcur, *dt), ctx->st);  // (runs while the host decides)
   HIPCHK(hipGetLastError());
   ctx->fl_ctmp = ctx->fl_cvar;  // ctmp = cvar
   ctx->cvar = outb;
   double e;
   int f;
-  int rc = reduce(ctx, ctx->part_c, ctx->nb_rhs, &e, &f);
-  if (rc) return rc;
+  if ((rc = reduce_wait(ctx, &e, &f))) return rc;
   if (ctx->c.tol_rel <= 1.0) {
     *err = e;
     *dt = adjust_timestep(ctx, e, *dt);
@@ -1167,10 +1189,11 @@ extern "C" int fv_create(fv_ctx **out, const fv_config *cfg) {
   ctx->nb_rhs = rhs_blocks(g);
   const int nb_part = strip_cols(c.inum) * strip_blocks(c.jnum, 1) + 1;  // the finest tiling, which batches may choose
   ok = ok && dalloc(&ctx->part_r, sizeof(double) * 2 * nb_part) &&
-       dalloc(&ctx->part_c, sizeof(double) * 2 * nb_part) && dalloc(&ctx->d_red, sizeof(double) * 2);
+       dalloc(&ctx->part_c, sizeof(double) * 2 * nb_part);
   ok = ok && hipMalloc((void **)&ctx->d_ctl, sizeof(Ctl)) == hipSuccess &&
        hipMemsetAsync(ctx->d_ctl, 0, sizeof(Ctl), ctx->st) == hipSuccess && hipStreamSynchronize(ctx->st) == hipSuccess;
-  ok = ok && hipHostMalloc((void **)&ctx->h_red, sizeof(double) * 2) == hipSuccess;
+  ok = ok && hipHostMalloc((void **)&ctx->h_red, sizeof(double) * 3) == hipSuccess;
+  if (ok) std::memset(ctx->h_red, 0, sizeof(double) * 3);
   ok = ok && hipHostMalloc((void **)&ctx->h_ctl, sizeof(Ctl)) == hipSuccess;
   for (int q = 0; q < 2 && ok && c.outbound; q++) {
     ok = dalloc(&ctx->grav[q], sizeof(double) * (PM_HDR + 2 * ctx->NI));
@@ -1285,7 +1308,6 @@ extern "C" int fv_destroy(fv_ctx *ctx) {
   if (ctx->bks) (void)hipFree(ctx->bks);
   if (ctx->part_r) (void)hipFree(ctx->part_r);
   if (ctx->part_c) (void)hipFree(ctx->part_c);
-  if (ctx->d_red) (void)hipFree(ctx->d_red);
   if (ctx->d_ctl) (void)hipFree(ctx->d_ctl);
   if (ctx->d_ring) (void)hipFree(ctx->d_ring);
   if (ctx->d_col) (void)hipFree(ctx->d_col);
@@ -1495,7 +1517,7 @@ extern "C" int fv_step(fv_ctx *ctx, int *done) {
 }
 
 // fv_step with the reduction scratch of its kernels (per-workgroup partials
-// of the end-of-step evaluation and of the last stage, the reduction result)
+// of the end-of-step evaluation and of the last stage)
 // in the library's static device array instead of the context's buffers: the
 // call allocates no device or pinned memory.  Every call on one device shares
 // that array; the partials are written by every workgroup before they are
@@ -1512,14 +1534,12 @@ extern "C" int fv_step_noalloc(fv_ctx *ctx, int *done) {
   if (cur != ctx->dev) return fail(ctx, "fv_step_noalloc: the context's device is not the current device");
   double *s = nullptr;
   HIPCHK(scratch_address(ctx->dev, &s));
-  double *const own[3] = {ctx->part_r, ctx->part_c, ctx->d_red};
+  double *const own[2] = {ctx->part_r, ctx->part_c};
   ctx->part_r = s + SCRATCH_PART_R;
   ctx->part_c = s + SCRATCH_PART_C;
-  ctx->d_red = s + SCRATCH_RED;
   const int rc = fv_step(ctx, done);
   ctx->part_r = own[0];
   ctx->part_c = own[1];
-  ctx->d_red = own[2];
   return rc;
 }
 

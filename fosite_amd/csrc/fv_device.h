@@ -231,7 +231,8 @@ void launch_remap(const Geom &g, const RemapArgs &a, int V, hipStream_t s);
 // applied in the same pass)
 void launch_frame(const Geom &g, const void *src, void *dst, int sign, int V, hipStream_t s,
                   const Ctl *ctl = nullptr, const void *w2 = nullptr);
-void launch_reduce(const double *part, int n, double *out, hipStream_t s);
+// out (pinned host memory): max, flags, then no
+void launch_reduce(const double *part, int n, double *out, double no, hipStream_t s);
 // Host arrays of the C ABI ([V][NJ][NI], FP64) to and from state buffers.
 // k_readout: the conserved state u into oc and the primitive one into op (each
 // may be null): the stored pvar p (v + w when add_w), or Convert2Primitive of u
@@ -298,12 +299,11 @@ void launch_bflux_multi(const BfluxArgs *tab, int n, int bpm, hipStream_t s);
 void launch_accrete_multi(const AccreteArgs *tab, int n, hipStream_t s);
 
 // Reduction scratch of the allocation-free step (fv_step_noalloc): a static
-// device array, one copy per device, laid out as the reduction result (2
-// values), then the per-workgroup partials of the end-of-step evaluation and
+// device array, one copy per device, laid out as the per-workgroup partials of the end-of-step evaluation and
 // of the last stage (2 values per workgroup each).  At most
 // SCRATCH_MAX_BLOCKS workgroups per launch.
 constexpr int SCRATCH_MAX_BLOCKS = 16384;
-constexpr int SCRATCH_RED = 0, SCRATCH_PART_R = 32, SCRATCH_PART_C = SCRATCH_PART_R + 2 * SCRATCH_MAX_BLOCKS;
+constexpr int SCRATCH_PART_R = 0, SCRATCH_PART_C = SCRATCH_PART_R + 2 * SCRATCH_MAX_BLOCKS;
 constexpr int SCRATCH_DOUBLES = SCRATCH_PART_C + 2 * SCRATCH_MAX_BLOCKS;
 // device address of the scratch array on device dev (looked up once per
 // device, with that device current); hipSuccess or the lookup's error

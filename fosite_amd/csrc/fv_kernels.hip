@@ -117,8 +117,9 @@ __global__ __launch_bounds__(256) void k_control_multi(const ControlEntry *__res
   control_block(E.ctl, E.part_c, E.part_r, E.nb);
 }
 
-// max over part[2b] and OR over part[2b+1]; out[0] = max, out[1] = flags
-__global__ __launch_bounds__(256) void k_reduce(const double *part, int n, double *out) {
+// max over part[2b] and OR over part[2b+1]; out[0] = max, out[1] = flags,
+// then out[2] = no, in host memory that the host watches
+__global__ __launch_bounds__(256) void k_reduce(const double *part, int n, double *out, double no) {
   __shared__ double redd[4];
   __shared__ int redi[4];
   double m = -DBL_MAX;
@@ -132,6 +133,8 @@ __global__ __launch_bounds__(256) void k_reduce(const double *part, int n, doubl
   if (threadIdx.x == 0) {
     out[0] = m;
     out[1] = (double)f;
+    __threadfence_system();
+    __hip_atomic_store(out + 2, no, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -435,8 +438,8 @@ void launch_bflux(const BfluxArgs &bf, hipStream_t s) {
 void launch_accrete(const AccreteArgs &p, hipStream_t s) {
   hipLaunchKernelGGL(k_accrete, dim3(1), dim3(64, 4), 0, s, p);
 }
-void launch_reduce(const double *part, int n, double *out, hipStream_t s) {
-  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(256), 0, s, part, n, out);
+void launch_reduce(const double *part, int n, double *out, double no, hipStream_t s) {
+  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(256), 0, s, part, n, out, no);
 }
 
 }  // namespace fv

@@ -145,9 +145,8 @@ int fv_run(fv_ctx *ctx, int nsteps, int *taken);
 /* fv_step that allocates nothing.  No counterpart in the reference: for
  * callers that cannot allocate device memory (tight serving loops, harnesses
  * that forbid hipMalloc).  Its kernels' reduction scratch (per-workgroup
- * partials of the end-of-step evaluation and of the last stage, and the
- * reduction result) is a static device array of the library, one per
- * device, instead of the context's buffers; the context itself still comes
+ * partials of the end-of-step evaluation and of the last stage) is a static
+ * device array of the library, one per device, instead of the context's buffers; the context itself still comes
  * from fv_create.  Limit: 16384 workgroups per RHS launch (64 x 8 cells each,
  * 8.4 M cells); larger meshes return an error.  Calls on one device share
  * the array: calls that overlap on one device (other host threads, other
