@@ -574,25 +574,31 @@ static __device__ int blk_or(int v, int *red) {
 }
 // ----------------------------------------------------------- reconstruction
 // limiters, reconstruction_linear.f90:645-733
-// LIM = 0: limiter chosen at run time from g.limiter
 // a1, a2: differences to the lower and the higher neighbour um, up
+// fsign(one, a) * fsign(one, b) > zero of the reference's conditions: the sign
+// bits agree
+__device__ __forceinline__ bool same_sign(double a, double b) {
+  return (__double2hiint(a) ^ __double2hiint(b)) >= 0;
+}
+__device__ __forceinline__ bool same_sign(float a, float b) {
+  return (__float_as_int(a) ^ __float_as_int(b)) >= 0;
+}
 template <typename T, int LIM>
 __device__ __forceinline__ T limited(const Geom &g, T a1, T a2, T um, T up) {
-  const T one = T(1), zero = T(0), tiny = Real<T>::tiny;
-  switch (LIM ? LIM : g.limiter) {
+  const T zero = T(0), tiny = Real<T>::tiny;
+  switch (LIM) {
     case MINMOD:
-      return (fsign(one, a1) * fsign(one, a2) > zero) ? fsign(fmin2(fabs(a1), fabs(a2)), a1) : zero;
+      return same_sign(a1, a2) ? fsign(fmin2(fabs(a1), fabs(a2)), a1) : zero;
     case MONOCENT: {
       const T th = (T)g.theta;
       const T b1 = th * a1, b2 = th * a2, b3 = T(0.5) * (up - um);
-      if ((fsign(one, b1) * fsign(one, b2) > zero) && (fsign(one, b2) * fsign(one, b3) > zero))
-        return fsign(fmin2(fmin2(fabs(b1), fabs(b2)), fabs(b3)), b1);
-      return zero;
+      const T m = fsign(fmin2(fmin2(fabs(b1), fabs(b2)), fabs(b3)), b1);
+      return same_sign(b1, b2) & same_sign(b2, b3) ? m : zero;
     }
     case SWEBY:
     case SUPERBEE: {
-      const T q = (LIM ? LIM : g.limiter) == SUPERBEE ? T(2) : (T)g.theta;
-      return (fsign(one, a1) * fsign(one, a2) > zero)
+      const T q = LIM == SUPERBEE ? T(2) : (T)g.theta;
+      return same_sign(a1, a2)
                  ? fsign(fmax2(fmin2(q * fabs(a1), fabs(a2)), fmin2(fabs(a1), q * fabs(a2))), a1)
                  : zero;
     }
@@ -607,6 +613,28 @@ __device__ __forceinline__ T limited(const Geom &g, T a1, T a2, T um, T up) {
   }
 }
 
+// f(integral constant): the limiter of LIM, or with LIM = 0 the run-time choice
+// (one branch for all of a row's slopes)
+template <int N>
+struct Limited {
+  static constexpr int value = N;
+};
+template <int LIM, class F>
+__device__ __forceinline__ void with_limiter(const Geom &g, F f) {
+  if constexpr (LIM != 0) {
+    f(Limited<LIM>());
+  } else {
+    switch (g.limiter) {
+      case MINMOD: f(Limited<MINMOD>()); break;
+      case MONOCENT: f(Limited<MONOCENT>()); break;
+      case SWEBY: f(Limited<SWEBY>()); break;
+      case SUPERBEE: f(Limited<SUPERBEE>()); break;
+      case OSPRE: f(Limited<OSPRE>()); break;
+      case VANLEER: f(Limited<VANLEER>()); break;
+      default: f(Limited<NOLIMIT>()); break;
+    }
+  }
+}
 // V limited slopes at once.  Van Leer in FP64 divides with dv, which is exact
 // while no numerator has bits below the subnormal limit; the return value is
 // the least binary exponent of the non-zero numerators (frexp's), and below
@@ -615,22 +643,27 @@ constexpr int SLOPE_EXACT = -960;
 template <typename T, int V, int LIM>
 __device__ __forceinline__ int slopes(const Geom &g, const T *a1, const T *a2, const T *um, const T *up, T *s) {
   int t = 0;
+  if constexpr (LIM == VANLEER && sizeof(T) == 8) {
 #pragma unroll
-  for (int l = 0; l < V; l++) {
-    if constexpr (LIM == VANLEER && sizeof(T) == 8) {
+    for (int l = 0; l < V; l++) {
       const T b1 = fabs(a1[l]), b2 = fabs(a2[l]), num = a1[l] * b2 + a2[l] * b1;
       t = min(t, __builtin_amdgcn_frexp_exp(num));
       s[l] = dv(num, b1 + b2 + Real<T>::tiny);
-    } else {
-      s[l] = limited<T, LIM>(g, a1[l], a2[l], um[l], up[l]);
     }
+  } else {
+    with_limiter<LIM>(g, [&](auto lim) {
+#pragma unroll
+      for (int l = 0; l < V; l++) s[l] = limited<T, decltype(lim)::value>(g, a1[l], a2[l], um[l], up[l]);
+    });
   }
   return t;
 }
 template <typename T, int V, int LIM>
 __device__ __forceinline__ void slopes_exact(const Geom &g, const T *a1, const T *a2, const T *um, const T *up, T *s) {
+  with_limiter<LIM>(g, [&](auto lim) {
 #pragma unroll
-  for (int l = 0; l < V; l++) s[l] = limited<T, LIM>(g, a1[l], a2[l], um[l], up[l]);
+    for (int l = 0; l < V; l++) s[l] = limited<T, decltype(lim)::value>(g, a1[l], a2[l], um[l], up[l]);
+  });
 }
 // whether some lane needs the exact form (compile-time false where none can)
 template <typename T, int LIM>
