@@ -401,6 +401,12 @@ void rhs_flags(const fv_ctx *ctx, int &fp, int &fc, int &add, int &sub) {
   }
 }
 
+// The end-of-step evaluation forms the FARGO remap of each row as it marches
+// along y, where its y boundary is periodic (else the rows of a strip are not
+// consecutive source rows) and no k_visc reads the remapped state first; the
+// other FARGO steps launch k_remap before it.
+bool remap_fused(const fv_ctx *ctx) { return ctx->c.fargo && ctx->c.bc[2] == PERIODIC && !ctx->c.vismodel; }
+
 // ComputeRHS on the main state (pvar, cvar) -> coeff(1) and the new cvar
 // (fresh buffer, ghost cells included); also the CFL inverse time step and
 // the CheckData flags (timedisc_base.f90:1666-1742).  remap = 1 evaluates it
@@ -410,7 +416,7 @@ int rhs_main(fv_ctx *ctx, int checkbm, int remap, double t) {
   rhs_flags(ctx, ctx->fl_pvar, ctx->fl_cvar, add, sub);
   const int pmin = (ctx->V == 4 && (checkbm & CHECK_PMIN)) ? 1 : 0;
   int in = ctx->cvar;
-  if (remap) {  // FargoAdvectionY into a free buffer
+  if (remap && !remap_fused(ctx)) {  // FargoAdvectionY into a free buffer
     const int rb = pick_free(ctx, ctx->cvar, ctx->cold, -1);
     RemapArgs r{ctx->buf[ctx->cvar], ctx->buf[rb], ctx->dt, nullptr};
     long pk = prof_begin(ctx);
@@ -427,6 +433,8 @@ int rhs_main(fv_ctx *ctx, int checkbm, int remap, double t) {
   a.yout = ctx->buf[outb];
   a.add_bg = add;
   a.sub_bg = sub;
+  a.remap = remap && remap_fused(ctx);
+  a.dt_step = ctx->dt;
   a.pmin_clamp = pmin;
   a.want_cfl = 1;
   a.want_check = checkbm != CHECK_NOTHING;
@@ -824,7 +832,7 @@ void fast_step_args(fv_ctx *ctx, Ctl *ctl, int xin, int xout, int tb, int rb, in
     f.acc.ctl = ctl;
   }
   int y = tb;
-  f.remap = ctx->c.fargo != 0;
+  f.remap = ctx->c.fargo != 0 && !remap_fused(ctx);
   if (f.remap) {
     f.rm = RemapArgs{ctx->buf[tb], ctx->buf[rb], 0.0, ctl};
     y = rb;
@@ -833,6 +841,7 @@ void fast_step_args(fv_ctx *ctx, Ctl *ctl, int xin, int xout, int tb, int rb, in
   a.Y = ctx->buf[y];
   a.nk = 0;
   a.ctl = ctl;
+  a.remap = remap_fused(ctx);
   a.kout = ctx->k0[k0out];
   a.yout = ctx->buf[xout];
   a.add_bg = a.sub_bg = steady;
@@ -1714,6 +1723,7 @@ struct fv_batch {
   BfluxArgs *d_bfl = nullptr, *h_bfl = nullptr;
   AccreteArgs *d_acc = nullptr, *h_acc = nullptr;
   int acc_n = 0, acc_bpm = 0;
+  int end_mode = 2;                  // of the end-of-step launch: 3 with a member that remaps in it
   unsigned *d_tiles = nullptr;
   size_t tiles_cap = 0;
   int cand_off[NCAND] = {}, cand_n[NCAND] = {}, remap_off = 0, remap_n = 0;
@@ -1833,8 +1843,10 @@ int rebuild(fv_batch *b) {
     b->cap = cap;
   }
   b->acc_n = b->acc_bpm = 0;
+  b->end_mode = 2;
   for (int d = 0; d < n; d++) {
     const fv_ctx *x = b->sims[d];
+    if (remap_fused(x)) b->end_mode = 3;
     if (!x->grav[0]) continue;
     b->acc_n++;
     b->acc_bpm = std::max(b->acc_bpm, (x->V * 2 * (x->c.inum + x->c.jnum) + 255) / 256);
@@ -1849,7 +1861,7 @@ int rebuild(fv_batch *b) {
   b->remap_off = (int)all.size();
   for (int d = 0; d < n; d++) {
     const fv_ctx *x = b->sims[d];
-    if (x->c.fargo != 2) continue;
+    if (x->c.fargo != 2 || remap_fused(x)) continue;
     const int nbx = (x->c.inum + 63) / 64, nby = remap_rows_blocks(x->c.jnum);
     for (int by = 0; by < nby; by++)
       for (int bx = 0; bx < nbx; bx++) all.push_back(tile_code(d, bx, by));
@@ -1883,7 +1895,7 @@ void enqueue_batch_step(fv_batch *b, int p, int c) {
     launch_accrete_multi(b->d_acc + (size_t)p * cap, b->acc_n, b->st);
   }
   launch_rhs_multi(b->d_rhs + (size_t)(p * m + m - 1) * cap, tl, b->cand_n[c], b->V, b->dtype, b->limiter,
-                   cand_rows(b, c), 2, 0, b->st);
+                   cand_rows(b, c), b->end_mode, 0, b->st);
   launch_control_multi(b->d_cent + (size_t)c * cap, n, b->st);
 }
 

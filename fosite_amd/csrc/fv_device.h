@@ -119,6 +119,10 @@ struct StageArgsT {
   T *yout;              // transformed state incl. ghost cells, or null
   int add_bg, sub_bg;   // FARGO frame change at entry / before the fluxes
   int pmin_clamp;       // Euler CHECK_PMIN round trip (timedisc_base.f90:1150-1164)
+  // end-of-step evaluation of a FARGO step: on FargoAdvectionY(Y), whose shifts
+  // take this%dt (host-controlled: dt_step)
+  int remap;
+  double dt_step;
   int want_cfl, want_check;
   double *part;         // per-block partials: [2*b] max 1/dt, [2*b+1] check flags
   // fused final combination (last stage only)
@@ -287,7 +291,7 @@ constexpr int REMAP_ROWS = FV_REMAP_ROWS;
 __host__ __device__ inline int remap_rows_blocks(int jnum) { return (jnum + 4 * REMAP_ROWS - 1) / (4 * REMAP_ROWS); }
 // batch launchers: ntiles blocks over the tile list; rows = strip rows of the list
 // mode: 0 RK stage rhs, 1 last stage with the final combination (nk slopes in
-// their stage sums), 2 end-of-step evaluation
+// their stage sums), 2 end-of-step evaluation, 3 with members whose StageArgs::remap is set
 void launch_rhs_multi(const RhsEntry *tab, const unsigned *tiles, int ntiles, int V, int dtype, int limiter,
                       int rows, int mode, int nk, hipStream_t s);
 void launch_remap_multi(const RemapEntry *tab, const unsigned *tiles, int ntiles, int V, int dtype, hipStream_t s);

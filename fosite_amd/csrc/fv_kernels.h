@@ -26,7 +26,8 @@
 //     gravity and FARGO sources, rhs assembly, CFL and data checks follow.
 //   * in the last stage of a step, the final RK combination and the embedded
 //     error norm (pointwise) replace the store of the stage's rhs.
-// k_remap: FARGO azimuthal shift of the combined state (y direction only).
+// k_remap: FARGO azimuthal shift of the combined state (y direction only), where
+// the end-of-step k_rhs does not form it on the fly.
 // k_control: one block; in device-controlled batches it reduces the partials
 // of the last stage and of the end-of-step k_rhs, runs the accept test and
 // the CFL update.  Kernel boundaries order everything: no grid-wide fences.
@@ -266,11 +267,194 @@ __device__ __forceinline__ void frame_sub(T *u, T w) {
   u[2] = u[2] - u[0] * w;
 }
 
+// fsign(one, a) * fsign(one, b) > zero of the reference's conditions: the sign
+// bits agree
+__device__ __forceinline__ bool same_sign(double a, double b) {
+  return (__double2hiint(a) ^ __double2hiint(b)) >= 0;
+}
+__device__ __forceinline__ bool same_sign(float a, float b) {
+  return (__float_as_int(a) ^ __float_as_int(b)) >= 0;
+}
+
+// ------------------------------------------------------------ FARGO remap
+// FargoAdvectionY (timedisc_base.f90:1935-2069) of one interior cell from
+// the combined state: per ring the shift d = w*dt/dly split into its nearest
+// integer and a fraction, minmod-limited linear transport by the fraction,
+// then CSHIFT(., -shift) over JMIN:JMAX.  Rows outside JMIN:JMAX come from
+// the comoving-frame CenterBoundary (prim round trip, no frame change).
+
+// this%dt of the step as AcceptSolution will set it, with the round's halt flag
+// (host-controlled launches read dummies: no branch ahead of the loads)
+struct StepTime {
+  double dt, dts;  // the step control's dt; this%dt
+  int halt;
+  __device__ __forceinline__ StepTime(const Geom &g, const Ctl *ctl, double dt_step) {
+    const double *h = ctl ? &ctl->time : g.ring;
+    const int hf = *(ctl ? &ctl->halt : reinterpret_cast<const int *>(g.ring));
+    const double t = h[0];
+    dt = h[1];
+    dts = ctl ? (t + dt) - t : dt_step;
+    halt = ctl ? hf : 0;
+  }
+};
+// the shift of a ring (background velocity w, cell length dly)
+template <typename T>
+struct RingShift {
+  T d;    // the fraction
+  int m;  // the integer, in (-J, J)
+  __device__ __forceinline__ RingShift(const Geom &g, double w, double dly, const StepTime &st) {
+    const int J = g.jnum;
+    const double dd = w * st.dts / dly, shift = round(dd);
+    d = (T)(dd - shift);
+    // shifts of more than a ring are rare, and the exact fmod is slow
+    m = fabs(shift) < 2147483648.0 ? (int)shift : (int)fmod(shift, (double)J);
+    if (__any(m >= J || m <= -J)) m %= J;
+  }
+  // source row of row j (0 .. J-1, as j)
+  static __device__ __forceinline__ int source(int j, int m, int J) {
+    int s = j - m;
+    if (s < 0) s += J;
+    if (s >= J) s -= J;
+    return s;
+  }
+};
+// the limited transport of one row by the fraction d, from its five source cells
+template <typename T, int V>
+__device__ __forceinline__ void fargo_row(const T (*v)[V], T d, T *u) {
+  const T one = T(1), zero = T(0), half = T(0.5);
+#pragma unroll
+  for (int l = 0; l < V; l++) {
+    T dq[4], dql[3];
+#pragma unroll
+    for (int q = 0; q < 4; q++) dq[q] = v[q + 1][l] - v[q][l];
+#pragma unroll
+    for (int q = 0; q < 3; q++)
+      dql[q] = same_sign(dq[q], dq[q + 1]) ? fsign(fmin2(fabs(dq[q]), fabs(dq[q + 1])), dq[q]) : zero;
+    T f0, f1;  // flux(js-1), flux(js)
+    if (d > zero) {
+      f0 = v[1][l] + half * dql[0] * (one - d);
+      f1 = v[2][l] + half * dql[1] * (one - d);
+    } else {
+      f0 = v[2][l] - half * dql[1] * (one + d);
+      f1 = v[3][l] - half * dql[2] * (one + d);
+    }
+    u[l] = v[2][l] - d * (f1 - f0);
+  }
+}
+// The transport marching along a ring whose y boundary is periodic.  Row c's
+// flux towards c+1 reads the cells e-1, e, e+1 with e = c or, for d <= 0, c+1,
+// and is the next row's flux from below: a row costs one new cell, one limited
+// difference and one flux.  The cells beyond the mesh as row c sees them (the
+// round trip of the rows at the other end) occur at c = 0 and c >= J-2 only,
+// and row 0 sees other cells below it than row J-1 does above.  Bound by VALU
+// issue like the strip around it (the five-cell form of fargo_row costs three
+// limited differences and four fluxes a row).  us for the remap and the
+// end-of-step launch, separate -> five cells per row in the strip -> this:
+//   64x128 FP64 15.7 -> 13.0 -> 12.7, 512x1024 FP64 30.9 -> 29.6 -> 27.3,
+//   512x1024 FP32 20.2 -> 19.3 -> 18.1
+template <typename T, int V>
+struct FargoMarch {
+  T d, k;                     // the fraction; a flux's factor of the limited difference
+  bool up;                    // e = c
+  int c;                      // source row of the next row
+  T tm[V], t0[V], t1[V], f[V];  // cells e-2, e-1, e; flux from below
+  // (m: the ring's integer shift, j: the first row, 0 .. J-1)
+  __device__ __forceinline__ FargoMarch(const RingShift<T> &sh, int j, int J) : d(sh.d), up(sh.d > T(0)) {
+    k = up ? T(1) - d : -(T(1) + d);
+    c = RingShift<T>::source(j, sh.m, J);
+  }
+  __device__ __forceinline__ int e() const { return up ? c : c + 1; }
+  // row of the first cell (e-2) in memory order, 0 .. J-1
+  __device__ __forceinline__ int first(int J) const { return e() < 2 ? e() - 2 + J : e() - 2; }
+  __device__ __forceinline__ void flux(const T *a, const T *b, const T *n, T *F) const {
+#pragma unroll
+    for (int l = 0; l < V; l++) {
+      const T q0 = b[l] - a[l], q1 = n[l] - b[l];
+      const T s = same_sign(q0, q1) ? fsign(fmin2(fabs(q0), fabs(q1)), q0) : T(0);
+      F[l] = b[l] + T(0.5) * s * k;
+    }
+  }
+  // the cell at row s as row c sees it (the density comes back as it was)
+  static __device__ __forceinline__ void ghost(const Geom &g, int s, T *t) {
+    T p[V], u[V];
+    c2p<T, V>(t, p, (T)g.gamma);
+    p2c<T, V>(p, u, (T)g.gamma);
+#pragma unroll
+    for (int l = 1; l < V; l++) t[l] = s < 0 || s >= g.jnum ? u[l] : t[l];
+  }
+  // the first row's flux from below, from the cells tm, t0, t1
+  __device__ __forceinline__ void begin(const Geom &g) {
+    T a[V], b[V], n[V];
+#pragma unroll
+    for (int l = 0; l < V; l++) a[l] = tm[l], b[l] = t0[l], n[l] = t1[l];
+    if (__any(c < 2 || c >= g.jnum - 2)) {
+      ghost(g, e() - 2, a);
+      ghost(g, e() - 1, b);
+      ghost(g, e(), n);
+    }
+    flux(a, b, n, f);
+  }
+  // the next row from its new cell, e+1
+  __device__ __forceinline__ void next(const Geom &g, const T *t2, T *u) {
+    T F[V];
+    if (__any(c == 0 || c >= g.jnum - 2)) {
+      T a[V], b[V], n[V], x[V], f0[V];
+#pragma unroll
+      for (int l = 0; l < V; l++) x[l] = tm[l], a[l] = t0[l], b[l] = t1[l], n[l] = t2[l];
+      ghost(g, e() - 2, x);
+      ghost(g, e() - 1, a);
+      ghost(g, e(), b);
+      ghost(g, e() + 1, n);
+      flux(a, b, n, F);
+      flux(x, a, b, f0);
+#pragma unroll
+      for (int l = 0; l < V; l++) f[l] = c == 0 ? f0[l] : f[l];
+    } else {
+      flux(t0, t1, t2, F);
+    }
+#pragma unroll
+    for (int l = 0; l < V; l++) {
+      u[l] = (up ? t1[l] : t0[l]) - d * (F[l] - f[l]);
+      tm[l] = t0[l];
+      t0[l] = t1[l];
+      t1[l] = t2[l];
+      f[l] = F[l];
+    }
+    c = c + 1 == g.jnum ? 0 : c + 1;
+  }
+};
+// one source cell of the transport; rows beyond the mesh hold the y boundary's
+// cells after CenterBoundary's round trip
+template <typename T, int V>
+__device__ __forceinline__ void ycell_load(const Geom &g, const T *Y, int i, int jj, T *u) {
+  const int jmin = GH, jmax = GH + g.jnum - 1;
+  const int js = jj < jmin   ? (g.bc[2] == PERIODIC ? jj + g.jnum : jmin)
+                 : jj > jmax ? (g.bc[3] == PERIODIC ? jj - g.jnum : jmax)
+                             : jj;
+  const long ix = cidx(g, i, js);
+#pragma unroll
+  for (int l = 0; l < V; l++) u[l] = (Y + l * g.FS)[ix];
+}
+template <typename T, int V>
+__device__ __forceinline__ void ycell_ghost(const Geom &g, int jj, T *u) {
+  if (jj < GH || jj >= GH + g.jnum) {
+    T p[V];
+    c2p<T, V>(u, p, (T)g.gamma);
+    p2c<T, V>(p, u, (T)g.gamma);
+  }
+}
+template <typename T, int V>
+__device__ __forceinline__ void ycell(const Geom &g, const T *Y, int i, int jj, T *u) {
+  ycell_load<T, V>(g, Y, i, jj, u);
+  ycell_ghost<T, V>(g, jj, u);
+}
+
 // ------------------------------------------------------------ input state
 // KM: coefficient slots of the tableau (3 for up to three stages, else MAXK);
 // loops over stages are unrolled to KM with run-time guards on nk, or with
 // EXACT over exactly KM slopes
-template <typename T, int V, int KM, bool EXACT = false>
+// RM: the state is the FARGO remap of Y (no stage sum)
+template <typename T, int V, int KM, bool EXACT = false, bool RM = false>
 struct In {
   const Geom &g;
   const StageArgsT<T> &a;
@@ -329,6 +513,17 @@ struct In {
 
   // input state at an interior cell
   __forceinline__ __device__ void interior(int i, int j, T *s) const {
+    if constexpr (RM) {
+      const RingShift<T> sh(g, ring(g, R_W, i), ring(g, R_DLY, i), StepTime(g, a.ctl, a.dt_step));
+      const int js = GH + sh.source(j - GH, sh.m, g.jnum);
+      T v[5][V];
+#pragma unroll
+      for (int q = 0; q < 5; q++) ycell_load<T, V>(g, a.Y, i, js - 2 + q, v[q]);
+#pragma unroll
+      for (int q = 0; q < 5; q++) ycell_ghost<T, V>(g, js - 2 + q, v[q]);
+      fargo_row<T, V>(v, sh.d, s);
+      return;
+    }
     const long ix = cidx(g, i, j);
     // all loads first (uniform branches only), then the stage sum
     T y[V], kv[KA][V];
@@ -575,14 +770,6 @@ static __device__ int blk_or(int v, int *red) {
 // ----------------------------------------------------------- reconstruction
 // limiters, reconstruction_linear.f90:645-733
 // a1, a2: differences to the lower and the higher neighbour um, up
-// fsign(one, a) * fsign(one, b) > zero of the reference's conditions: the sign
-// bits agree
-__device__ __forceinline__ bool same_sign(double a, double b) {
-  return (__double2hiint(a) ^ __double2hiint(b)) >= 0;
-}
-__device__ __forceinline__ bool same_sign(float a, float b) {
-  return (__float_as_int(a) ^ __float_as_int(b)) >= 0;
-}
 template <typename T, int LIM>
 __device__ __forceinline__ T limited(const Geom &g, T a1, T a2, T um, T up) {
   const T zero = T(0), tiny = Real<T>::tiny;
@@ -913,13 +1100,14 @@ __host__ __device__ inline int xcd_grid(int n) { return ((n + XCDS - 1) / XCDS) 
 
 // -------------------------------------------------------------- RHS pieces
 // launch modes of the RHS kernel
-enum RhsMode { M_STAGE = 0, M_LAST = 1, M_END = 2 };
+// (M_REMAP: the end-of-step evaluation on the FARGO remap of Y)
+enum RhsMode { M_STAGE = 0, M_LAST = 1, M_END = 2, M_REMAP = 3 };
 template <typename T>
 __host__ __device__ inline int rhs_aux(const Geom &g, const StageArgsT<T> &a) {
   return a.bfa.out ? rhs_aux_max(g, a.bfa.V) : 1;
 }
 template <typename T>
-inline int rhs_mode(const StageArgsT<T> &a) { return a.ynew ? M_LAST : (a.nk == 0 ? M_END : M_STAGE); }
+inline int rhs_mode(const StageArgsT<T> &a) { return a.ynew ? M_LAST : a.nk ? M_STAGE : a.remap ? M_REMAP : M_END; }
 
 // Source terms of the cells of one ring.  Of the commutator coefficients only
 // c_yxy differs from zero on the supported meshes (fv_create checks it).
@@ -1093,86 +1281,28 @@ struct Combination {
   }
 };
 
-// ------------------------------------------------------------ FARGO remap
-// FargoAdvectionY (timedisc_base.f90:1935-2069) of one interior cell from
-// the combined state: per ring the shift d = w*dt/dly split into its nearest
-// integer and a fraction, minmod-limited linear transport by the fraction,
-// then CSHIFT(., -shift) over JMIN:JMAX.  Rows outside JMIN:JMAX come from
-// the comoving-frame CenterBoundary (prim round trip, no frame change).
-template <typename T, int V>
-__device__ __forceinline__ void ycell(const Geom &g, const T *Y, int i, int jj, T *u) {
-  const int jmin = GH, jmax = GH + g.jnum - 1;
-  int js = jj;
-  bool ghost = false;
-  if (jj < jmin) {
-    ghost = true;
-    js = g.bc[2] == PERIODIC ? jj + g.jnum : jmin;
-  } else if (jj > jmax) {
-    ghost = true;
-    js = g.bc[3] == PERIODIC ? jj - g.jnum : jmax;
-  }
-  const long ix = cidx(g, i, js);
-#pragma unroll
-  for (int l = 0; l < V; l++) u[l] = Y[l * g.FS + ix];
-  if (ghost) {
-    T p[V];
-    c2p<T, V>(u, p, (T)g.gamma);
-    p2c<T, V>(p, u, (T)g.gamma);
-  }
-}
-
-// one block (bx, by) of the remap: 64 rings x REMAP_ROWS*4 rows.  A thread
-// takes REMAP_ROWS consecutive rows of its ring; while their source rows do
-// not wrap around the ring, they share one window of REMAP_ROWS+4 source
-// cells (each cell's arithmetic is unchanged), otherwise every row loads its
-// own five.
+// one block (bx, by) of the separate remap (y boundaries that are not periodic,
+// and viscous steps, whose k_visc reads the remapped state): 64 rings x
+// REMAP_ROWS*4 rows.  A thread takes REMAP_ROWS consecutive rows of its ring;
+// while their source rows do not wrap around the ring, they share one window
+// of REMAP_ROWS+4 source cells (each cell's arithmetic is unchanged),
+// otherwise every row loads its own five.
 template <typename T, int V>
 __device__ __forceinline__ void remap_block(const Geom &g, const RemapArgsT<T> &a, int bx, int by) {
   constexpr int RR = REMAP_ROWS;
   const int i = GH + bx * 64 + threadIdx.x, jb = (by * 4 + threadIdx.y) * RR;
   if (i >= GH + g.inum || jb >= g.jnum) return;
   const int jmin = GH, J = g.jnum;
-  // the step control and the ring's values in one memory latency
-  // (host-controlled launches read dummies)
-  const double *h = a.ctl ? &a.ctl->time : g.ring;
-  const double t = h[0], dt = h[1], w = ring(g, R_W, i), dly = ring(g, R_DLY, i);
-  const int halt = *(a.ctl ? &a.ctl->halt : reinterpret_cast<const int *>(g.ring));
-  if (a.ctl && halt) return;
-  const double dts = a.ctl ? (t + dt) - t : a.dt_step;  // this%dt as AcceptSolution will set it
-  double dd = w * dts / dly;
-  const double shift = round(dd);
-  const T d = (T)(dd - shift);
-  // source row of the first row: jmin + ((jb - shift) mod J); shifts of more
-  // than a ring are rare, and the exact fmod is slow
-  int m = fabs(shift) < 2147483648.0 ? (int)shift : (int)fmod(shift, (double)J);
-  if (__any(m >= J || m <= -J)) m %= J;
-  int j0 = jb - m;
-  if (j0 < 0) j0 += J;
-  if (j0 >= J) j0 -= J;
+  const StepTime st(g, a.ctl, a.dt_step);
+  const RingShift<T> sh(g, ring(g, R_W, i), ring(g, R_DLY, i), st);
+  if (st.halt) return;
+  const int j0 = sh.source(jb, sh.m, J);
   const int nr = J - jb < RR ? J - jb : RR;
-  const T one = T(1), zero = T(0), half = T(0.5);
-  // the limited transport of one row from its five source cells
   auto row = [&](const T (*v)[V], int j) {
-    const long ix = cidx(g, i, j);
+    T u[V];
+    fargo_row<T, V>(v, sh.d, u);
 #pragma unroll
-    for (int l = 0; l < V; l++) {
-      T dq[4], dql[3];
-#pragma unroll
-      for (int q = 0; q < 4; q++) dq[q] = v[q + 1][l] - v[q][l];
-#pragma unroll
-      for (int q = 0; q < 3; q++)
-        dql[q] = (fsign(one, dq[q]) * fsign(one, dq[q + 1]) > zero) ? fsign(fmin2(fabs(dq[q]), fabs(dq[q + 1])), dq[q])
-                                                                   : zero;
-      T f0, f1;  // flux(js-1), flux(js)
-      if (d > zero) {
-        f0 = v[1][l] + half * dql[0] * (one - d);
-        f1 = v[2][l] + half * dql[1] * (one - d);
-      } else {
-        f0 = v[2][l] - half * dql[1] * (one + d);
-        f1 = v[3][l] - half * dql[2] * (one + d);
-      }
-      a.out[l * g.FS + ix] = v[2][l] - d * (f1 - f0);
-    }
+    for (int l = 0; l < V; l++) (a.out + l * g.FS)[cidx(g, i, j)] = u[l];
   };
   if (j0 + nr <= J) {  // no wrap: one window
     T v[RR + 4][V];

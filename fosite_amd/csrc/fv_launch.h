@@ -33,7 +33,7 @@ static void with_last_slopes(int nk, F f) {
 template <typename T, int V, int LIM, int RMAX>
 static void rhs_rows(const Geom &g, const StageArgsT<T> &a, hipStream_t s) {
   const int mode = rhs_mode(a), n = strip_cols(g.inum) * strip_blocks(g.jnum, g.rows);
-  const dim3 grid(xcd_grid(n) + (mode == M_END ? rhs_aux(g, a) : 0)), block(64 * SWAVES);
+  const dim3 grid(xcd_grid(n) + (mode >= M_END ? rhs_aux(g, a) : 0)), block(64 * SWAVES);
   switch (mode) {
     case M_STAGE:
       with_stage_slopes(a.nk, [&](auto n) {
@@ -44,6 +44,10 @@ static void rhs_rows(const Geom &g, const StageArgsT<T> &a, hipStream_t s) {
       with_last_slopes(a.nk, [&](auto n) {
         hipLaunchKernelGGL((k_rhs<T, V, LIM, decltype(n)::value, M_LAST, RMAX>), grid, block, 0, s, g, a);
       });
+      break;
+    case M_REMAP:
+      if constexpr (sizeof(T) == 8 || V == 3)  // (FARGO with Euler physics runs in FP64)
+        hipLaunchKernelGGL((k_rhs<T, V, LIM, 0, M_REMAP, RMAX>), grid, block, 0, s, g, a);
       break;
     default: hipLaunchKernelGGL((k_rhs<T, V, LIM, 0, M_END, RMAX>), grid, block, 0, s, g, a); break;
   }
@@ -106,6 +110,10 @@ static void rhs_multi_rows(const RhsEntry *tab, const unsigned *tiles, int n, in
         hipLaunchKernelGGL((k_rhs_multi<T, V, LIM, decltype(k)::value, M_LAST, RMAX>), dim3(n), block, 0, s, tab, tiles,
                            rows);
       });
+      break;
+    case M_REMAP:
+      if constexpr (sizeof(T) == 8 || V == 3)
+        hipLaunchKernelGGL((k_rhs_multi<T, V, LIM, 0, M_REMAP, RMAX>), dim3(n), block, 0, s, tab, tiles, rows);
       break;
     default:
       hipLaunchKernelGGL((k_rhs_multi<T, V, LIM, 0, M_END, RMAX>), dim3(n), block, 0, s, tab, tiles, rows);

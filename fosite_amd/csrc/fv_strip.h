@@ -80,7 +80,7 @@ struct StripOut {
 
 template <typename T, int V, int LIM, int NK, int MODE, int RMAX>
 __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T> &a, int bx, int j0, int nr, T *hx) {
-  constexpr bool kEnd = MODE == M_END, kLast = MODE == M_LAST;
+  constexpr bool kRemap = MODE == M_REMAP, kEnd = MODE == M_END || kRemap, kLast = MODE == M_LAST;
   using Row = RowIn<T, V, NK>;
   using Comb = Combination<T, V, NK>;
   // the last stage's sums over k_1 .. k_{s-1}: formed when a row arrives and
@@ -114,7 +114,20 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
   // (byte offsets from scalar row pointers)
   const unsigned lo = (unsigned)i * sizeof(T);
   auto at = [&](const T *row) { return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(row) + lo); };
+  // kRemap: rows are read at the lane's source row of the FARGO shift, one
+  // after the other around the ring; src is the next to load
+  int src = 0;
+  auto load_src = [&](T *y) {
+    const unsigned ix = (unsigned)(GH + src) * (unsigned)g.P + (unsigned)i;
+#pragma unroll
+    for (int l = 0; l < V; l++) y[l] = (a.Y + l * g.FS)[ix];
+    src = src + 1 == g.jnum ? 0 : src + 1;
+  };
   auto load_at = [&](int j, Row &R) {
+    if constexpr (kRemap) {
+      load_src(R.y);
+      return;
+    }
     const long base = (long)source_row(j) * g.P;
 #pragma unroll
     for (int l = 0; l < V; l++) R.y[l] = at(a.Y + l * g.FS + base);
@@ -128,8 +141,10 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
   // the step's halt flag and dt (host-controlled launches read a dummy).
   constexpr int PRE = NK * V <= 8 ? 4 : 1;
   Row pre[4], re;
+  if constexpr (!kRemap) {
 #pragma unroll
-  for (int q = 0; q < PRE; q++) load_at(j0 - 2 + q, pre[q]);
+    for (int q = 0; q < PRE; q++) load_at(j0 - 2 + q, pre[q]);
+  }
   // edge columns of ER rows at a time: lane = slot * ER + row, slots = columns
   // -2, -1, 0, 1 and ce-1, ce, ce+1, ce-2; x ghost cells load the interior cell
   // that their boundary rule starts from
@@ -142,8 +157,10 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
   auto load_edge = [&](int e0) {
     const int jj = min(j0 + e0 + er, j0 + nr - 1);
     const long ix = cidx(g, is, jj);
+    if constexpr (!kRemap) {
 #pragma unroll
-    for (int l = 0; l < V; l++) re.y[l] = (a.Y + l * g.FS)[ix];
+      for (int l = 0; l < V; l++) re.y[l] = (a.Y + l * g.FS)[ix];
+    }
 #pragma unroll
     for (int q = 0; q < NK; q++)
 #pragma unroll
@@ -151,7 +168,7 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
     e_ds = cl<T>(g, C_RDYS, jj + 1);
     e_dn = cl<T>(g, C_RDYN, jj + 1);
   };
-  load_edge(0);
+  if constexpr (!kRemap) load_edge(0);
   const AbsorbingSpeeds<T> as(g, east);
   const T e_ws = rg<T>(g, R_W, is), e_w = rg<T>(g, R_W, ii), e_off = rg<T>(g, eq == 1 ? R_RDXE : R_RDXW, ii);
   const T e_csE = rg<T>(g, R_CSE, i0 - 1), e_csW = rg<T>(g, R_CSW, i0), e_dA = rg<T>(g, R_DAXW, i0);
@@ -163,17 +180,52 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
   const T dAxn = rg<T>(g, R_DAXW, i + 1), dAy = rg<T>(g, R_DAYS, i);
   const T dydzdV = rg<T>(g, R_DYDZDV, i), dzdxdV = rg<T>(g, R_DZDXDV, i);
   const SourceRing<T, V> sr(g, a, i);
-  const int halt = *(a.ctl ? &a.ctl->halt : reinterpret_cast<const int *>(g.ring));
-  const double ctl_dt = *(a.ctl ? &a.ctl->dt : g.ring);
+  const StepTime st(g, a.ctl, kRemap ? a.dt_step : 0.0);
+  const double w_d = kRemap ? ring(g, R_W, i) : 0.0, dly_d = kRemap ? ring(g, R_DLY, i) : 1.0;
+  const double ew_d = kRemap ? ring(g, R_W, is) : 0.0, edly_d = kRemap ? ring(g, R_DLY, is) : 1.0;
   asm volatile("" ::: "memory");  // keeps the loads above this branch
-  if (a.ctl && halt) return {0.0, 0.0, 0, 1};
-  const In<T, V, NK, true> in(g, a, want_check, a.ctl ? ctl_dt : a.dt);
+  if (st.halt) return {0.0, 0.0, 0, 1};
+  const In<T, V, NK, true> in(g, a, want_check, a.ctl ? st.dt : a.dt);
+  // kRemap: the strip's columns (from two rows below its first) and the edge
+  // lanes' cells, each marching along its ring
+  const RingShift<T> sh(g, w_d, dly_d, st), esh(g, ew_d, edly_d, st);
+  const int jf = j0 - 2 - GH;
+  FargoMarch<T, V> fm(sh, kRemap && jf < 0 ? jf + g.jnum : jf, g.jnum);
+  T ewin[kRemap ? 4 : 1][V];
+  auto load_ewin = [&](int e0) {
+    int sq = FargoMarch<T, V>(esh, min(j0 + e0 + er, j0 + nr - 1) - GH, g.jnum).first(g.jnum);
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const unsigned ex = (unsigned)(GH + sq) * (unsigned)g.P + (unsigned)is;
+#pragma unroll
+      for (int l = 0; l < V; l++) ewin[q][l] = (a.Y + l * g.FS)[ex];
+      sq = sq + 1 == g.jnum ? 0 : sq + 1;
+    }
+  };
+  if constexpr (kRemap) {
+    src = fm.first(g.jnum);
+    load_src(fm.tm);
+    load_src(fm.t0);
+    load_src(fm.t1);
+#pragma unroll
+    for (int q = 0; q < PRE; q++) load_src(pre[q].y);
+    load_edge(0);
+    load_ewin(0);
+    fm.begin(g);
+  }
 
   // ---- edge columns
   for (int e0 = 0;;) {
     const int jj = j0 + e0 + er;
     const bool on = e0 + er < nr;
     T u[V], p[V], s[V], ur[V];
+    if constexpr (kRemap) {
+      FargoMarch<T, V> em(esh, min(jj, j0 + nr - 1) - GH, g.jnum);
+#pragma unroll
+      for (int l = 0; l < V; l++) em.tm[l] = ewin[0][l], em.t0[l] = ewin[1][l], em.t1[l] = ewin[2][l];
+      em.begin(g);
+      em.next(g, ewin[3], re.y);
+    }
     in.stage_sum(re.y, re.k, s);
     in.to_prim(e_ws, s, ur, p);
     T pl[V], pr[V];
@@ -251,6 +303,7 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
     if constexpr (RMAX <= ER) break;
     if ((e0 += ER) >= nr) break;
     load_edge(e0);
+    if constexpr (kRemap) load_ewin(e0);
   }
   wave_sync();
 
@@ -266,7 +319,13 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
   auto enter = [&](int r, const Row &R, T *u, T *geo, T *ext, Comb &cb) {
     const int j = j0 + r;
     T s[V], ur[V], p[V];
-    in.stage_sum(R.y, R.k, s);
+    if constexpr (kRemap) {
+      T y[V];
+      fm.next(g, R.y, y);
+      in.stage_sum(y, R.k, s);
+    } else {
+      in.stage_sum(R.y, R.k, s);
+    }
     const unsigned ix = (unsigned)j * (unsigned)g.P + (unsigned)i;
     if (j < jmin || j > jmax) {  // y ghost row
       if (a.add_bg) frame_add<T, V>(s, w);
@@ -503,7 +562,7 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
 // k = 0 evaluates the corner ghost cells, which are in no strip (data checks,
 // CFL and the new state, SetCornerEdges, boundary_generic.f90:434-517); the
 // others make the step's boundary-flux accumulation (device-controlled steps).
-template <typename T, int V>
+template <typename T, int V, bool RM>
 __device__ __forceinline__ void rhs_aux_block(const Geom &g, const StageArgsT<T> &a, int k, int naux, int b) {
   if (a.ctl && a.ctl->halt) return;
   const double dt = a.ctl ? a.ctl->dt : a.dt;
@@ -513,14 +572,36 @@ __device__ __forceinline__ void rhs_aux_block(const Geom &g, const StageArgsT<T>
     return;
   }
   if (t >= 64 || !(a.want_cfl || a.want_check)) return;
+  // lane = cell + 16 * part: the two interior cells behind the x boundary's
+  // rule, the one behind the y boundary's, (none); all of them in one pass,
+  // so that the chain is one evaluation long
+  const int q = t & 15, part = t >> 4;
+  const int ga = 1 + (q & 1), gb = 1 + ((q >> 1) & 1), cE = (q >> 2) & 1, cN = q >> 3;
+  const int imin = GH, imax = GH + g.inum - 1, jmin = GH, jmax = GH + g.jnum - 1;
+  const int ir = cE ? imax : imin, jr = cN ? jmax : jmin, bx = cE ? g.bc[1] : g.bc[0], by = cN ? g.bc[3] : g.bc[2];
+  const int si = part >= 2 ? ir
+                 : bx == PERIODIC ? (cE ? imin + ga - 1 : imax - ga + 1)
+                 : bx == ABSORBING ? (cE ? imax - 1 + part : imin + part)
+                                   : ir;
+  const int sj = part < 2 ? jr : by == PERIODIC ? (cN ? jmin + gb - 1 : jmax - gb + 1) : jr;
+  const In<T, V, 0, true, RM> in(g, a, a.want_check, dt);
+  T u[V], p[V], px[V], pR[V], py[V];
+  in.prim_interior(si, sj, px);
+#pragma unroll
+  for (int l = 0; l < V; l++) {
+    pR[l] = __shfl(px[l], q + 16, 64);
+    py[l] = __shfl(px[l], q + 32, 64);
+  }
   T cfl = -Real<T>::huge;
   int flags = 0;
   if (t < 16) {
-    const int ga = 1 + (t & 1), gb = 1 + ((t >> 1) & 1), cE = (t >> 2) & 1, cN = t >> 3;
-    const int gi = cE ? GH + g.inum - 1 + ga : GH - ga, gj = cN ? GH + g.jnum - 1 + gb : GH - gb;
-    const In<T, V, 0, true> in(g, a, a.want_check, dt);
-    T u[V], p[V];
-    in.ghost_final(gi, gj, u, p, flags);
+    if (bx == ABSORBING) absorbing_math<T, V>(cE, AbsorbingSpeeds<T>(g, cE), in.gam, px, pR, px);
+    // SetCornerEdges
+    const bool only_x = ga == 2 && gb == 1, only_y = ga == 1 && gb == 2;
+#pragma unroll
+    for (int l = 0; l < V; l++) p[l] = only_x ? px[l] : only_y ? py[l] : T(0.5) * (px[l] + py[l]);
+    const int gi = cE ? imax + ga : imin - ga, gj = cN ? jmax + gb : jmin - gb;
+    in.ghost_from_prim(rg<T>(g, R_W, gi), p, u, flags);
     if (a.want_cfl) {
       const T cs = (V == 4) ? sound_speed(in.gam, p[0], p[3]) : rg<T>(g, R_CS, gi);
       cfl = cell_invdt(g, gi, p[1], p[2], cs);
@@ -565,7 +646,7 @@ __device__ __forceinline__ void rhs_block(const Geom &g, const StageArgsT<T> &a,
       a.part_c[2 * b + 1] = 0.0;
     }
   }
-  if constexpr (MODE == M_END) {
+  if constexpr (MODE >= M_END) {
     if (!(a.want_cfl || a.want_check)) return;
     blk_max_or0(o.invdt, o.flags, redd, redi);
     if (t == 0) {
@@ -586,7 +667,7 @@ __global__ __launch_bounds__(64 * SWAVES, (strip_occupancy<T, V, NK, MODE>())) v
   const int nbx = strip_cols(g.inum), n = nbx * strip_blocks(g.jnum, g.rows), grid = xcd_grid(n);
   const int t = xcd_tile(blockIdx.x, n), k = (int)blockIdx.x - grid;
   if (k >= 0) {  // behind the strips' workgroups, so that the XCDs' shares of those stay even
-    if constexpr (MODE == M_END) rhs_aux_block<T, V>(g, a, k, gridDim.x - grid, n);
+    if constexpr (MODE >= M_END) rhs_aux_block<T, V, MODE == M_REMAP>(g, a, k, gridDim.x - grid, n);
   } else if (t < n) {
     rhs_block<T, V, LIM, NK, MODE, RMAX>(g, a, g.rows, t % nbx, t / nbx, t);
   }
@@ -603,10 +684,16 @@ __global__ __launch_bounds__(64 * SWAVES, (strip_occupancy<T, V, NK, MODE>())) v
   const RhsEntry &E = tab[tile_disk(e)];
   const StageArgsT<T> &a = reinterpret_cast<const StageArgsT<T> &>(E.a);
   const int nbx = strip_cols(E.g.inum), nby = strip_blocks(E.g.jnum, rows), bx = tile_bx(e), by = tile_by(e);
-  if (by < nby)
+  if (MODE == M_REMAP && !a.remap) {  // a member without FARGO beside others
+    if (by < nby)
+      rhs_block<T, V, LIM, NK, M_END, RMAX>(E.g, a, rows, bx, by, bx + by * nbx);
+    else
+      rhs_aux_block<T, V, false>(E.g, a, bx, rhs_aux_max(E.g, V), nbx * nby);
+  } else if (by < nby) {
     rhs_block<T, V, LIM, NK, MODE, RMAX>(E.g, a, rows, bx, by, bx + by * nbx);
-  else if (MODE == M_END)
-    rhs_aux_block<T, V>(E.g, a, bx, rhs_aux_max(E.g, V), nbx * nby);
+  } else if (MODE >= M_END) {
+    rhs_aux_block<T, V, MODE == M_REMAP>(E.g, a, bx, rhs_aux_max(E.g, V), nbx * nby);
+  }
 }
 
 }  // namespace fv
