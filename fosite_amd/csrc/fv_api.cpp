@@ -791,9 +791,11 @@ struct FastStep {
   AccreteArgs acc;
   StageArgs end;       // end-of-step ComputeRHS: CFL, data checks, new state with ghosts
 };
-void fast_step_args(fv_ctx *ctx, Ctl *ctl, int xin, int xout, int tb, int rb, int k0in, int k0out, int bin,
+// (step s of a round; own_control: with k_control after every step)
+void fast_step_args(fv_ctx *ctx, Ctl *dctl, int s, bool own_control, int xin, int xout, int tb, int rb, int k0in, int k0out, int bin,
                     int gin, int win, int vin, FastStep &f) {
   const int steady = ctx->c.fargo ? 1 : 0;
+  CtlHead *ctl = !own_control && s % 2 == 0 ? &dctl->odd : dctl;
   f.g = ctx->g;
   f.cbv = ctx->c.fargo == 1;
   int ystage = xin;
@@ -817,6 +819,12 @@ void fast_step_args(fv_ctx *ctx, Ctl *ctl, int xin, int xout, int tb, int rb, in
     a.ctl = ctl;
     a.add_bg = a.sub_bg = steady;
     set_acc(ctx, a, gin);
+    if (m == 1 && !own_control) {
+      a.prev = s % 2 == 0 ? dctl : &dctl->odd;
+      a.ctl_out = ctl;
+      a.hist = dctl;
+      a.part_c = ctx->part_c;
+    }
     f.st[m - 1] = a;
   }
   // accretion: the stage evaluations see unchanged boundary fluxes (their
@@ -872,10 +880,32 @@ void visc_device(fv_ctx *ctx, const Geom &g, StageArgs &a, double c_cur, double 
   a.vsrc = ctx->d_vsrc;
 }
 
-void enqueue_fast_step(fv_ctx *ctx, int xin, int xout, int tb, int rb, int k0in, int k0out, int bin, int gin,
+// Rounds whose first stages take the step control along (k_rhs open_step), with
+// one k_control behind the round: wherever the step begins with a first stage
+// (FARGO type 1 begins with k_wsum, viscous steps with k_visc), and the
+// workgroups, each of which reads all partials, are no more than the chip holds
+// at once (512 of 256 threads, two per CU).  us per step with k_control -> with
+// open_step: 64x128 disk 36.1 -> 35.2, 256x256 Riemann problem 37.9 -> 36.3,
+// 512x1024 disk 74.7 -> 74.1 (FP32 53.0 -> 51.9), 1024x2048 Euler disk with
+// seven stages (512 workgroups) 871 -> 860.
+constexpr int OPEN_STEP_BLOCKS = 512;
+bool own_control(const fv_ctx *ctx) {
+  return ctx->c.fargo == 1 || ctx->c.vismodel || ctx->nb_rhs > OPEN_STEP_BLOCKS;
+}
+
+// the step control behind the last of n steps (own_control: behind every step)
+void enqueue_control(fv_ctx *ctx, int n) {
+  const CtlHead *prev = !own_control(ctx) && n % 2 ? &ctx->d_ctl->odd : ctx->d_ctl;
+  long pk = prof_begin(ctx);
+  launch_control(prev, ctx->d_ctl, ctx->part_c, ctx->part_r, ctx->nb_rhs, ctx->st,
+                 ctx->c.vismodel ? ctx->d_vpart : nullptr, ctx->nb_vis);
+  prof_end(ctx, pk, K_CONTROL, 32.0 * ctx->nb_rhs);
+}
+
+void enqueue_fast_step(fv_ctx *ctx, int s, int xin, int xout, int tb, int rb, int k0in, int k0out, int bin, int gin,
                        int win, int vin) {
   FastStep f;
-  fast_step_args(ctx, ctx->d_ctl, xin, xout, tb, rb, k0in, k0out, bin, gin, win, vin, f);
+  fast_step_args(ctx, ctx->d_ctl, s, own_control(ctx), xin, xout, tb, rb, k0in, k0out, bin, gin, win, vin, f);
   const bool vis = ctx->c.vismodel != 0;
   if (f.cbv) {
     long pk = prof_begin(ctx);
@@ -905,17 +935,14 @@ void enqueue_fast_step(fv_ctx *ctx, int xin, int xout, int tb, int rb, int k0in,
   long pk = prof_begin(ctx);
   launch_rhs(f.g, f.end, ctx->V, ctx->st);
   prof_end(ctx, pk, K_RHS_END, 3.0 * word_bytes(ctx));
-  pk = prof_begin(ctx);
-  launch_control(ctx->d_ctl, ctx->part_c, ctx->part_r, ctx->nb_rhs, ctx->st, vis ? ctx->d_vpart : nullptr,
-                 ctx->nb_vis);
-  prof_end(ctx, pk, K_CONTROL, 32.0 * ctx->nb_rhs);
+  if (own_control(ctx)) enqueue_control(ctx, s + 1);
 }
 
 // step-control header of a device-controlled batch of at most nmax steps.
 // ctx->dt is the CFL step of the last CalcTimestep; the first device step
 // takes it after the output-time clipping the host applies at the start of
 // every Step (io/fileio_base.f90:604-620), as k_control does for the others.
-void prime_ctl(const fv_ctx *ctx, Ctl *h, int nmax) {
+void prime_ctl(const fv_ctx *ctx, Ctl *h, int nmax, bool own) {
   std::memset(h, 0, offsetof(Ctl, err_hist));
   double dt = ctx->dt;
   if ((ctx->time + dt) / ctx->t_out > 1.0)
@@ -932,6 +959,7 @@ void prime_ctl(const fv_ctx *ctx, Ctl *h, int nmax) {
   h->beta = ctx->c.beta;
   h->order = ctx->c.order;
   h->nsteps = nmax;
+  h->open = own;  // (each k_control follows the step it evaluates)
   h->vis = ctx->c.vismodel ? 1 : 0;
   h->cvis = ctx->c.cvis;
 }
@@ -994,8 +1022,8 @@ int get_graph(fv_ctx *ctx, int x0, int x1, int tb, int rb, int k0, int b0, int g
   HIPCHK(hipStreamBeginCapture(ctx->st, hipStreamCaptureModeThreadLocal));
   const int g1 = ctx->grav[0] ? 1 - g0 : g0, t1 = ctx->c.fargo == 1;
   for (int s = 0; s < nsteps; s += 2) {
-    enqueue_fast_step(ctx, x0, x1, tb, rb, k0, 1 - k0, b0, g0, w0, v0);
-    enqueue_fast_step(ctx, x1, x0, tb, rb, 1 - k0, k0, 1 - b0, g1, t1 ? 1 - w0 : w0, t1 ? 1 - v0 : v0);
+    enqueue_fast_step(ctx, 0, x0, x1, tb, rb, k0, 1 - k0, b0, g0, w0, v0);
+    enqueue_fast_step(ctx, 1, x1, x0, tb, rb, 1 - k0, k0, 1 - b0, g1, t1 ? 1 - w0 : w0, t1 ? 1 - v0 : v0);
   }
   HIPCHK(hipStreamEndCapture(ctx->st, &graph));
   hipGraphExec_t exec;
@@ -1031,7 +1059,7 @@ int run_batch(fv_ctx *ctx, int nmax, int *done_steps, int *halted) {
   const int k0 = ctx->k0cur, b0 = ctx->bcur, g0 = ctx->gcur, g1 = ctx->grav[0] ? 1 - g0 : g0;
   const int w0 = ctx->wcur, v0 = ctx->vcur, t1 = ctx->c.fargo == 1;
   Ctl *h = ctx->h_ctl;
-  prime_ctl(ctx, h, nmax);
+  prime_ctl(ctx, h, nmax, own_control(ctx));
   // graphs of GRAPH_STEPS steps, the rest of the round in pairs of steps: a
   // graph launch leaves the device idle for about 5 us (64x128 disk, us per step
   // with graphs of 2, 4, 8, 16 steps: 40.5, 39.3, 38.6, 38.3)
@@ -1050,11 +1078,13 @@ int run_batch(fv_ctx *ctx, int nmax, int *done_steps, int *halted) {
     for (int s = whole * GRAPH_STEPS; s < nmax; s += 2) HIPCHK(hipGraphLaunch(pair, ctx->st));
   } else {  // timed or eager: the same launches, issued one by one
     for (int s = 0; s < nmax; s++)
-      enqueue_fast_step(ctx, s % 2 ? x1 : x0, s % 2 ? x0 : x1, tb, rb, s % 2 ? 1 - k0 : k0, s % 2 ? k0 : 1 - k0,
+      enqueue_fast_step(ctx, s, s % 2 ? x1 : x0, s % 2 ? x0 : x1, tb, rb, s % 2 ? 1 - k0 : k0, s % 2 ? k0 : 1 - k0,
                         s % 2 ? 1 - b0 : b0, s % 2 ? g1 : g0, (s % 2 && t1) ? 1 - w0 : w0,
                         (s % 2 && t1) ? 1 - v0 : v0);
     HIPCHK(hipGetLastError());
   }
+  // (graphs hold an even number of steps)
+  if (!own_control(ctx)) enqueue_control(ctx, graphs ? 0 : nmax);
   HIPCHK(hipMemcpyAsync(h, ctx->d_ctl, sizeof(Ctl), hipMemcpyDeviceToHost, ctx->st));
   HIPCHK(hipStreamSynchronize(ctx->st));
   prof_collect(ctx);
@@ -1716,7 +1746,7 @@ struct fv_batch {
   Ctl *d_ctl = nullptr, *h_ctl = nullptr;
   RhsEntry *d_rhs = nullptr, *h_rhs = nullptr;          // [2 parities][m launches][cap]
   RemapEntry *d_remap = nullptr, *h_remap = nullptr;    // [2][cap]
-  ControlEntry *d_cent = nullptr, *h_cent = nullptr;    // [NCAND][cap]
+  ControlEntry *d_cent = nullptr, *h_cent = nullptr;    // [2][NCAND][cap], behind an even / odd step
   // point-mass accretion members: the step's boundary-flux accumulation and
   // UpdateGravity before the end-of-step evaluation, [2 parities][cap] each,
   // acc_n entries used (members in order), acc_bpm workgroups per member
@@ -1830,11 +1860,11 @@ int rebuild(fv_batch *b) {
     BCHK(hipMalloc((void **)&b->d_ctl, sizeof(Ctl) * cap));
     BCHK(hipMalloc((void **)&b->d_rhs, sizeof(RhsEntry) * 2 * m * cap));
     BCHK(hipMalloc((void **)&b->d_remap, sizeof(RemapEntry) * 2 * cap));
-    BCHK(hipMalloc((void **)&b->d_cent, sizeof(ControlEntry) * NCAND * cap));
+    BCHK(hipMalloc((void **)&b->d_cent, sizeof(ControlEntry) * 2 * NCAND * cap));
     BCHK(hipHostMalloc((void **)&b->h_ctl, sizeof(Ctl) * cap));
     BCHK(hipHostMalloc((void **)&b->h_rhs, sizeof(RhsEntry) * 2 * m * cap));
     BCHK(hipHostMalloc((void **)&b->h_remap, sizeof(RemapEntry) * 2 * cap));
-    BCHK(hipHostMalloc((void **)&b->h_cent, sizeof(ControlEntry) * NCAND * cap));
+    BCHK(hipHostMalloc((void **)&b->h_cent, sizeof(ControlEntry) * 2 * NCAND * cap));
     BCHK(hipMalloc((void **)&b->d_bfl, sizeof(BfluxArgs) * 2 * cap));
     BCHK(hipMalloc((void **)&b->d_acc, sizeof(AccreteArgs) * 2 * cap));
     BCHK(hipHostMalloc((void **)&b->h_bfl, sizeof(BfluxArgs) * 2 * cap));
@@ -1881,6 +1911,9 @@ int rebuild(fv_batch *b) {
   return 0;
 }
 
+// as own_control, by the workgroups of the whole launch
+bool batch_own_control(const fv_batch *b, int c) { return b->cand_n[c] > OPEN_STEP_BLOCKS; }
+
 // the launches of one device step of parity p under tiling c
 void enqueue_batch_step(fv_batch *b, int p, int c) {
   const int m = b->m, cap = b->cap, n = (int)b->sims.size();
@@ -1896,7 +1929,13 @@ void enqueue_batch_step(fv_batch *b, int p, int c) {
   }
   launch_rhs_multi(b->d_rhs + (size_t)(p * m + m - 1) * cap, tl, b->cand_n[c], b->V, b->dtype, b->limiter,
                    cand_rows(b, c), b->end_mode, 0, b->st);
-  launch_control_multi(b->d_cent + (size_t)c * cap, n, b->st);
+  if (batch_own_control(b, c)) launch_control_multi(b->d_cent + (size_t)(NCAND + c) * cap, n, b->st);
+}
+// K steps, with the step control behind the last one where the first stages take it along
+void enqueue_batch_steps(fv_batch *b, int K, int c) {
+  for (int s = 0; s < K; s++) enqueue_batch_step(b, s % 2, c);
+  if (!batch_own_control(b, c))
+    launch_control_multi(b->d_cent + (size_t)(K % 2 * NCAND + c) * b->cap, (int)b->sims.size(), b->st);
 }
 
 int batch_graph(fv_batch *b, int K, int c, hipGraphExec_t *out) {
@@ -1907,7 +1946,7 @@ int batch_graph(fv_batch *b, int K, int c, hipGraphExec_t *out) {
     }
   hipGraph_t graph;
   BCHK(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
-  for (int s = 0; s < K; s++) enqueue_batch_step(b, s % 2, c);
+  enqueue_batch_steps(b, K, c);
   BCHK(hipStreamEndCapture(b->st, &graph));
   hipGraphExec_t exec;
   hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
@@ -1947,7 +1986,7 @@ int batch_round(fv_batch *b, const std::vector<int> &want, int K, int c, bool ti
     Ctl *h = &b->h_ctl[d];
     Ctl *dc = b->d_ctl + d;
     if (want[d] > 0) {
-      prime_ctl(x, h, want[d]);
+      prime_ctl(x, h, want[d], batch_own_control(b, c));
     } else {
       std::memset(h, 0, offsetof(Ctl, err_hist));
       h->halt = 1;
@@ -1962,7 +2001,7 @@ int batch_round(fv_batch *b, const std::vector<int> &want, int K, int c, bool ti
     for (int p = 0; p < 2; p++) {
       FastStep f;
       const int gin = (p && x->grav[0]) ? 1 - x->gcur : x->gcur;  // the point mass alternates as the state
-      fast_step_args(x, dc, p ? r.x1 : r.x0, p ? r.x0 : r.x1, r.tb, r.rb, p ? 1 - r.k0 : r.k0,
+      fast_step_args(x, dc, p, batch_own_control(b, c), p ? r.x1 : r.x0, p ? r.x0 : r.x1, r.tb, r.rb, p ? 1 - r.k0 : r.k0,
                      p ? r.k0 : 1 - r.k0, p ? 1 - r.b0 : r.b0, gin, x->wcur, x->vcur, f);  // no FARGO type 1
       if (f.accrete) {
         b->h_bfl[(size_t)p * cap + ai] = f.bfl;
@@ -1978,7 +2017,10 @@ int batch_round(fv_batch *b, const std::vector<int> &want, int K, int c, bool ti
     }
     for (int cc = 0; cc < NCAND; cc++) {
       const int nb = strip_cols(x->c.inum) * strip_blocks(x->c.jnum, rows_of[cc]);
-      b->h_cent[(size_t)cc * cap + d] = ControlEntry{dc, x->part_c, x->part_r, nb};
+      // behind an odd number of steps without their own control: the other header
+      for (int p = 0; p < 2; p++)
+        b->h_cent[(size_t)(p * NCAND + cc) * cap + d] =
+            ControlEntry{p && !batch_own_control(b, cc) ? &dc->odd : dc, dc, x->part_c, x->part_r, nb};
     }
     if (x->grav[0]) ai++;
   }
@@ -1986,18 +2028,18 @@ int batch_round(fv_batch *b, const std::vector<int> &want, int K, int c, bool ti
                         hipMemcpyHostToDevice, b->st));
   BCHK(hipMemcpyAsync(b->d_rhs, b->h_rhs, sizeof(RhsEntry) * 2 * m * cap, hipMemcpyHostToDevice, b->st));
   BCHK(hipMemcpyAsync(b->d_remap, b->h_remap, sizeof(RemapEntry) * 2 * cap, hipMemcpyHostToDevice, b->st));
-  BCHK(hipMemcpyAsync(b->d_cent, b->h_cent, sizeof(ControlEntry) * NCAND * cap, hipMemcpyHostToDevice, b->st));
+  BCHK(hipMemcpyAsync(b->d_cent, b->h_cent, sizeof(ControlEntry) * 2 * NCAND * cap, hipMemcpyHostToDevice, b->st));
   if (b->acc_n) {
     BCHK(hipMemcpyAsync(b->d_bfl, b->h_bfl, sizeof(BfluxArgs) * 2 * cap, hipMemcpyHostToDevice, b->st));
     BCHK(hipMemcpyAsync(b->d_acc, b->h_acc, sizeof(AccreteArgs) * 2 * cap, hipMemcpyHostToDevice, b->st));
   }
   if (timed) {
     BCHK(hipEventRecord(b->t0, b->st));
-    for (int s = 0; s < K; s++) enqueue_batch_step(b, s % 2, c);
+    enqueue_batch_steps(b, K, c);
     BCHK(hipGetLastError());
     BCHK(hipEventRecord(b->t1, b->st));
   } else if (eager_launches()) {
-    for (int s = 0; s < K; s++) enqueue_batch_step(b, s % 2, c);
+    enqueue_batch_steps(b, K, c);
     BCHK(hipGetLastError());
   } else {
     hipGraphExec_t exec;

@@ -62,9 +62,14 @@ struct CtlHead {
   double invdt;
   double cvis, invdt_v;  // viscosity (vis = 1): its Courant number and the last step's viscous 1/dt
   int halt, reason, step, nsteps, flags, vis;
+  int open;              // the step of this header has run and its partials are not yet evaluated
 };
 struct Ctl : CtlHead {
   double err_hist[CTL_HIST], dt_hist[CTL_HIST];
+  // Steps whose first stage takes the step control of the step before along
+  // alternate between the two headers: even steps of a round read the first
+  // and write this one, odd steps the other way round
+  CtlHead odd;
 };
 
 // Boundary-flux accumulation of one step (timedisc_rkfehlberg.f90:216-259):
@@ -79,7 +84,7 @@ struct BfluxArgs {
   double dt;            // host-controlled step; device rounds take Ctl::dt
   int nk, V, NI, NJ, P, inum, jnum, dtype;
   long FS;
-  Ctl *ctl;             // a device-controlled k_bflux launch: dt and halting from here
+  const CtlHead *ctl;   // a device-controlled k_bflux launch: dt and halting from here
 };
 
 // Point-mass accretion (gravity_pointmass.f90:79-85, 383-428).  A state
@@ -98,7 +103,7 @@ struct AccreteArgs {
   double dt;            // ComputeRHS's dt argument (host-controlled)
   int dt_ctl;           // device rounds: dt = Ctl::dt
   int zero_accrate;     // device rounds: the stage evaluations before (dmass = 0, dt > 0) left accrate = 0
-  Ctl *ctl;             // device rounds: halting
+  const CtlHead *ctl;   // device rounds: halting
 };
 
 // One right-hand-side evaluation (timedisc_base.f90:1073-1271) on the RK
@@ -114,7 +119,14 @@ struct StageArgsT {
   double a[MAXK];       // Butcher coefficients of this stage
   int nk;
   double dt;            // time step (host-controlled)
-  Ctl *ctl;             // device-controlled: dt and halting come from here
+  const CtlHead *ctl;   // device-controlled: dt and halting come from here
+  // the first stage of a device-controlled step, where no k_control ran since
+  // the step before (prev set): every workgroup evaluates that step's control
+  // from its partials (part, part_c) and header prev; one writes the new header
+  // to ctl_out (= ctl) and the step's history to hist
+  const CtlHead *prev;
+  CtlHead *ctl_out;
+  Ctl *hist;
   T *kout;              // rhs (interior cells); unused with ynew
   T *yout;              // transformed state incl. ghost cells, or null
   int add_bg, sub_bg;   // FARGO frame change at entry / before the fluxes
@@ -193,7 +205,7 @@ struct RemapArgsT {
   const T *Y;
   T *out;               // remapped interior cells
   double dt_step;       // this%dt (host-controlled)
-  Ctl *ctl;             // device-controlled: dt_step = (time+dt)-time, halting
+  const CtlHead *ctl;   // device-controlled: dt_step = (time+dt)-time, halting
 };
 using RemapArgs = RemapArgsT<double>;
 
@@ -212,6 +224,7 @@ struct RemapEntry {
   RemapArgs a;
 };
 struct ControlEntry {
+  const CtlHead *prev;
   Ctl *ctl;
   const double *part_c, *part_r;
   int nb;
@@ -234,7 +247,7 @@ void launch_remap(const Geom &g, const RemapArgs &a, int V, hipStream_t s);
 // (w2: the w row, of the state's element type, of a second frame change
 // applied in the same pass)
 void launch_frame(const Geom &g, const void *src, void *dst, int sign, int V, hipStream_t s,
-                  const Ctl *ctl = nullptr, const void *w2 = nullptr);
+                  const CtlHead *ctl = nullptr, const void *w2 = nullptr);
 // out (pinned host memory): max, flags, then no
 void launch_reduce(const double *part, int n, double *out, double no, hipStream_t s);
 // Host arrays of the C ABI ([V][NJ][NI], FP64) to and from state buffers.
@@ -257,8 +270,9 @@ void launch_visc(const Geom &g, const StageArgs &a, const VisArgs &v, int V, hip
 // (v + w when add_w); v.update: the dynamic viscosity from that pvar
 void launch_visc_cfl(const Geom &g, const VisArgs &v, const double *pv, int add_w, double *part, int nblocks, int V,
                      hipStream_t s);
+// the step control of the step whose header is prev (if it is open) into ctl;
 // part_v/nbv: the viscous 1/dt partials of the end-of-step k_visc (or null)
-void launch_control(Ctl *ctl, const double *part_c, const double *part_r, int nb, hipStream_t s,
+void launch_control(const CtlHead *prev, Ctl *ctl, const double *part_c, const double *part_r, int nb, hipStream_t s,
                     const double *part_v = nullptr, int nbv = 0);
 // k_visc workgroups of a mesh (tiles of 64 x 8 cells over the ghost-inclusive mesh)
 int visc_blocks(const Geom &g);
@@ -267,7 +281,7 @@ void launch_accrete(const AccreteArgs &p, hipStream_t s);
 // FARGO type 1: w(i) = SUM_j v(i,j)*wfactor(i) / JNUM per ring into the ring
 // arrays (FP64 and, for the precision form, FP32)
 void launch_wsum(const Geom &g, const double *v, double *ring, float *ringf, hipStream_t s,
-                 const Ctl *ctl = nullptr);
+                 const CtlHead *ctl = nullptr);
 // k_rhs: strips of 64 columns x up to STRIP_ROWS rows, one per wave,
 // STRIP_WAVES of them above each other in a workgroup
 constexpr int STRIP_ROWS = 16, STRIP_WAVES = 4;

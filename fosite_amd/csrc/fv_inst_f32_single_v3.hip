@@ -4,6 +4,6 @@
 namespace fv {
 template void rhs_single<float, 3>(const Geom &, const StageArgsT<float> &, hipStream_t);
 template void remap_single<float>(const Geom &, const RemapArgsT<float> &, int, hipStream_t);
-template void frame_single<float>(const Geom &, const void *, void *, int, int, const Ctl *, const void *,
+template void frame_single<float>(const Geom &, const void *, void *, int, int, const CtlHead *, const void *,
                                   hipStream_t);
 }  // namespace fv

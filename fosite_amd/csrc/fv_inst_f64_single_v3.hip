@@ -4,6 +4,6 @@
 namespace fv {
 template void rhs_single<double, 3>(const Geom &, const StageArgsT<double> &, hipStream_t);
 template void remap_single<double>(const Geom &, const RemapArgsT<double> &, int, hipStream_t);
-template void frame_single<double>(const Geom &, const void *, void *, int, int, const Ctl *, const void *,
+template void frame_single<double>(const Geom &, const void *, void *, int, int, const CtlHead *, const void *,
                                    hipStream_t);
 }  // namespace fv

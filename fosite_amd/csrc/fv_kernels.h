@@ -288,7 +288,7 @@ __device__ __forceinline__ bool same_sign(float a, float b) {
 struct StepTime {
   double dt, dts;  // the step control's dt; this%dt
   int halt;
-  __device__ __forceinline__ StepTime(const Geom &g, const Ctl *ctl, double dt_step) {
+  __device__ __forceinline__ StepTime(const Geom &g, const CtlHead *ctl, double dt_step) {
     const double *h = ctl ? &ctl->time : g.ring;
     const int hf = *(ctl ? &ctl->halt : reinterpret_cast<const int *>(g.ring));
     const double t = h[0];
@@ -969,6 +969,90 @@ static __device__ void control_next(CtlHead *c, double invdt, int flags, double 
   if (c->step >= c->nsteps) halt(c, H_BATCH);
 }
 
+// Step control of the step of header prev, by the 256 threads of a workgroup:
+// embedded error from the last stage's partials, accept test, then CFL and data
+// checks from the end-of-step partials and the next time step.  Every thread
+// ends with the new header.  A halted or not open header stays as it is.
+struct ControlShared {
+  double e[4], m[4], v[4];
+  int f[4];
+};
+struct StepControl {
+  CtlHead h;
+  double err, dt_ran;
+  int step, ran;
+  __device__ __forceinline__ StepControl(const CtlHead *prev, const double *part_c, const double *part_r, int nb,
+                                         const double *part_v, int nbv, ControlShared &sh) {
+    // the whole header first: one memory latency beside the partials', and the
+    // decisions below then run on registers
+    h = *prev;
+    const int t = threadIdx.x;
+    double e = -DBL_MAX, m = -DBL_MAX, v = -DBL_MAX;
+    int f = 0;
+    constexpr int Q = 4;  // partials per thread and pass, all loaded before the first is used
+    for (int b0 = t; b0 < nb; b0 += Q * 256) {
+      double pe[Q], pm[Q], pf[Q];
+#pragma unroll
+      for (int q = 0; q < Q; q++) {  // (beyond the end: the last one again)
+        const int b = min(b0 + q * 256, nb - 1);
+        pe[q] = part_c[2 * b];
+        pm[q] = part_r[2 * b];
+        pf[q] = part_r[2 * b + 1];
+      }
+#pragma unroll
+      for (int q = 0; q < Q; q++) {
+        e = fmax2(e, pe[q]);
+        m = fmax2(m, pm[q]);
+        f |= (int)pf[q];
+      }
+    }
+    if (t == 0) {  // the corner cells' partial
+      m = fmax2(m, part_r[2 * nb]);
+      f |= (int)part_r[2 * nb + 1];
+    }
+    if (part_v) {
+      for (int b = t; b < nbv; b += 256) v = fmax2(v, part_v[2 * b]);
+    }
+    ran = !h.halt && h.open;
+    step = h.step;
+    dt_ran = h.dt;
+    err = 0.0;
+    if (!ran) return;
+    // one barrier: wave results to LDS, every thread combines
+    e = wave_max(e);
+    m = wave_max(m);
+    v = wave_max(v);
+    f = wave_or(f);
+    if ((t & 63) == 0) {
+      sh.e[t >> 6] = e;
+      sh.m[t >> 6] = m;
+      sh.v[t >> 6] = v;
+      sh.f[t >> 6] = f;
+    }
+    __syncthreads();
+    e = m = v = -DBL_MAX;  // from -DBL_MAX in wave order, as blk_max
+    f = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      e = fmax2(e, sh.e[k]);
+      m = fmax2(m, sh.m[k]);
+      v = fmax2(v, sh.v[k]);
+      f |= sh.f[k];
+    }
+    err = e;
+    control_accept(&h, e);
+    if (!h.halt) control_next(&h, m, f, v);
+  }
+  // by one thread: the new header, and the history of the step that ran
+  __device__ __forceinline__ void store(CtlHead *out, Ctl *hist) const {
+    if (ran) {
+      hist->err_hist[step] = err;
+      hist->dt_hist[step] = dt_ran;
+    }
+    *out = h;
+  }
+};
+
 // ------------------------------------------------ boundary-flux accounting
 // One element of the boundary rows (west/east rows of every field first, then
 // south/north): loaded, then its new bxflux(j,side,l) / byflux(i,side,l) after
@@ -1344,7 +1428,7 @@ __global__ __launch_bounds__(256) void k_remap_multi(const RemapEntry *__restric
 // - rho*w2, rounded as the two passes round.  ctl: a device-controlled step,
 // skipped once the round has halted.
 template <typename T, int V>
-__global__ __launch_bounds__(256) void k_frame(Geom g, const T *src, T *dst, int sign, const Ctl *ctl, const T *w2) {
+__global__ __launch_bounds__(256) void k_frame(Geom g, const T *src, T *dst, int sign, const CtlHead *ctl, const T *w2) {
   if (ctl && ctl->halt) return;
   const int i = blockIdx.x * 64 + threadIdx.x, j = blockIdx.y * 4 + threadIdx.y;
   if (i >= g.NI || j >= g.NJ) return;
@@ -1618,7 +1702,7 @@ void rhs_single(const Geom &g, const StageArgsT<T> &a, hipStream_t s);
 template <typename T>
 void remap_single(const Geom &g, const RemapArgsT<T> &a, int V, hipStream_t s);
 template <typename T>
-void frame_single(const Geom &g, const void *src, void *dst, int sign, int V, const Ctl *ctl, const void *w2,
+void frame_single(const Geom &g, const void *src, void *dst, int sign, int V, const CtlHead *ctl, const void *w2,
                   hipStream_t s);
 template <typename T, int V>
 void rhs_multi(const RhsEntry *tab, const unsigned *tiles, int n, int limiter, int rows, int mode, int nk,

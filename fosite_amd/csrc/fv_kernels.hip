@@ -8,75 +8,16 @@
 
 namespace fv {
 
-// Step control of a device-controlled batch (one block): embedded error of
-// the step from the partials of the last stage, accept test, then CFL and
-// data checks from the end-of-step k_rhs partials and the next time step.
-__device__ __forceinline__ void control_block(Ctl *ctl, const double *part_c, const double *part_r, int nb,
-                                              const double *part_v = nullptr, int nbv = 0) {
-  __shared__ double rede[4], redm[4], redv[4];
-  __shared__ int redi[4];
-  // the whole header first: one memory latency beside the partials', and the
-  // decisions below then run on registers
-  CtlHead h = *ctl;
-  double e = -DBL_MAX, m = -DBL_MAX, v = -DBL_MAX;
-  int f = 0;
-  constexpr int Q = 4;  // partials per thread and pass, all loaded before the first is used
-  for (int b0 = threadIdx.x; b0 < nb; b0 += Q * 256) {
-    double pe[Q], pm[Q], pf[Q];
-#pragma unroll
-    for (int q = 0; q < Q; q++) {  // (beyond the end: the last one again)
-      const int b = min(b0 + q * 256, nb - 1);
-      pe[q] = part_c[2 * b];
-      pm[q] = part_r[2 * b];
-      pf[q] = part_r[2 * b + 1];
-    }
-#pragma unroll
-    for (int q = 0; q < Q; q++) {
-      e = fmax2(e, pe[q]);
-      m = fmax2(m, pm[q]);
-      f |= (int)pf[q];
-    }
-  }
-  if (threadIdx.x == 0) {  // the corner cells' partial
-    m = fmax2(m, part_r[2 * nb]);
-    f |= (int)part_r[2 * nb + 1];
-  }
-  if (part_v) {
-    for (int b = threadIdx.x; b < nbv; b += blockDim.x) v = fmax2(v, part_v[2 * b]);
-  }
-  if (h.halt) return;
-  // one barrier: wave results to LDS, thread 0 combines
-  e = wave_max(e);
-  m = wave_max(m);
-  v = wave_max(v);
-  f = wave_or(f);
-  const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    rede[w] = e;
-    redm[w] = m;
-    redv[w] = v;
-    redi[w] = f;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {  // from -DBL_MAX in wave order, as blk_max
-    e = m = v = -DBL_MAX;
-    f = 0;
-    for (int k = 0; k < nw; k++) {
-      e = fmax2(e, rede[k]);
-      m = fmax2(m, redm[k]);
-      v = fmax2(v, redv[k]);
-      f |= redi[k];
-    }
-    ctl->err_hist[h.step] = e;
-    ctl->dt_hist[h.step] = h.dt;
-    control_accept(&h, e);
-    if (!h.halt) control_next(&h, m, f, v);
-    *static_cast<CtlHead *>(ctl) = h;
-  }
+// Step control of a device-controlled batch (one block), where no k_rhs takes it along
+__device__ __forceinline__ void control_block(const CtlHead *prev, Ctl *ctl, const double *part_c, const double *part_r,
+                                              int nb, const double *part_v = nullptr, int nbv = 0) {
+  __shared__ ControlShared sh;
+  const StepControl c(prev, part_c, part_r, nb, part_v, nbv, sh);
+  if (threadIdx.x == 0) c.store(ctl, ctl);
 }
-__global__ __launch_bounds__(256) void k_control(Ctl *ctl, const double *part_c, const double *part_r, int nb,
-                                                 const double *part_v, int nbv) {
-  control_block(ctl, part_c, part_r, nb, part_v, nbv);
+__global__ __launch_bounds__(256) void k_control(const CtlHead *prev, Ctl *ctl, const double *part_c,
+                                                 const double *part_r, int nb, const double *part_v, int nbv) {
+  control_block(prev, ctl, part_c, part_r, nb, part_v, nbv);
 }
 // host-controlled steps: the boundary-flux accumulation of a step
 __global__ __launch_bounds__(256) void k_bflux(BfluxArgs bf) {
@@ -114,7 +55,7 @@ __global__ __launch_bounds__(256) void k_accrete_multi(const AccreteArgs *__rest
 // one block per mesh of a batch
 __global__ __launch_bounds__(256) void k_control_multi(const ControlEntry *__restrict__ tab) {
   const ControlEntry &E = tab[blockIdx.x];
-  control_block(E.ctl, E.part_c, E.part_r, E.nb);
+  control_block(E.prev, E.ctl, E.part_c, E.part_r, E.nb);
 }
 
 // max over part[2b] and OR over part[2b+1]; out[0] = max, out[1] = flags,
@@ -147,7 +88,7 @@ __global__ __launch_bounds__(256) void k_reduce(const double *part, int n, doubl
 // costing one memory latency.
 constexpr int WS_RINGS = 16, WS_ROWS = 256, WS_RG = 64 / WS_RINGS;
 __global__ __launch_bounds__(256) void k_wsum(Geom g, const double *__restrict__ v, double *ring, float *ringf,
-                                              const Ctl *ctl) {
+                                              const CtlHead *ctl) {
   __shared__ double buf[2][WS_ROWS][WS_RINGS];
   if (ctl && ctl->halt) return;  // a device-controlled step after the round halted
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -391,16 +332,16 @@ void launch_remap(const Geom &g, const RemapArgs &a, int V, hipStream_t s) {
     remap_single<double>(g, a, V, s);
   }
 }
-void launch_frame(const Geom &g, const void *src, void *dst, int sign, int V, hipStream_t s, const Ctl *ctl,
+void launch_frame(const Geom &g, const void *src, void *dst, int sign, int V, hipStream_t s, const CtlHead *ctl,
                   const void *w2) {
   if (g.dtype == 1)
     frame_single<float>(g, src, dst, sign, V, ctl, w2, s);
   else
     frame_single<double>(g, src, dst, sign, V, ctl, w2, s);
 }
-void launch_control(Ctl *ctl, const double *part_c, const double *part_r, int nb, hipStream_t s,
+void launch_control(const CtlHead *prev, Ctl *ctl, const double *part_c, const double *part_r, int nb, hipStream_t s,
                     const double *part_v, int nbv) {
-  hipLaunchKernelGGL(k_control, dim3(1), dim3(256), 0, s, ctl, part_c, part_r, nb, part_v, nbv);
+  hipLaunchKernelGGL(k_control, dim3(1), dim3(256), 0, s, prev, ctl, part_c, part_r, nb, part_v, nbv);
 }
 int visc_blocks(const Geom &g) { return ((g.NI + VT_X - 1) / VT_X) * ((g.NJ + VT_Y - 1) / VT_Y); }
 void launch_rhs_multi(const RhsEntry *tab, const unsigned *tiles, int ntiles, int V, int dtype, int limiter,
@@ -428,7 +369,7 @@ void launch_bflux_multi(const BfluxArgs *tab, int n, int bpm, hipStream_t s) {
 void launch_accrete_multi(const AccreteArgs *tab, int n, hipStream_t s) {
   hipLaunchKernelGGL(k_accrete_multi, dim3(n), dim3(64, 4), 0, s, tab);
 }
-void launch_wsum(const Geom &g, const double *v, double *ring, float *ringf, hipStream_t s, const Ctl *ctl) {
+void launch_wsum(const Geom &g, const double *v, double *ring, float *ringf, hipStream_t s, const CtlHead *ctl) {
   hipLaunchKernelGGL(k_wsum, dim3((g.NI + WS_RINGS - 1) / WS_RINGS), dim3(256), 0, s, g, v, ring, ringf, ctl);
 }
 void launch_bflux(const BfluxArgs &bf, hipStream_t s) {

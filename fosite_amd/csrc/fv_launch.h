@@ -81,7 +81,7 @@ void remap_single(const Geom &g, const RemapArgsT<T> &a, int V, hipStream_t s) {
     hipLaunchKernelGGL((k_remap<T, 4>), grid, block, 0, s, g, a);
 }
 template <typename T>
-void frame_single(const Geom &g, const void *src, void *dst, int sign, int V, const Ctl *ctl, const void *w2,
+void frame_single(const Geom &g, const void *src, void *dst, int sign, int V, const CtlHead *ctl, const void *w2,
                   hipStream_t s) {
   dim3 grid((g.NI + 63) / 64, (g.NJ + 3) / 4), block(64, 4);
   const T *sp = static_cast<const T *>(src);

@@ -78,8 +78,27 @@ struct StripOut {
   int flags, halted;
 };
 
+// The first stage of a device-controlled step evaluates the control of the step
+// before, in every workgroup on the same partials, beside its own loads; the
+// workgroup of tile 0 writes the new header.  This replaces a k_control launch
+// per step (4.3 to 4.5 us, most of it launch and memory latency); letting the
+// last workgroup of the end-of-step launch do it costs an L2 write-back per
+// workgroup instead.
+template <int MODE, int NK>
+constexpr bool kTakesControl = MODE == M_STAGE && NK == 1;
+template <typename T>
+__device__ __forceinline__ void open_step(const StageArgsT<T> &a, int b, int nb, ControlShared &sh, double &dt,
+                                          int &halt) {
+  StepControl c(a.prev, a.part_c, a.part, nb, nullptr, 0, sh);
+  c.h.open = 1;
+  if (b == 0 && threadIdx.x == 0) c.store(a.ctl_out, a.hist);
+  dt = c.h.dt;
+  halt = c.h.halt;
+}
+
 template <typename T, int V, int LIM, int NK, int MODE, int RMAX>
-__device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T> &a, int bx, int j0, int nr, T *hx) {
+__device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T> &a, int bx, int j0, int nr, T *hx,
+                                              int b, int nb, ControlShared &csh) {
   constexpr bool kRemap = MODE == M_REMAP, kEnd = MODE == M_END || kRemap, kLast = MODE == M_LAST;
   using Row = RowIn<T, V, NK>;
   using Comb = Combination<T, V, NK>;
@@ -180,10 +199,13 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
   const T dAxn = rg<T>(g, R_DAXW, i + 1), dAy = rg<T>(g, R_DAYS, i);
   const T dydzdV = rg<T>(g, R_DYDZDV, i), dzdxdV = rg<T>(g, R_DZDXDV, i);
   const SourceRing<T, V> sr(g, a, i);
-  const StepTime st(g, a.ctl, kRemap ? a.dt_step : 0.0);
+  StepTime st(g, a.ctl, kRemap ? a.dt_step : 0.0);
   const double w_d = kRemap ? ring(g, R_W, i) : 0.0, dly_d = kRemap ? ring(g, R_DLY, i) : 1.0;
   const double ew_d = kRemap ? ring(g, R_W, is) : 0.0, edly_d = kRemap ? ring(g, R_DLY, is) : 1.0;
   asm volatile("" ::: "memory");  // keeps the loads above this branch
+  if constexpr (kTakesControl<MODE, NK>) {
+    if (a.prev) open_step<T>(a, b, nb, csh, st.dt, st.halt);
+  }
   if (st.halt) return {0.0, 0.0, 0, 1};
   const In<T, V, NK, true> in(g, a, want_check, a.ctl ? st.dt : a.dt);
   // kRemap: the strip's columns (from two rows below its first) and the edge
@@ -626,16 +648,21 @@ __device__ __forceinline__ void rhs_aux_block(const Geom &g, const StageArgsT<T>
 
 // one workgroup: SWAVES strips of `rows` rows above each other
 template <typename T, int V, int LIM, int NK, int MODE, int RMAX>
-__device__ __forceinline__ void rhs_block(const Geom &g, const StageArgsT<T> &a, int rows, int bx, int by, int b) {
+__device__ __forceinline__ void rhs_block(const Geom &g, const StageArgsT<T> &a, int rows, int bx, int by, int b,
+                                          int nb) {
   __shared__ T hx[SWAVES][RMAX * HX<V>];
   __shared__ double redd[SWAVES];
   __shared__ int redi[SWAVES];
+  __shared__ ControlShared csh;
   const int t = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int j0 = GH + (by * SWAVES + wv) * rows, nr = min(rows, GH + g.jnum - j0);
   StripOut o{-DBL_MAX, -DBL_MAX, 0, 0};
   if (nr > 0)
-    o = rhs_strip<T, V, LIM, NK, MODE, RMAX>(g, a, bx, j0, nr, hx[wv]);
-  else
+    o = rhs_strip<T, V, LIM, NK, MODE, RMAX>(g, a, bx, j0, nr, hx[wv], b, nb, csh);
+  else if (kTakesControl<MODE, NK> && a.prev) {  // (joins the barrier)
+    double dt;
+    open_step<T>(a, b, nb, csh, dt, o.halted);
+  } else
     o.halted = a.ctl && a.ctl->halt;
   if (o.halted) return;
   if constexpr (MODE == M_LAST) {
@@ -669,7 +696,7 @@ __global__ __launch_bounds__(64 * SWAVES, (strip_occupancy<T, V, NK, MODE>())) v
   if (k >= 0) {  // behind the strips' workgroups, so that the XCDs' shares of those stay even
     if constexpr (MODE >= M_END) rhs_aux_block<T, V, MODE == M_REMAP>(g, a, k, gridDim.x - grid, n);
   } else if (t < n) {
-    rhs_block<T, V, LIM, NK, MODE, RMAX>(g, a, g.rows, t % nbx, t / nbx, t);
+    rhs_block<T, V, LIM, NK, MODE, RMAX>(g, a, g.rows, t % nbx, t / nbx, t, n);
   }
 }
 
@@ -686,11 +713,11 @@ __global__ __launch_bounds__(64 * SWAVES, (strip_occupancy<T, V, NK, MODE>())) v
   const int nbx = strip_cols(E.g.inum), nby = strip_blocks(E.g.jnum, rows), bx = tile_bx(e), by = tile_by(e);
   if (MODE == M_REMAP && !a.remap) {  // a member without FARGO beside others
     if (by < nby)
-      rhs_block<T, V, LIM, NK, M_END, RMAX>(E.g, a, rows, bx, by, bx + by * nbx);
+      rhs_block<T, V, LIM, NK, M_END, RMAX>(E.g, a, rows, bx, by, bx + by * nbx, nbx * nby);
     else
       rhs_aux_block<T, V, false>(E.g, a, bx, rhs_aux_max(E.g, V), nbx * nby);
   } else if (by < nby) {
-    rhs_block<T, V, LIM, NK, MODE, RMAX>(E.g, a, rows, bx, by, bx + by * nbx);
+    rhs_block<T, V, LIM, NK, MODE, RMAX>(E.g, a, rows, bx, by, bx + by * nbx, nbx * nby);
   } else if (MODE >= M_END) {
     rhs_aux_block<T, V, MODE == M_REMAP>(E.g, a, bx, rhs_aux_max(E.g, V), nbx * nby);
   }
