@@ -1239,7 +1239,7 @@ extern "C" int fv_create(fv_ctx **out, const fv_config *cfg) {
     if (ok && c.dtype == 1) ok = hipMalloc((void **)&ctx->gravf[q], sizeof(float) * 2 * ctx->NI) == hipSuccess;
   }
   if (c.vismodel) {
-    ctx->nb_vis = visc_blocks(g);
+    ctx->nb_vis = visc_blocks(g.NI, g.NJ);
     ok = ok && dalloc(&ctx->d_vsrc, sizeof(double) * (ctx->V - 1) * ctx->FS) &&
          dalloc(&ctx->d_vpart, sizeof(double) * 2 * ctx->nb_vis);
   }
@@ -1377,7 +1377,7 @@ extern "C" int fv_device_bytes(const fv_config *c, double *bytes) {
     b += 2.0 * 8.0 * NJ * P + (8.0 + (c->dtype == 1 ? 4.0 : 0.0)) * R_COUNT * NI;
   if (c->outbound) b += 2.0 * (8.0 * (PM_HDR + 2.0 * NI) + (c->dtype == 1 ? 4.0 * 2.0 * NI : 0.0));
   if (c->vismodel)                                      // viscous source, its step partials
-    b += 8.0 * (V - 1.0) * NJ * P + 16.0 * std::ceil(NI / 64.0) * std::ceil(NJ / 8.0);
+    b += 8.0 * (V - 1.0) * NJ * P + 16.0 * visc_blocks((int)NI, (int)NJ);
   if (c->vismodel >= 2)                                 // viscosity, e_phi/r, r^2; Euler ALPHA: sound speeds
     b += (c->vismodel == 2 && V == 4 ? 6.0 : 4.0) * 8.0 * NJ * P;
   b += 2.0 * 2.0 * 8.0 * nbp;                          // CFL and error partials

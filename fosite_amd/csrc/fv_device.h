@@ -274,8 +274,25 @@ void launch_visc_cfl(const Geom &g, const VisArgs &v, const double *pv, int add_
 // part_v/nbv: the viscous 1/dt partials of the end-of-step k_visc (or null)
 void launch_control(const CtlHead *prev, Ctl *ctl, const double *part_c, const double *part_r, int nb, hipStream_t s,
                     const double *part_v = nullptr, int nbv = 0);
-// k_visc workgroups of a mesh (tiles of 64 x 8 cells over the ghost-inclusive mesh)
-int visc_blocks(const Geom &g);
+// k_visc: strips of up to VW columns (two halo lanes at either side of a wave),
+// VWAVES of them above each other in a workgroup.  Columns per strip: corner
+// cells take the y boundary's value from the lane of the edge column, so no
+// strip begins with the last column
+constexpr int VW = 60, VWAVES = 4, VROWS = 16;
+__host__ __device__ inline int visc_width(int NI) {
+  return NI % VW != 1 ? VW : NI % (VW - 1) != 1 ? VW - 1 : VW - 2;
+}
+__host__ __device__ inline int visc_cols(int NI) { return (NI + visc_width(NI) - 1) / visc_width(NI); }
+// rows per strip: about two waves per SIMD, and no more halo than half of the rows read
+__host__ __device__ inline int visc_rows(int NI, int NJ) {
+  const long r = ((long)visc_cols(NI) * NJ + 2047) / 2048;
+  return r < 4 ? 4 : r > VROWS ? VROWS : (int)r;
+}
+// workgroups of a mesh of NI x NJ cells, ghost cells included
+__host__ __device__ inline int visc_blocks(int NI, int NJ) {
+  const int rows = visc_rows(NI, NJ) * VWAVES;
+  return visc_cols(NI) * ((NJ + rows - 1) / rows);
+}
 void launch_bflux(const BfluxArgs &bf, hipStream_t s);
 void launch_accrete(const AccreteArgs &p, hipStream_t s);
 // FARGO type 1: w(i) = SUM_j v(i,j)*wfactor(i) / JNUM per ring into the ring

@@ -538,42 +538,9 @@ struct In {
     stage_sum(y, kv, s);
   }
 
-  // stage states of two interior cells (p0, p1 say which are wanted): all
-  // loads of both cells are issued before any arithmetic
-  __forceinline__ __device__ void interior2(bool p0, int ia, int ja, T *s0, bool p1, int ib, int jb, T *s1) const {
-    const unsigned x0 = (unsigned)ja * (unsigned)g.P + (unsigned)ia;
-    const unsigned x1 = (unsigned)jb * (unsigned)g.P + (unsigned)ib;
-    T y0[V], y1[V], k0[KA][V], k1[KA][V];
-    if (p0) {
-#pragma unroll
-      for (int l = 0; l < V; l++) y0[l] = (a.Y + l * g.FS)[x0];
-#pragma unroll
-      for (int q = 0; q < KM; q++)
-        if (q < nk) {
-#pragma unroll
-          for (int l = 0; l < V; l++) k0[q][l] = (a.k[q] + l * g.FS)[x0];
-        }
-    }
-    if (p1) {
-#pragma unroll
-      for (int l = 0; l < V; l++) y1[l] = (a.Y + l * g.FS)[x1];
-#pragma unroll
-      for (int q = 0; q < KM; q++)
-        if (q < nk) {
-#pragma unroll
-          for (int l = 0; l < V; l++) k1[q][l] = (a.k[q] + l * g.FS)[x1];
-        }
-    }
-    stage_sum(y0, k0, s0);
-    stage_sum(y1, k1, s1);
-  }
-
   // ComputeRHS transform (timedisc_base.f90:1098-1208): ur = cvar after the
   // frame change, CenterBoundary and PMIN (real frame), pr = pvar at that
   // point, uc = cvar handed to the fluxes
-  __forceinline__ __device__ void transform(int i, const T *s, T *ur, T *pr, T *uc) const {
-    transform_at(rg<T>(g, R_W, i), s, ur, pr, uc);
-  }
   __forceinline__ __device__ void transform_at(T w, const T *s, T *ur, T *pr, T *uc) const {
     to_prim(w, s, ur, pr);
     comoving(w, s, ur, pr, uc);
@@ -625,70 +592,7 @@ struct In {
     c2p<T, V>(s, p, gam);
   }
 
-  // absorbing boundary, x direction (absorbing_math) at row j
-  __forceinline__ __device__ void absorbing_x(int east, int j, T *p) const {
-    const int imin = GH, imax = GH + g.inum - 1;
-    const int i1 = east ? imax : imin, i2 = east ? imax - 1 : imin + 1;
-    const int iL = i1 < i2 ? i1 : i2, iR = i1 < i2 ? i2 : i1;
-    T pL[V], pR[V];
-    prim_interior(iL, j, pL);
-    prim_interior(iR, j, pR);
-    absorbing_math<T, V>(east, AbsorbingSpeeds<T>(g, east), gam, pL, pR, p);
-  }
-
-  // x-ghost (side, layer 1..2) at interior row j
-  __forceinline__ __device__ void ghost_we(int east, int gl, int j, T *p) const {
-    const int imin = GH, imax = GH + g.inum - 1, bc = east ? g.bc[1] : g.bc[0];
-    if (bc == NO_GRADIENTS)
-      prim_interior(east ? imax : imin, j, p);
-    else if (bc == PERIODIC)
-      prim_interior(east ? imin + gl - 1 : imax - gl + 1, j, p);
-    else
-      absorbing_x(east, j, p);
-  }
-  // y-ghost (side, layer) at interior column i
-  __forceinline__ __device__ void ghost_sn(int north, int gl, int i, T *p) const {
-    const int jmin = GH, jmax = GH + g.jnum - 1, bc = north ? g.bc[3] : g.bc[2];
-    if (bc == NO_GRADIENTS)
-      prim_interior(i, north ? jmax : jmin, p);
-    else
-      prim_interior(i, north ? jmin + gl - 1 : jmax - gl + 1, p);
-  }
-
-  // pvar of any ghost cell after CenterBoundary: boundary rules in the order
-  // W, E, S, N, then SetCornerEdges (boundary_generic.f90:434-517)
-  __forceinline__ __device__ void ghost_prim(int i, int j, T *p) const {
-    const int imin = GH, imax = GH + g.inum - 1, jmin = GH, jmax = GH + g.jnum - 1;
-    const bool xg = i < imin || i > imax, yg = j < jmin || j > jmax;
-    if (xg && !yg) {
-      const int east = i > imax;
-      ghost_we(east, east ? i - imax : imin - i, j, p);
-    } else if (yg && !xg) {
-      const int north = j > jmax;
-      ghost_sn(north, north ? j - jmax : jmin - j, i, p);
-    } else {
-      const int east = i > imax, north = j > jmax;
-      const int ga = east ? i - imax : imin - i, gb = north ? j - jmax : jmin - j;
-      const int ir = east ? imax : imin, jr = north ? jmax : jmin;
-      if (ga == 2 && gb == 1) {
-        ghost_we(east, 2, jr, p);
-      } else if (ga == 1 && gb == 2) {
-        ghost_sn(north, 2, ir, p);
-      } else {
-        T px[V], py[V];
-        ghost_we(east, ga, jr, px);
-        ghost_sn(north, gb, ir, py);
-#pragma unroll
-        for (int l = 0; l < V; l++) p[l] = T(0.5) * (px[l] + py[l]);
-      }
-    }
-  }
-
   // final ghost state: PMIN round trip, prim->cons, data check, frame change
-  __forceinline__ __device__ void ghost_final(int i, int j, T *u, T *p, int &flags) const {
-    ghost_prim(i, j, p);
-    ghost_from_prim(rg<T>(g, R_W, i), p, u, flags);
-  }
   __forceinline__ __device__ void ghost_from_prim(T w, T *p, T *u, int &flags) const {
     if (V == 4 && a.pmin_clamp) p[3] = fmax2(p[3], (T)g.pmin);
     p2c<T, V>(p, u, gam);
@@ -1472,255 +1376,6 @@ __global__ __launch_bounds__(256) void k_frame(Geom g, const T *src, T *dst, int
   for (int l = 0; l < V; l++) dst[l * g.FS + ix] = u[l];
 }
 
-// ------------------------------------------------------------- viscosity
-// dynamic viscosity of one cell from the local angular velocity
-// e_phi/r . v + Omega (sources_viscosity.f90:377-394): ALPHA (etafkt_alpha)
-// alpha*rho*cs^2/|Omega_l|, BETA (etafkt_beta, 457-466) beta*rho*r^2*|Omega_l|
-// with the bary-centre radius
-__device__ __forceinline__ double alpha_dynvis(const VisArgs &va, long ix, long FS, double rho, double vx, double vy,
-                                               double cs) {
-  double om = va.ephir[ix] * vx;
-  om = om + va.ephir[FS + ix] * vy;
-  om = om + va.omega;
-  if (va.model == VIS_BETA) return va.dynconst * rho * va.ephir[2 * FS + ix] * fabs(om);
-  return va.dynconst * rho * (cs * cs) / fabs(om);
-}
-// Divergence of a vector field in 2-D curvilinear coordinates from its face
-// averages (mesh_midpoint.f90:156-232, 586-630): arguments are the west,
-// own, east x components and the south, own, north y components; the z terms
-// of the reference's expression are zero and kept as such (they turn a -0
-// into +0)
-__device__ __forceinline__ double div_faces(const Geom &g, int i, double xw, double x0, double xe, double ys,
-                                            double y0, double yn) {
-  const double fw = 0.5 * (xw + x0), fe = 0.5 * (xe + x0), fs = 0.5 * (ys + y0), fn = 0.5 * (yn + y0);
-  return ring(g, R_DYDZDV, i) * (ring(g, R_DAXE, i) * fe - ring(g, R_DAXW, i) * fw) +
-         ring(g, R_DZDXDV, i) * (ring(g, R_DAYN, i) * fn - ring(g, R_DAYS, i) * fs) + 0.0 * (0.0 * 0.0 - 0.0 * 0.0) +
-         0.0 * 0.0 + 0.0 * 0.0 - 0.0 * 0.0 - 0.0 * 0.0;
-}
-
-// the divergence part of k_visc for the interior cell (i, j) at (r, c) of
-// the inner region
-template <int V, int SX, int RX>
-__device__ __forceinline__ void visc_divergence(const Geom &g, const VisArgs &va, int i, int j, int r, int c,
-                                                double (*Fu)[SX], double (*Fv)[SX], double (*Txx)[RX],
-                                                double (*Tyy)[RX], double (*Txy)[RX]) {
-  const double dydzdV = ring(g, R_DYDZDV, i), dzdxdV = ring(g, R_DZDXDV, i);
-  const double axw = ring(g, R_DAXW, i), axe = ring(g, R_DAXE, i), ays = ring(g, R_DAYS, i), ayn = ring(g, R_DAYN, i);
-  const double cxyx = ring(g, R_CXYX, i), cyxy = ring(g, R_CYXY, i);
-  const double xx0 = Txx[r][c], xy0 = Txy[r][c], yy0 = Tyy[r][c];
-  const double sx = dydzdV * (axe * (0.5 * (Txx[r][c + 1] + xx0)) - axw * (0.5 * (Txx[r][c - 1] + xx0))) +
-                    dzdxdV * (ayn * (0.5 * (Txy[r + 1][c] + xy0)) - ays * (0.5 * (Txy[r - 1][c] + xy0))) +
-                    0.0 * (0.0 * 0.0 - 0.0 * 0.0) + cxyx * xy0 + 0.0 * 0.0 - cyxy * yy0 - 0.0 * 0.0;
-  const double sy = dydzdV * (axe * (0.5 * (Txy[r][c + 1] + xy0)) - axw * (0.5 * (Txy[r][c - 1] + xy0))) +
-                    dzdxdV * (ayn * (0.5 * (Tyy[r + 1][c] + yy0)) - ays * (0.5 * (Tyy[r - 1][c] + yy0))) +
-                    0.0 * (0.0 * 0.0 - 0.0 * 0.0) + (-cxyx) * xx0 + 0.0 * 0.0 - (-cyxy) * xy0 - 0.0 * 0.0;
-  const long ix = cidx(g, i, j);
-  va.src[ix] = sx;
-  va.src[g.FS + ix] = sy;
-  if constexpr (V == 4) {
-    // (T.v)_x and (T.v)_y at the cell (dr, dc) of the inner region
-    auto tvx = [&](int dr, int dc) {
-      return Fu[dr + 1][dc + 1] * Txx[dr][dc] + Fv[dr + 1][dc + 1] * Txy[dr][dc];
-    };
-    auto tvy = [&](int dr, int dc) {
-      return Fu[dr + 1][dc + 1] * Txy[dr][dc] + Fv[dr + 1][dc + 1] * Tyy[dr][dc];
-    };
-    va.src[2 * g.FS + ix] =
-        div_faces(g, i, tvx(r, c - 1), tvx(r, c), tvx(r, c + 1), tvy(r - 1, c), tvy(r, c), tvy(r + 1, c));
-  }
-}
-
-// viscous 1/dt of one cell (sources_viscosity.f90:507-577, the 2-D x-y
-// branch): (max(a+, -a-) + 2 nu/dl)/dl summed over both directions, the wave
-// speeds of CalcTimestep, nu = eta/rho
-__device__ __forceinline__ double visc_invdt(const Geom &g, int i, double rho, double u, double v, double cs,
-                                             double eta) {
-  const double mnx = fmin2(0.0, u - cs), mxx = fmax2(0.0, u + cs);
-  const double mny = fmin2(0.0, v - cs), mxy = fmax2(0.0, v + cs);
-  const double kin = eta / rho, dlx = ring(g, R_DLX, i), dly = ring(g, R_DLY, i);
-  return (fmax2(mxx, -mnx) + 2 * kin / dlx) / dlx + (fmax2(mxy, -mny) + 2 * kin / dly) / dly;
-}
-
-// Viscous source of one RHS evaluation (sources_viscosity.f90:481-500;
-// physics_eulerisotherm.f90:982-1072, physics_euler.f90:1887-1918), FP64:
-// ExternalSources sees Timedisc%pvar after CenterBoundary and the PMIN clamp,
-// in the real frame.  Tiles of VT_X x VT_Y cells cover the whole
-// ghost-inclusive mesh, one thread per cell; LDS holds
-//   density and velocities on the tile and a two-cell halo,
-//   the dynamic viscosity and the stresses on the tile and a one-cell halo
-// (the reference forms the stresses on every cell but the outermost ghost
-// layer, and the divergence reads them one cell around each interior cell).
-// Three phases: pvar (and, with an ALPHA update, the dynamic viscosity of
-// every own cell into va.dyn), stresses, divergence into va.src.
-constexpr int VT_X = 64, VT_Y = 8;
-#ifndef FV_VISC_WAVES_PER_SIMD
-#define FV_VISC_WAVES_PER_SIMD 1
-#endif
-template <int V, int KM>
-__global__ __launch_bounds__(VT_X *VT_Y, FV_VISC_WAVES_PER_SIMD) void k_visc(Geom g, StageArgs a, VisArgs va) {
-  constexpr int SX = VT_X + 4, SY = VT_Y + 4, RX = VT_X + 2, RY = VT_Y + 2, NT = VT_X * VT_Y;
-  __shared__ double Fr[SY][SX], Fu[SY][SX], Fv[SY][SX];  // rho, vx, vy; [r + 2][c + 2]
-  __shared__ double Dy[RY][RX], Txx[RY][RX], Tyy[RY][RX], Txy[RY][RX];  // [r + 1][c + 1]
-  __shared__ double Pown[V == 4 ? VT_Y : 1][V == 4 ? VT_X : 1];  // Euler: pressure of the own cells
-  __shared__ double red[VT_X * VT_Y / 64];
-  if (a.ctl && a.ctl->halt) return;
-  const In<double, V, KM> in(g, a, false, a.ctl ? a.ctl->dt : a.dt);  // device-controlled: this step's dt
-  const int tx = threadIdx.x, ty = threadIdx.y, t = tx + VT_X * ty;
-  const int i0 = blockIdx.x * VT_X, j0 = blockIdx.y * VT_Y;
-  const int imin = GH, imax = GH + g.inum - 1, jmin = GH, jmax = GH + g.jnum - 1;
-  const bool alpha = va.model == VIS_ALPHA || va.model == VIS_BETA;  // viscosity from the local rotation
-  const bool euler_cs = V == 4 && va.model == VIS_ALPHA;               // Physics%bccsound of Euler physics
-  // UpdateViscosity's time test (sources_viscosity.f90:371): decided by the
-  // host, or here from the step's time and dt in device-controlled steps
-  bool update = va.update;
-  if (a.ctl) {
-    const double tc = a.ctl->time + va.c_cur * a.ctl->dt, tp = a.ctl->time + va.c_prev * a.ctl->dt;
-    update = tc != tp || tc == 0.0;
-  }
-
-  // ---- phase 1: pvar of the footprint; dynamic viscosity of the inner
-  // region.  At most two footprint cells per thread: every load of both
-  // (state, stage slopes, stored viscosity) is issued before any arithmetic.
-  static_assert(SX * SY <= 2 * NT, "two footprint cells per thread");
-  int fr[2], fc[2], fi[2], fj[2];
-  bool inm[2], inr[2], inreg[2];
-#pragma unroll
-  for (int h = 0; h < 2; h++) {
-    const int q = t + h * NT;
-    fr[h] = q / SX - 2;
-    fc[h] = q % SX - 2;
-    fi[h] = i0 + fc[h];
-    fj[h] = j0 + fr[h];
-    inm[h] = q < SX * SY && fi[h] >= 0 && fi[h] < g.NI && fj[h] >= 0 && fj[h] < g.NJ;
-    inr[h] = inm[h] && fi[h] >= imin && fi[h] <= imax && fj[h] >= jmin && fj[h] <= jmax;
-    inreg[h] = inm[h] && fr[h] >= -1 && fr[h] <= VT_Y && fc[h] >= -1 && fc[h] <= VT_X;
-  }
-  double dst[2] = {va.dynconst, va.dynconst};
-  if (alpha && !update) {
-#pragma unroll
-    for (int h = 0; h < 2; h++)
-      if (inreg[h]) dst[h] = va.dyn[cidx(g, fi[h], fj[h])];
-  }
-  double s[2][V];
-  in.interior2(inr[0], fi[0], fj[0], s[0], inr[1], fi[1], fj[1], s[1]);
-#pragma unroll
-  for (int h = 0; h < 2; h++) {
-    if (!inm[h]) continue;
-    const int r = fr[h], c = fc[h], ii = fi[h], jj = fj[h];
-    double p[V];
-    if (inr[h]) {
-      double ur[V], uc[V];
-      in.transform(ii, s[h], ur, p, uc);
-    } else {
-      in.ghost_prim(ii, jj, p);
-      if (V == 4 && a.pmin_clamp) p[3] = fmax2(p[3], g.pmin);
-    }
-    Fr[r + 2][c + 2] = p[0];
-    Fu[r + 2][c + 2] = p[1];
-    Fv[r + 2][c + 2] = p[2];
-    const bool own = r >= 0 && r < VT_Y && c >= 0 && c < VT_X;
-    if constexpr (V == 4) {
-      if (va.part && own) Pown[r][c] = p[3];
-      if (euler_cs && a.nk == 0 && own) va.cs_out[cidx(g, ii, jj)] = sound_speed(g.gamma, p[0], p[3]);
-    }
-    if (inreg[h]) {
-      double d = dst[h];
-      if (alpha && update) {
-        const long ix = cidx(g, ii, jj);
-        double cs = 0.0;  // (BETA does not use it)
-        if constexpr (V == 4) {
-          if (euler_cs) cs = a.nk == 0 ? sound_speed(g.gamma, p[0], p[3]) : va.cs_in[ix];
-        } else {
-          cs = ring(g, R_CS, ii);
-        }
-        d = alpha_dynvis(va, ix, g.FS, p[0], p[1], p[2], cs);
-        if (r >= 0 && r < VT_Y && c >= 0 && c < VT_X) va.dyn[ix] = d;
-      }
-      Dy[r + 1][c + 1] = d;
-    }
-  }
-  __syncthreads();
-
-  // ---- phase 2: stresses (physics_eulerisotherm.f90:1017-1072, 2-D x-y) on
-  // the inner region's cells that are not in the outermost ghost layer
-#pragma unroll
-  for (int q0 = 0; q0 < RX * RY; q0 += NT) {
-    const int q = q0 + t;
-    if (q >= RX * RY) break;
-    const int r = q / RX - 1, c = q % RX - 1, ii = i0 + c, jj = j0 + r;
-    if (ii < 1 || ii > g.NI - 2 || jj < 1 || jj > g.NJ - 2) continue;
-    const int fr = r + 2, fc = c + 2;
-    const double u0 = Fu[fr][fc], v0 = Fv[fr][fc];
-    const double uw = Fu[fr][fc - 1], ue = Fu[fr][fc + 1], us = Fu[fr - 1][fc], un = Fu[fr + 1][fc];
-    const double vw = Fv[fr][fc - 1], ve = Fv[fr][fc + 1], vs = Fv[fr - 1][fc], vn = Fv[fr + 1][fc];
-    const double eta = Dy[r + 1][c + 1];
-    const double bulk = alpha ? -(2. / 3.) * eta : va.bulkconst;
-    const double dlx = ring(g, R_DLX, ii), dly = ring(g, R_DLY, ii);
-    const double cxyx = ring(g, R_CXYX, ii), cyxy = ring(g, R_CYXY, ii);
-    const double dv = bulk * div_faces(g, ii, uw, u0, ue, vs, v0, vn);
-    Txx[r + 1][c + 1] = eta * ((ue - uw) / dlx + 2.0 * cxyx * v0) + dv;
-    Tyy[r + 1][c + 1] = eta * ((vn - vs) / dly + 2.0 * cyxy * u0) + dv;
-    Txy[r + 1][c + 1] = eta * (0.5 * ((ve - vw) / dlx + (un - us) / dly) - cxyx * u0 - cyxy * v0);
-  }
-  __syncthreads();
-
-  // ---- phase 3: tensor divergence (mesh_midpoint.f90:279-335, btyx = btxy)
-  // and, for Euler, the divergence of T.v (physics_euler.f90:1887-1918)
-  const int i = i0 + tx, j = j0 + ty;
-  if (i >= imin && i <= imax && j >= jmin && j <= jmax)
-    visc_divergence<V, SX, RX>(g, va, i, j, ty + 1, tx + 1, Fu, Fv, Txx, Tyy, Txy);
-  if (!va.part) return;
-  // the viscous limit of this evaluation's pvar on the own cell, every cell of
-  // the mesh (as k_visc_cfl on Timedisc%pvar: comoving velocities under FARGO)
-  double m = -DBL_MAX;
-  if (i < g.NI && j < g.NJ) {
-    const double rho = Fr[ty + 2][tx + 2], u = Fu[ty + 2][tx + 2];
-    const double v = a.sub_bg ? Fv[ty + 2][tx + 2] - ring(g, R_W, i) : Fv[ty + 2][tx + 2];
-    double cs;
-    if constexpr (V == 4)
-      cs = sound_speed(g.gamma, rho, Pown[ty][tx]);
-    else
-      cs = ring(g, R_CS, i);
-    m = visc_invdt(g, i, rho, u, v, cs, Dy[ty + 1][tx + 1]);
-  }
-  m = blk_max(m, red);
-  if (t == 0) {
-    const int b = blockIdx.x + blockIdx.y * gridDim.x;
-    va.part[2 * b] = m;
-    va.part[2 * b + 1] = 0.0;
-  }
-}
-
-// Viscous time-step limit (sources_viscosity.f90:507-577, the 2-D x-y
-// branch) on the stored pvar pv of the last evaluation, all cells:
-// (max(a+, -a-) + 2 nu/dl)/dl summed over the directions, nu = eta/rho, with
-// the wave speeds CalcTimestep uses (v + w when add_w).  va.update: the
-// dynamic viscosity from pv itself (UpdateViscosity at the same time 0).
-template <int V>
-__global__ __launch_bounds__(256) void k_visc_cfl(Geom g, VisArgs va, const double *__restrict__ pv, int add_w,
-                                                  double *part) {
-  __shared__ double red[4];
-  double m = -DBL_MAX;
-  const long n = (long)g.NI * g.NJ;
-  for (long k = (long)blockIdx.x * 256 + threadIdx.x; k < n; k += (long)gridDim.x * 256) {
-    const int i = (int)(k % g.NI), j = (int)(k / g.NI);
-    const long ix = cidx(g, i, j);
-    const double rho = pv[ix], u = pv[g.FS + ix];
-    double v = pv[2 * g.FS + ix];
-    if (add_w) v = v + ring(g, R_W, i);
-    const double cs = (V == 4) ? sound_speed(g.gamma, rho, pv[3 * g.FS + ix]) : ring(g, R_CS, i);
-    double d = va.dynconst;
-    if (va.model == VIS_ALPHA || va.model == VIS_BETA)
-      d = va.update ? alpha_dynvis(va, ix, g.FS, rho, u, v, cs) : va.dyn[ix];
-    m = fmax2(m, visc_invdt(g, i, rho, u, v, cs, d));
-  }
-  m = blk_max(m, red);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = m;
-    part[2 * blockIdx.x + 1] = 0.0;
-  }
-}
-
 // typed launchers, explicitly instantiated in fv_inst_*.hip (one translation
 // unit per element type and kernel family, compiled in parallel)
 template <typename T, int V>
@@ -1733,9 +1388,6 @@ void frame_single(const Geom &g, const void *src, void *dst, int sign, int V, co
 template <typename T, int V>
 void rhs_multi(const RhsEntry *tab, const unsigned *tiles, int n, int limiter, int rows, int mode, int nk,
                hipStream_t s);
-// coefficient slots k_visc is compiled for, by tableau size
-constexpr int KM_SMALL = 3;
-inline int km_for(int stages) { return stages <= KM_SMALL ? KM_SMALL : MAXK; }
 template <typename T>
 void remap_multi(const RemapEntry *tab, const unsigned *tiles, int n, int V, hipStream_t s);
 

@@ -4,7 +4,7 @@
 #include <cstring>
 #include <mutex>
 
-#include "fv_kernels.h"
+#include "fv_visc.h"
 
 namespace fv {
 
@@ -172,15 +172,23 @@ void launch_cfl_pvar(const Geom &g, const void *pv, int add_w, double *part, int
   }
 }
 
+// (NK: the slopes in the launch's stage sum)
+template <int NK>
+static void visc_slopes(const Geom &g, const StageArgs &a, const VisArgs &v, int V, dim3 grid, dim3 block,
+                        hipStream_t s) {
+  if (V == 3) hipLaunchKernelGGL((k_visc<3, NK>), grid, block, 0, s, g, a, v);
+  else hipLaunchKernelGGL((k_visc<4, NK>), grid, block, 0, s, g, a, v);
+}
 void launch_visc(const Geom &g, const StageArgs &a, const VisArgs &v, int V, hipStream_t s) {
-  const dim3 grid((g.NI + VT_X - 1) / VT_X, (g.NJ + VT_Y - 1) / VT_Y), block(VT_X, VT_Y);
-  const bool small = km_for(g.stages) == KM_SMALL;
-  if (V == 3) {
-    if (small) hipLaunchKernelGGL((k_visc<3, KM_SMALL>), grid, block, 0, s, g, a, v);
-    else hipLaunchKernelGGL((k_visc<3, MAXK>), grid, block, 0, s, g, a, v);
-  } else {
-    if (small) hipLaunchKernelGGL((k_visc<4, KM_SMALL>), grid, block, 0, s, g, a, v);
-    else hipLaunchKernelGGL((k_visc<4, MAXK>), grid, block, 0, s, g, a, v);
+  const dim3 grid(visc_blocks(g.NI, g.NJ)), block(64 * VWAVES);
+  switch (a.nk) {
+    case 0: visc_slopes<0>(g, a, v, V, grid, block, s); break;
+    case 1: visc_slopes<1>(g, a, v, V, grid, block, s); break;
+    case 2: visc_slopes<2>(g, a, v, V, grid, block, s); break;
+    case 3: visc_slopes<3>(g, a, v, V, grid, block, s); break;
+    case 4: visc_slopes<4>(g, a, v, V, grid, block, s); break;
+    case 5: visc_slopes<5>(g, a, v, V, grid, block, s); break;
+    default: visc_slopes<6>(g, a, v, V, grid, block, s); break;
   }
 }
 void launch_visc_cfl(const Geom &g, const VisArgs &v, const double *pv, int add_w, double *part, int nblocks, int V,
@@ -343,7 +351,6 @@ void launch_control(const CtlHead *prev, Ctl *ctl, const double *part_c, const d
                     const double *part_v, int nbv) {
   hipLaunchKernelGGL(k_control, dim3(1), dim3(256), 0, s, prev, ctl, part_c, part_r, nb, part_v, nbv);
 }
-int visc_blocks(const Geom &g) { return ((g.NI + VT_X - 1) / VT_X) * ((g.NJ + VT_Y - 1) / VT_Y); }
 void launch_rhs_multi(const RhsEntry *tab, const unsigned *tiles, int ntiles, int V, int dtype, int limiter,
                       int rows, int mode, int nk, hipStream_t s) {
   if (dtype == 1) {
