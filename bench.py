@@ -38,21 +38,21 @@ KERNEL_NAMES = {
     "rhs": "fv::k_rhs<double,3,VANLEER,1,M_STAGE>: stage 2 (stage sum over k_1, ghost cells, RHS)",
     "rhs_combine": "fv::k_rhs<double,3,VANLEER,2,M_LAST>: stage 3 with the final combination and "
                    "embedded error",
-    "rhs_end": "fv::k_rhs<double,3,VANLEER,0,M_END>: end-of-step RHS (CFL, data checks, new state)",
-    "remap": "fv::k_remap<double,3>: FARGO azimuthal remap",
+    "rhs_end": "fv::k_rhs<double,3,VANLEER,0,M_REMAP>: end-of-step RHS on the FARGO remap (CFL, data "
+               "checks, new state)",
 }
 METRIC = "cell-updates/s & HBM GB/s vs plain FP64 at stated err; p50/p99 run latency"
 
 
-def b_alg(V=3, w=8, s=3, fargo=True):
+def b_alg(V=3, w=8, s=3):
     """Algorithmic HBM bytes per cell-update of one s-stage step as this
     implementation moves them: stage m (2..s-1) reads the state and m-1 stage
     slopes and writes one slope (m+1 words); the last stage also forms the
     final combination, reading the state and s-1 slopes and writing the new
-    state (s+1); the FARGO remap reads and writes the state (2); the
-    end-of-step RHS reads it and writes the first slope of the next step and
-    the stored state (3).  w bytes per word, V conserved fields."""
-    return w * V * (sum(m + 1 for m in range(2, s)) + (s + 1) + (2 if fargo else 0) + 3)
+    state (s+1); the end-of-step RHS reads it (through the FARGO remap) and
+    writes the first slope of the next step and the stored state (3).  w bytes
+    per word, V conserved fields."""
+    return w * V * (sum(m + 1 for m in range(2, s)) + (s + 1) + 3)
 
 
 def cpu_model():
@@ -483,7 +483,7 @@ def main():
     # launch bracketed by HIP events on the simulation's stream
     sim.profile(True)
     sim.run(a.profile_steps)
-    stats = {k: sim.kernel_stats(k) for k in ("rhs", "rhs_combine", "rhs_end", "remap", "control")}
+    stats = {k: sim.kernel_stats(k) for k in ("rhs", "rhs_combine", "rhs_end", "control")}
     sim.profile(False)
     kernels = {k: {"launches": n, "mean_launch_us": 1e3 * t / max(n, 1),
                    "alg_bytes_per_launch": b / max(n, 1),
