@@ -58,8 +58,8 @@ __device__ __forceinline__ double visc_invdt(double dlx, double dly, double rho,
 // every cell but the outermost ghost layer), and the divergence of the row
 // below that (mesh_midpoint.f90:279-335, btyx = btxy), into va.src.  Neighbours
 // along x come through DPP, along y from registers: no LDS, no barrier but the
-// final reduction's.  Bound by VALU issue and by the latency of the march's
-// loads (issued one row ahead).  Tiles of 64 x 8 cells with three phases in LDS
+// final reduction's.  Bound by the latency of the march's loads
+// (issued one row ahead; 40% of a wave's life) and by VALU issue (28%).  Tiles of 64 x 8 cells with three phases in LDS
 // before: 41 KB each, so three tiles per CU and a second, half empty round at
 // 512x1024, and up to six dependent evaluations per ghost cell.
 // us per launch at 512x1024 (ALPHA, isothermal; stage, last stage, end of step),
