@@ -73,19 +73,23 @@ __device__ __forceinline__ float mx(float a, float b) { return __builtin_fmaxf(a
 // The FP64 quotient dv is Newton's iteration on the hardware reciprocal with
 // Markstein's final correction (P. Markstein, IBM J. Res. Dev. 34, 1990): a/b
 // rounds as IEEE division does while the operands, the quotient and the
-// residual a - b*q (2^-53 of a) stay in the normal range.  It leaves out the
-// rescaling of extreme exponents and the special-case fix-up (3 of 11
-// instructions, 12 of about 56 issue cycles); an infinite or zero divisor
-// gives NaN where IEEE gives 0 or Inf, both of which the data checks and the
-// error norm treat alike.  Densities, pressures, sound speeds and wave speeds
-// take it; quotients of differences, which do reach the subnormal range ahead
-// of a signal, take dvx or the guarded forms below.
+// residual a - b*q (2^-53 of a) stay in the normal range, and the last
+// instruction gives IEEE's results for operands that are zero, infinite or NaN.
+// It leaves out the rescaling of extreme exponents: a quotient that overflows
+// comes out as NaN where IEEE gives Inf.  Both fail CheckData and make a flux
+// NaN, but a maximum or minimum drops NaN: kt_core and cell_invdt, whose
+// quotients go there, take care of it.  Densities, pressures, sound speeds and
+// wave speeds take dv; quotients of differences, which do reach the subnormal
+// range ahead of a signal, take dvx or the guarded forms below.  us per step,
+// IEEE operations everywhere -> with dv, sq and these guards: 256x256 Riemann
+// problem 38.2 -> 36.6, 251x333 Euler box with five stages 96.5 -> 94.3,
+// 1024x2048 Euler disk with seven 902 -> 880.
 __device__ __forceinline__ double dv(double a, double b) {
   double y = __builtin_amdgcn_rcp(b);
   y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
   y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
   const double q = a * y;
-  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), y, q), b, a);
 }
 __device__ __forceinline__ float dv(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
 __device__ __forceinline__ double dvx(double a, double b) { return a / b; }
@@ -102,6 +106,8 @@ __device__ __forceinline__ double sq(double a) {
   return __builtin_fma(__builtin_fma(-s, s, a), h, s);
 }
 __device__ __forceinline__ float sq(float a) { return __builtin_amdgcn_sqrtf(a); }
+__device__ __forceinline__ double sqx(double a) { return sqrt(a); }
+__device__ __forceinline__ float sqx(float a) { return sq(a); }
 __device__ __forceinline__ double lg(double a) { return log(a); }
 __device__ __forceinline__ float lg(float a) { return __logf(a); }
 __device__ __forceinline__ double ex(double a) { return exp(a); }
@@ -166,16 +172,21 @@ __device__ __forceinline__ void p2c(const T *p, T *u, T gamma) {
   u[2] = p[0] * p[2];
   if (V == 4) u[3] = dv(p[3], gamma - T(1)) + T(0.5) * p[0] * (p[1] * p[1] + p[2] * p[2]);
 }
-// SQRT(MAX(2*TINY, gamma*P/rho)) (physics_euler.f90:2682-2689); FP64: the
-// floor's square root is a constant
+// SQRT(MAX(2*TINY, gamma*P/rho)) (physics_euler.f90:2682-2689)
 template <typename T>
 __device__ __forceinline__ T sound_speed(T gamma, T rho, T pr) {
-  const T x = dv(gamma * pr, rho);
+  return sqx(fmax2(T(2) * Real<T>::tiny, dvx(gamma * pr, rho)));
+}
+// The same at a face, FP64: the floor's square root is a constant, and NaN
+// stands for Inf (a zero density, an overflow; the first factor of the
+// condition keeps the floor for a pressure that is NaN or not positive)
+template <typename T>
+__device__ __forceinline__ T face_sound_speed(T gamma, T rho, T pr) {
   if constexpr (sizeof(T) == 8) {
-    const T s = sq(x);
-    return x > T(2) * Real<T>::tiny ? s : T(0x1.6a09e667f3bcdp-511);
+    const T y = gamma * pr, x = dv(y, rho), s = sq(x);
+    return (y > T(0)) & !(x <= T(2) * Real<T>::tiny) ? s : T(0x1.6a09e667f3bcdp-511);
   } else {
-    return sq(fmax2(T(2) * Real<T>::tiny, x));
+    return sound_speed(gamma, rho, pr);
   }
 }
 
@@ -614,7 +625,10 @@ template <typename T>
 __device__ __forceinline__ T cell_invdt(T dlx, T dly, T u, T v, T cs) {
   const T mnx = mn(T(0), u - cs), mxx = mx(T(0), u + cs);
   const T mny = mn(T(0), v - cs), mxy = mx(T(0), v + cs);
-  return dv(mx(mxx, -mnx), dlx) + dv(mx(mxy, -mny), dly);
+  const T x = dv(mx(mxx, -mnx), dlx) + dv(mx(mxy, -mny), dly);
+  // (both numerators are numbers or Inf: a NaN is an overflow, which the
+  // maximum over the cells would drop)
+  return x == x ? x : T(__builtin_huge_val());
 }
 template <typename T>
 __device__ __forceinline__ T cell_invdt(const Geom &g, int i, T u, T v, T cs) {
@@ -798,8 +812,8 @@ __device__ __forceinline__ void kt_core(const Geom &g, int d, const T *UL, const
   const int un = 1 + d, ut = 2 - d;
   const T gam = (T)g.gamma, zero = T(0);
   if (V == 4) {
-    csL = sound_speed(gam, pl[0], pl[3]);
-    csR = sound_speed(gam, pr[0], pr[3]);
+    csL = face_sound_speed(gam, pl[0], pl[3]);
+    csR = face_sound_speed(gam, pr[0], pr[3]);
   }
   const T vL = pl[un], vR = pr[un];
   const T amin = mn(mn(zero, vR - csR), vL - csL);
@@ -818,7 +832,11 @@ __device__ __forceinline__ void kt_core(const Geom &g, int d, const T *UL, const
   }
   fL[ut] = UL[ut] * vL;
   fR[ut] = UR[ut] * vR;
-  const T fac = dv(dA, amax - amin);
+  T dif = amax - amin;
+  // a face_sound_speed of NaN, which the wave speeds drop, makes the flux NaN,
+  // as the Inf in its place does (fac = 0 against Inf in the bracket)
+  if constexpr (V == 4 && sizeof(T) == 8) dif = __builtin_fma(0.0, csL + csR, dif);
+  const T fac = dv(dA, dif);
 #pragma unroll
   for (int l = 0; l < V; l++) F[l] = fac * (amax * fL[l] - amin * fR[l] + amin * amax * (UR[l] - UL[l]));
 }
@@ -1183,10 +1201,7 @@ struct SourceRing {
     // (physics_euler.f90:2368-2400, elemental physics_eulerisotherm.f90:
     // 3080-3088), with the real-frame velocities
     if (g.fargo) {
-      // FP64: the numerator scaled up, so that the quotient of a tiny radial
-      // momentum rounds as IEEE division does
-      const T m = ur[1] * T(0.5) * dw;
-      T tmp = sizeof(T) == 8 ? dv(m * T(0x1p200), dlx) * T(0x1p-200) : dv(m, dlx);
+      T tmp = dvx(ur[1] * T(0.5) * dw, dlx);
       geo[2] = geo[2] - tmp;
       if constexpr (V == 4) {
         tmp = tmp + ur[1] * -(cyxy * pr[2]);
