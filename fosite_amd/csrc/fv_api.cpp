@@ -591,8 +591,7 @@ bool pvar_moved_to_real_frame(const fv_ctx *ctx) {
   return ctx->c.fargo && ctx->pvalid && ctx->pflag && !ctx->fl_pvar;
 }
 int cfl_real_frame(fv_ctx *ctx) {
-  const long cells = (long)ctx->NI * ctx->NJ;
-  const int nb = (int)std::min<long>(ctx->nb_rhs, (cells + 255) / 256);
+  const int nb = cell_blocks(ctx->c.inum, ctx->c.jnum);
   launch_cfl_pvar(ctx->g, ctx->pbuf, 1, ctx->part_r, nb, ctx->V, ctx->st);
   HIPCHK(hipGetLastError());
   int f = 0;
@@ -611,8 +610,7 @@ int timestep(fv_ctx *ctx) {
   if (ctx->pvalid) {
     const int update = ctx->c.vismodel >= VIS_ALPHA && (ctx->time != ctx->vis_time || ctx->time == 0.0);
     ctx->vis_time = ctx->time;
-    const long cells = (long)ctx->NI * ctx->NJ;
-    const int nb = (int)std::min<long>(ctx->nb_rhs, (cells + 255) / 256);
+    const int nb = cell_blocks(ctx->c.inum, ctx->c.jnum);
     launch_visc_cfl(ctx->g, vis_args(ctx, update), ctx->pbuf, pvar_moved_to_real_frame(ctx) ? 1 : 0, ctx->part_r,
                     nb, ctx->V, ctx->st);
     HIPCHK(hipGetLastError());
@@ -1564,7 +1562,7 @@ extern "C" int fv_step(fv_ctx *ctx, int *done) {
 extern "C" int fv_step_noalloc(fv_ctx *ctx, int *done) {
   if (!ctx) return -1;
   if (ctx->prof) return fail(ctx, "fv_step_noalloc: kernel profiling (fv_profile) creates events; disable it");
-  const long tiles = (long)strip_cols(ctx->c.inum) * ((ctx->c.jnum + 7) / 8);  // of 64 x 8 cells
+  const int tiles = tile_blocks(ctx->c.inum, ctx->c.jnum);  // of 64 x 8 cells; cell_blocks is no more
   if (tiles > SCRATCH_MAX_BLOCKS || ctx->nb_rhs + 1 > SCRATCH_MAX_BLOCKS)
     return fail(ctx, "fv_step_noalloc: " + std::to_string(tiles) + " tiles of 64 x 8 cells exceed the " +
                          std::to_string(SCRATCH_MAX_BLOCKS) + " the static scratch holds (use fv_step)");

@@ -306,6 +306,17 @@ __host__ __device__ inline int strip_cols(int inum) { return (inum + 63) / 64; }
 __host__ __device__ inline int strip_blocks(int jnum, int rows) {
   return (jnum + rows * STRIP_WAVES - 1) / (rows * STRIP_WAVES);
 }
+// workgroups of the time-step kernels on a stored pvar (k_cfl_pvar, k_visc_cfl:
+// 256 threads over all cells, one partial each): two cells a thread on large
+// meshes, whatever the height of k_rhs's strips.  us per launch with one
+// workgroup per workgroup of k_rhs (256, 512) -> this (1024, 4096):
+//   512x1024   k_visc_cfl 10.6 -> 7.7, k_cfl_pvar 8.3 -> 5.5
+//   1024x2048  k_visc_cfl 22.4 -> 18.2, k_cfl_pvar 16.2 -> 12.7
+__host__ __device__ inline int tile_blocks(int inum, int jnum) { return strip_cols(inum) * ((jnum + 7) / 8); }
+__host__ __device__ inline int cell_blocks(int inum, int jnum) {
+  const long n = ((long)(inum + 2 * GH) * (jnum + 2 * GH) + 255) / 256, t = tile_blocks(inum, jnum);
+  return (int)(n < t ? n : t);
+}
 // auxiliary workgroups of an end-of-step launch: the corner ghost cells, and with the boundary-flux
 // accumulation up to 64 more
 __host__ __device__ inline int rhs_aux_max(const Geom &g, int V) {
