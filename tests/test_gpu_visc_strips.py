@@ -48,3 +48,15 @@ def test_gpu_visc_tall_strips_molecular():
     for n, cv, sc, rc, rs in run_pair(cfg, 1):
         assert sc["time"] == rs["time"] and sc["dt"] == rs["dt"], (n, sc, rs)
         assert np.array_equal(cv[:, 2:-2, 2:-2], rc[:, 2:-2, 2:-2], equal_nan=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("vismodel", [2, 3])
+def test_gpu_visc_tall_strips_rotation(vismodel):
+    """The same with a viscosity from the local rotation (ALPHA, BETA): e_phi/r
+    at 32989 angles."""
+    print("viscous tall strips", vismodel, flush=True)
+    cfg = dict(PROBLEMS["disk_alpha_fargo_nograd"](8, 32989), vismodel=vismodel)
+    for n, cv, sc, rc, rs in run_pair(cfg, 1):
+        assert sc["time"] == rs["time"] and sc["dt"] == rs["dt"], (n, sc, rs)
+        assert np.array_equal(cv[:, 2:-2, 2:-2], rc[:, 2:-2, 2:-2], equal_nan=True)
