@@ -131,7 +131,7 @@ def main():
     ap.add_argument("-j", type=int, default=8)
     ap.add_argument("--drivers-only", action="store_true")
     a = ap.parse_args()
-    if not os.path.isdir(a.ref):
+    if not os.path.isfile(os.path.join(a.ref, "fosite.f90")):
         print("reference checkout not found at %s; nothing to build" % a.ref)
         return 0
     objdir = os.path.join(OUT, "obj")
