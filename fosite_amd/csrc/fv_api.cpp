@@ -1219,7 +1219,6 @@ extern "C" int fv_create(fv_ctx **out, const fv_config *cfg) {
   g.rotframe = c.rotframe;
   g.twoomega = 2 * c.omega;
   g.dtype = c.dtype;
-  g.stages = ctx->tab.m;
   g.rows = strip_rows((long)strip_cols(c.inum) * c.jnum, c.dtype);
   // FV_RHS_TILE=32: strips of half the rows
   if (const char *e = std::getenv("FV_RHS_TILE")) g.rows = std::atoi(e) == 32 ? std::max(1, g.rows / 2) : g.rows;

@@ -40,7 +40,6 @@ struct Geom {
   int rotframe;         // rotating-frame source: 0 off, 1 centrifugal + Coriolis, 2 Coriolis only
   double twoomega;      // 2*Omega (sources_rotframe.f90:162); centrifugal terms in R_CACX, C_CACY
   int rows;             // k_rhs: rows of a wave's strip (1 .. STRIP_ROWS)
-  int stages;           // RK stages of the tableau (picks the kernels' coefficient slots)
   int dtype;            // stored state: 0 FP64 (plain drop-in), 1 FP32 (precision form)
   const double *ring;   // [R_COUNT][NI]
   const double *col;    // [C_COUNT][NJ]

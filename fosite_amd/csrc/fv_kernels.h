@@ -131,8 +131,6 @@ struct Acc {
     hi = s;
     lo = lo + (e - pe - cl * k);
   }
-  __device__ __forceinline__ float value() const { return hi + lo; }
-  __device__ __forceinline__ double wide() const { return (double)hi + (double)lo; }
 };
 
 // per-ring and per-column metric arrays: uniform base per id, 32-bit lane
@@ -461,29 +459,25 @@ __device__ __forceinline__ void ycell(const Geom &g, const T *Y, int i, int jj, 
 }
 
 // ------------------------------------------------------------ input state
-// KM: coefficient slots of the tableau (3 for up to three stages, else MAXK);
-// loops over stages are unrolled to KM with run-time guards on nk, or with
-// EXACT over exactly KM slopes
+// NK: the slopes in the launch's stage sum
 // RM: the state is the FARGO remap of Y (no stage sum)
-template <typename T, int V, int KM, bool EXACT = false, bool RM = false>
+template <typename T, int V, int NK, bool RM = false>
 struct In {
   const Geom &g;
   const StageArgsT<T> &a;
   double dt;
   T gam;
-  int nk;
   bool chk;  // CheckData on the ghost cells
-  // stage coefficients a(m,q)*dt, formed once (KM = 0: no stage sum)
-  static constexpr int KA = KM > 0 ? KM : 1;
+  // stage coefficients a(m,q)*dt, formed once
+  static constexpr int KA = NK > 0 ? NK : 1;
   double c[sizeof(T) == 8 ? KA : 1];
   float ch[sizeof(T) == 4 ? KA : 1];
 
   __forceinline__ __device__ In(const Geom &g_, const StageArgsT<T> &a_, bool chk_, double dt_)
       : g(g_), a(a_), dt(dt_), chk(chk_) {
-    nk = EXACT ? KM : a.nk;
     gam = (T)g.gamma;
 #pragma unroll
-    for (int q = 0; q < KM; q++) {
+    for (int q = 0; q < NK; q++) {
       const double cq = a.a[q] * dt;
       if constexpr (sizeof(T) == 8)
         c[q] = cq;
@@ -495,35 +489,29 @@ struct In {
   // s = Y - sum_q (a_q*dt) k_q for one cell from loaded values, in the
   // reference's order (FP64) or with FP32 fused multiply-adds.
   __forceinline__ __device__ void stage_sum(const T *y, const T (*kv)[V], T *s) const {
-    if constexpr (KM == 0) {
-#pragma unroll
-      for (int l = 0; l < V; l++) s[l] = y[l];
-      return;
-    }
     if constexpr (sizeof(T) == 8) {
 #pragma unroll
       for (int l = 0; l < V; l++) s[l] = y[l];
 #pragma unroll
-      for (int q = 0; q < KM; q++)
-        if (q < nk) {
+      for (int q = 0; q < NK; q++) {
 #pragma unroll
-          for (int l = 0; l < V; l++) s[l] = s[l] - c[q] * kv[q][l];
-        }
+        for (int l = 0; l < V; l++) s[l] = s[l] - c[q] * kv[q][l];
+      }
     } else {
       // the stage state only feeds an FP32 RHS evaluation: plain FP32 sums
 #pragma unroll
       for (int l = 0; l < V; l++) {
         float acc = (float)y[l];
 #pragma unroll
-        for (int q = 0; q < KM; q++)
-          if (q < nk) acc = fmaf(-ch[q], (float)kv[q][l], acc);
+        for (int q = 0; q < NK; q++) acc = fmaf(-ch[q], (float)kv[q][l], acc);
         s[l] = (T)acc;
       }
     }
   }
 
-  // input state at an interior cell
+  // input state of an end-of-step evaluation at an interior cell
   __forceinline__ __device__ void interior(int i, int j, T *s) const {
+    static_assert(NK == 0, "stage sums are formed from loaded rows");
     if constexpr (RM) {
       const RingShift<T> sh(g, ring(g, R_W, i), ring(g, R_DLY, i), StepTime(g, a.ctl, a.dt_step));
       const int js = GH + sh.source(j - GH, sh.m, g.jnum);
@@ -533,20 +521,11 @@ struct In {
 #pragma unroll
       for (int q = 0; q < 5; q++) ycell_ghost<T, V>(g, js - 2 + q, v[q]);
       fargo_row<T, V>(v, sh.d, s);
-      return;
+    } else {
+      const long ix = cidx(g, i, j);
+#pragma unroll
+      for (int l = 0; l < V; l++) s[l] = a.Y[l * g.FS + ix];
     }
-    const long ix = cidx(g, i, j);
-    // all loads first (uniform branches only), then the stage sum
-    T y[V], kv[KA][V];
-#pragma unroll
-    for (int l = 0; l < V; l++) y[l] = a.Y[l * g.FS + ix];
-#pragma unroll
-    for (int q = 0; q < KM; q++)
-      if (q < nk) {
-#pragma unroll
-        for (int l = 0; l < V; l++) kv[q][l] = a.k[q][l * g.FS + ix];
-      }
-    stage_sum(y, kv, s);
   }
 
   // ComputeRHS transform (timedisc_base.f90:1098-1208): ur = cvar after the

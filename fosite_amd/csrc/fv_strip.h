@@ -207,7 +207,7 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
     if (a.prev) open_step<T>(a, b, nb, csh, st.dt, st.halt);
   }
   if (st.halt) return {0.0, 0.0, 0, 1};
-  const In<T, V, NK, true> in(g, a, want_check, a.ctl ? st.dt : a.dt);
+  const In<T, V, NK> in(g, a, want_check, a.ctl ? st.dt : a.dt);
   // kRemap: the strip's columns (from two rows below its first) and the edge
   // lanes' cells, each marching along its ring
   const RingShift<T> sh(g, w_d, dly_d, st), esh(g, ew_d, edly_d, st);
@@ -606,7 +606,7 @@ __device__ __forceinline__ void rhs_aux_block(const Geom &g, const StageArgsT<T>
                  : bx == ABSORBING ? (cE ? imax - 1 + part : imin + part)
                                    : ir;
   const int sj = part < 2 ? jr : by == PERIODIC ? (cN ? jmin + gb - 1 : jmax - gb + 1) : jr;
-  const In<T, V, 0, true, RM> in(g, a, a.want_check, dt);
+  const In<T, V, 0, RM> in(g, a, a.want_check, dt);
   T u[V], p[V], px[V], pR[V], py[V];
   in.prim_interior(si, sj, px);
 #pragma unroll

@@ -78,7 +78,7 @@ __global__ __launch_bounds__(64 * VWAVES, 2) void k_visc(Geom g, StageArgs a, Vi
   double m = -DBL_MAX;
   if (a.ctl && a.ctl->halt) return;
   if (nr > 0) {
-    const In<double, V, NK, true> in(g, a, false, a.ctl ? a.ctl->dt : a.dt);  // device-controlled: this step's dt
+    const In<double, V, NK> in(g, a, false, a.ctl ? a.ctl->dt : a.dt);  // device-controlled: this step's dt
     const bool alpha = va.model == VIS_ALPHA || va.model == VIS_BETA;   // viscosity from the local rotation
     const bool euler_cs = V == 4 && va.model == VIS_ALPHA;              // Physics%bccsound of Euler physics
     // UpdateViscosity's time test (sources_viscosity.f90:371): decided by the
