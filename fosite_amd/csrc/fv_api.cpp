@@ -880,12 +880,17 @@ void visc_device(fv_ctx *ctx, const Geom &g, StageArgs &a, double c_cur, double 
 
 // Rounds whose first stages take the step control along (k_rhs open_step), with
 // one k_control behind the round: wherever the step begins with a first stage
-// (FARGO type 1 begins with k_wsum, viscous steps with k_visc), and the
-// workgroups, each of which reads all partials, are no more than the chip holds
-// at once (512 of 256 threads, two per CU).  us per step with k_control -> with
-// open_step: 64x128 disk 36.1 -> 35.2, 256x256 Riemann problem 37.9 -> 36.3,
-// 512x1024 disk 74.7 -> 74.1 (FP32 53.0 -> 51.9), 1024x2048 Euler disk with
-// seven stages (512 workgroups) 871 -> 860.
+// (FARGO type 1 begins with k_wsum, viscous steps with k_visc), up to 512
+// workgroups.  Every workgroup reads all partials and decides the step ahead of
+// its dt: while few rounds of workgroups follow each other on a CU that costs
+// less than the launch it saves, and the more partials and rounds there are, the
+// less is left.  us per step with k_control -> with open_step:
+//   64x128 disk 36.1 -> 35.2, 256x256 Riemann problem 37.9 -> 36.3
+//   512x1024 disk 74.7 -> 74.1 (FP32 53.0 -> 51.9)
+//   512 workgroups: 1024x2048 Euler disk with seven stages 871 -> 860
+//   768: the disk 1536x2048 282 -> 282, the Euler disk 1124 -> 1124
+//   1024: 2048x2048 Riemann problem 503.2 -> 503.6, FP32 disk 203 -> 205
+//   2048: 2048x4096 Euler disk 2963 -> 2968 (FP32 1718 -> 1722)
 constexpr int OPEN_STEP_BLOCKS = 512;
 bool own_control(const fv_ctx *ctx) {
   return ctx->c.fargo == 1 || ctx->c.vismodel || ctx->nb_rhs > OPEN_STEP_BLOCKS;
