@@ -1012,15 +1012,16 @@ int replay_device_steps(fv_ctx *ctx, const Ctl *h, int x0, int x1, int *halted) 
   return 0;
 }
 
-// a graph of nsteps (even) device-controlled steps
+// a graph of nsteps (even) device-controlled steps; without build: only if it is there
 int get_graph(fv_ctx *ctx, int x0, int x1, int tb, int rb, int k0, int b0, int g0, int w0, int v0, int nsteps,
-              hipGraphExec_t *out) {
+              bool build, hipGraphExec_t *out) {
   for (auto &e : ctx->graphs)
     if (e.x0 == x0 && e.x1 == x1 && e.t == tb && e.k0 == k0 && e.b0 == b0 && e.g0 == g0 && e.w0 == w0 &&
         e.v0 == v0 && e.nsteps == nsteps) {
       *out = e.exec;
       return 0;
     }
+  if (!build) return 0;
   hipGraph_t graph;
   HIPCHK(hipStreamBeginCapture(ctx->st, hipStreamCaptureModeThreadLocal));
   const int g1 = ctx->grav[0] ? 1 - g0 : g0, t1 = ctx->c.fargo == 1;
@@ -1063,22 +1064,33 @@ int run_batch(fv_ctx *ctx, int nmax, int *done_steps, int *halted) {
   const int w0 = ctx->wcur, v0 = ctx->vcur, t1 = ctx->c.fargo == 1;
   Ctl *h = ctx->h_ctl;
   prime_ctl(ctx, h, nmax, own_control(ctx));
-  // graphs of GRAPH_STEPS steps, the rest of the round in pairs of steps: a
-  // graph launch leaves the device idle for about 5 us (64x128 disk, us per step
-  // with graphs of 2, 4, 8, 16 steps: 40.5, 39.3, 38.6, 38.3)
+  // graphs of GRAPH_STEPS steps, the rest of the round ahead of them in pairs of
+  // steps: a graph launch leaves the device idle for about 5 us (64x128 disk, us
+  // per step with graphs of 2, 4, 8, 16 steps: 40.5, 39.3, 38.6, 38.3).  Where the
+  // long graph is yet to be built, another GRAPH_STEPS steps go in pairs, and it
+  // is built while the device works on them.  First round of a new state, us per
+  // step with the long graph built ahead of the round -> behind the pairs:
+  // 64x128 disk 48.6 -> 44.2 for 8 steps and 47.7 -> 42.6 for 10, 256x256 Riemann
+  // problem 48.3 -> 45.7 and 47.0 -> 43.9,
+  // 512x1024 disk 91.8 -> 89.0 for 10.
   constexpr int GRAPH_STEPS = 8;
   hipGraphExec_t exec = nullptr, pair = nullptr;
   const bool graphs = !ctx->prof && !eager_launches();
-  const int whole = nmax / GRAPH_STEPS;
+  int lead = nmax % GRAPH_STEPS;
+  auto graph = [&](int nsteps, hipGraphExec_t *out, bool build) {
+    return get_graph(ctx, x0, x1, tb, rb, k0, b0, g0, w0, v0, nsteps, build, out);
+  };
   if (graphs) {
-    int rc = whole ? get_graph(ctx, x0, x1, tb, rb, k0, b0, g0, w0, v0, GRAPH_STEPS, &exec) : 0;
-    if (!rc && nmax % GRAPH_STEPS) rc = get_graph(ctx, x0, x1, tb, rb, k0, b0, g0, w0, v0, 2, &pair);
-    if (rc) return rc;
+    graph(GRAPH_STEPS, &exec, false);
+    if (!exec) lead = std::min(nmax, lead + GRAPH_STEPS);
+    if (int rc = lead ? graph(2, &pair, true) : 0) return rc;
   }
   HIPCHK(hipMemcpyAsync(ctx->d_ctl, h, offsetof(Ctl, err_hist), hipMemcpyHostToDevice, ctx->st));
   if (graphs) {
-    for (int q = 0; q < whole; q++) HIPCHK(hipGraphLaunch(exec, ctx->st));
-    for (int s = whole * GRAPH_STEPS; s < nmax; s += 2) HIPCHK(hipGraphLaunch(pair, ctx->st));
+    for (int s = 0; s < lead; s += 2) HIPCHK(hipGraphLaunch(pair, ctx->st));
+    if (!exec && nmax >= GRAPH_STEPS)
+      if (int rc = graph(GRAPH_STEPS, &exec, true)) return rc;
+    for (int s = lead; s < nmax; s += GRAPH_STEPS) HIPCHK(hipGraphLaunch(exec, ctx->st));
   } else {  // timed or eager: the same launches, issued one by one
     for (int s = 0; s < nmax; s++)
       enqueue_fast_step(ctx, s, s % 2 ? x1 : x0, s % 2 ? x0 : x1, tb, rb, s % 2 ? 1 - k0 : k0, s % 2 ? k0 : 1 - k0,
