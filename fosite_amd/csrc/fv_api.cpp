@@ -1071,8 +1071,8 @@ int run_batch(fv_ctx *ctx, int nmax, int *done_steps, int *halted) {
   // is built while the device works on them.  First round of a new state, us per
   // step with the long graph built ahead of the round -> behind the pairs:
   // 64x128 disk 48.6 -> 44.2 for 8 steps and 47.7 -> 42.6 for 10, 256x256 Riemann
-  // problem 48.3 -> 45.7 and 47.0 -> 43.9,
-  // 512x1024 disk 91.8 -> 89.0 for 10.
+  // problem 48.3 -> 45.7 and 47.0 -> 43.9, 512x1024 disk 91.8 -> 89.0 for 10.
+  // (A round under way cannot fail for want of it: the pairs go on.)
   constexpr int GRAPH_STEPS = 8;
   hipGraphExec_t exec = nullptr, pair = nullptr;
   const bool graphs = !ctx->prof && !eager_launches();
@@ -1088,9 +1088,8 @@ int run_batch(fv_ctx *ctx, int nmax, int *done_steps, int *halted) {
   HIPCHK(hipMemcpyAsync(ctx->d_ctl, h, offsetof(Ctl, err_hist), hipMemcpyHostToDevice, ctx->st));
   if (graphs) {
     for (int s = 0; s < lead; s += 2) HIPCHK(hipGraphLaunch(pair, ctx->st));
-    if (!exec && nmax >= GRAPH_STEPS)
-      if (int rc = graph(GRAPH_STEPS, &exec, true)) return rc;
-    for (int s = lead; s < nmax; s += GRAPH_STEPS) HIPCHK(hipGraphLaunch(exec, ctx->st));
+    if (!exec && nmax >= GRAPH_STEPS && graph(GRAPH_STEPS, &exec, true)) exec = nullptr;
+    for (int s = lead; s < nmax; s += exec ? GRAPH_STEPS : 2) HIPCHK(hipGraphLaunch(exec ? exec : pair, ctx->st));
   } else {  // timed or eager: the same launches, issued one by one
     for (int s = 0; s < nmax; s++)
       enqueue_fast_step(ctx, s, s % 2 ? x1 : x0, s % 2 ? x0 : x1, tb, rb, s % 2 ? 1 - k0 : k0, s % 2 ? k0 : 1 - k0,
