@@ -73,25 +73,27 @@ __device__ __forceinline__ float mx(float a, float b) { return __builtin_fmaxf(a
 // The FP64 quotient dv is Newton's iteration on the hardware reciprocal with
 // Markstein's final correction (P. Markstein, IBM J. Res. Dev. 34, 1990): a/b
 // rounds as IEEE division does while the operands, the quotient and the
-// residual a - b*q (2^-53 of a) stay in the normal range, and the last
-// instruction gives IEEE's results for operands that are zero, infinite or NaN.
-// It leaves out the rescaling of extreme exponents: a quotient that overflows
-// comes out as NaN where IEEE gives Inf.  Both fail CheckData and make a flux
-// NaN, but a maximum or minimum drops NaN: kt_core and cell_invdt, whose
-// quotients go there, take care of it.  Densities, pressures, sound speeds and
-// wave speeds take dv; quotients of differences, which do reach the subnormal
+// residual a - b*q (2^-53 of a) stay in the normal range.  It leaves out the
+// rescaling of extreme exponents and the fix-up of special operands: a zero or
+// infinite divisor, an infinite dividend and a quotient that overflows give NaN
+// where IEEE gives 0 or Inf.  So it serves where such a NaN ends as the IEEE
+// value does: at faces, whose flux is NaN either way (kt_core), in slopes, which
+// are then formed again (any_exact), and in 1/dt (cell_invdt).  Cells take dvs,
+// which adds the fix-up; quotients of differences, which reach the subnormal
 // range ahead of a signal, take dvx or the guarded forms below.  us per step,
-// IEEE operations everywhere -> with dv, sq and these guards: 256x256 Riemann
-// problem 38.2 -> 36.6, 251x333 Euler box with five stages 96.5 -> 94.3,
-// 1024x2048 Euler disk with seven 902 -> 880.
+// IEEE operations everywhere -> this (without any care of special values):
+//   64x128 disk    35.2 -> 34.5 (34.3)    256x256 Riemann problem  36.7 -> 34.9 (34.0)
+//   512x1024 disk  72.5 -> 70.9 (70.3)    1024x2048 Euler disk     754 -> 724 (716)
 __device__ __forceinline__ double dv(double a, double b) {
   double y = __builtin_amdgcn_rcp(b);
   y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
   y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
   const double q = a * y;
-  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), y, q), b, a);
+  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
 }
+__device__ __forceinline__ double dvs(double a, double b) { return __builtin_amdgcn_div_fixup(dv(a, b), b, a); }
 __device__ __forceinline__ float dv(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
+__device__ __forceinline__ float dvs(float a, float b) { return dv(a, b); }
 __device__ __forceinline__ double dvx(double a, double b) { return a / b; }
 __device__ __forceinline__ float dvx(float a, float b) { return dv(a, b); }
 // Goldschmidt's iteration on the hardware reciprocal square root with two
@@ -155,9 +157,10 @@ __device__ __forceinline__ long cidx(const Geom &g, int i, int j) { return (long
 // ---------------------------------------------------------------- physics
 // Cons2Prim2d / Prim2Cons2d (physics_eulerisotherm.f90:2835-2881,
 // physics_euler.f90:3056-3104)
-template <typename T, int V>
+// (FACE: of a face state)
+template <typename T, int V, bool FACE = false>
 __device__ __forceinline__ void c2p(const T *u, T *p, T gamma) {
-  T inv = dv(T(1), u[0]);
+  T inv = FACE ? dv(T(1), u[0]) : dvs(T(1), u[0]);
   p[0] = u[0];
   p[1] = u[1] * inv;
   p[2] = u[2] * inv;
@@ -168,7 +171,7 @@ __device__ __forceinline__ void p2c(const T *p, T *u, T gamma) {
   u[0] = p[0];
   u[1] = p[0] * p[1];
   u[2] = p[0] * p[2];
-  if (V == 4) u[3] = dv(p[3], gamma - T(1)) + T(0.5) * p[0] * (p[1] * p[1] + p[2] * p[2]);
+  if (V == 4) u[3] = dvs(p[3], gamma - T(1)) + T(0.5) * p[0] * (p[1] * p[1] + p[2] * p[2]);
 }
 // SQRT(MAX(2*TINY, gamma*P/rho)) (physics_euler.f90:2682-2689)
 template <typename T>
@@ -605,9 +608,10 @@ __device__ __forceinline__ T cell_invdt(T dlx, T dly, T u, T v, T cs) {
   const T mnx = mn(T(0), u - cs), mxx = mx(T(0), u + cs);
   const T mny = mn(T(0), v - cs), mxy = mx(T(0), v + cs);
   const T x = dv(mx(mxx, -mnx), dlx) + dv(mx(mxy, -mny), dly);
-  // (both numerators are numbers or Inf: a NaN is an overflow, which the
-  // maximum over the cells would drop)
-  return x == x ? x : T(__builtin_huge_val());
+  // FP64: the numerators are numbers or Inf, so a NaN stands for Inf, which the
+  // maximum over the cells must not drop
+  if constexpr (sizeof(T) == 8) return x == x ? x : T(__builtin_huge_val());
+  return x;
 }
 template <typename T>
 __device__ __forceinline__ T cell_invdt(const Geom &g, int i, T u, T v, T cs) {
@@ -746,19 +750,26 @@ __device__ __forceinline__ void with_limiter(const Geom &g, F f) {
   }
 }
 // V limited slopes at once.  Van Leer in FP64 divides with dv, which is exact
-// while no numerator has bits below the subnormal limit; the return value is
-// the least binary exponent of the non-zero numerators (frexp's), and below
-// SLOPE_EXACT the caller takes slopes_exact.
+// while no numerator has bits below the subnormal limit or overflows: ex collects
+// the least binary exponent of the non-zero numerators (frexp's) and the high word
+// of the largest divisor, and where any_exact finds them out of range (divisors
+// from 2^511, NaN), the caller takes slopes_exact.
 constexpr int SLOPE_EXACT = -960;
+constexpr unsigned SLOPE_DIV_HI = (1023u + 511u) << 20;
+struct SlopeRange {
+  int num = 0;
+  unsigned div = 0;
+};
 template <typename T, int V, int LIM>
-__device__ __forceinline__ int slopes(const Geom &g, const T *a1, const T *a2, const T *um, const T *up, T *s) {
-  int t = 0;
+__device__ __forceinline__ void slopes(const Geom &g, const T *a1, const T *a2, const T *um, const T *up, T *s,
+                                       SlopeRange &ex) {
   if constexpr (LIM == VANLEER && sizeof(T) == 8) {
 #pragma unroll
     for (int l = 0; l < V; l++) {
-      const T b1 = fabs(a1[l]), b2 = fabs(a2[l]), num = a1[l] * b2 + a2[l] * b1;
-      t = min(t, __builtin_amdgcn_frexp_exp(num));
-      s[l] = dv(num, b1 + b2 + Real<T>::tiny);
+      const T b1 = fabs(a1[l]), b2 = fabs(a2[l]), num = a1[l] * b2 + a2[l] * b1, div = b1 + b2 + Real<T>::tiny;
+      ex.num = min(ex.num, __builtin_amdgcn_frexp_exp(num));
+      ex.div = max(ex.div, (unsigned)__double2hiint(div));
+      s[l] = dv(num, div);
     }
   } else {
     with_limiter<LIM>(g, [&](auto lim) {
@@ -766,7 +777,6 @@ __device__ __forceinline__ int slopes(const Geom &g, const T *a1, const T *a2, c
       for (int l = 0; l < V; l++) s[l] = limited<T, decltype(lim)::value>(g, a1[l], a2[l], um[l], up[l]);
     });
   }
-  return t;
 }
 template <typename T, int V, int LIM>
 __device__ __forceinline__ void slopes_exact(const Geom &g, const T *a1, const T *a2, const T *um, const T *up, T *s) {
@@ -777,14 +787,18 @@ __device__ __forceinline__ void slopes_exact(const Geom &g, const T *a1, const T
 }
 // whether some lane needs the exact form (compile-time false where none can)
 template <typename T, int LIM>
-__device__ __forceinline__ bool any_exact(int t) {
-  return LIM == VANLEER && sizeof(T) == 8 && __any(t < SLOPE_EXACT);
+__device__ __forceinline__ bool any_exact(const SlopeRange &ex) {
+  return LIM == VANLEER && sizeof(T) == 8 && __any((ex.num < SLOPE_EXACT) | (ex.div >= SLOPE_DIV_HI));
 }
 
 // KT flux across one interface from the two face states (fluxes_kt.f90:126-176,
 // physics_eulerisotherm.f90:555-686, 835-930, 2742-2817; physics_euler.f90:492-600)
 // d = 0: x-interface (normal momentum index 1), d = 1: y-interface (index 2).
-// kt_core takes both representations of the two face states.
+// kt_core takes both representations of the two face states.  Its quotients are
+// dv's: a zero face density makes the velocity Inf or NaN, and a zero or infinite
+// difference of the wave speeds fac Inf or 0 against 0 or Inf in the bracket, so
+// that the flux of every field is NaN as with IEEE quotients (an infinite face
+// density: that of the mass).
 template <typename T, int V>
 __device__ __forceinline__ void kt_core(const Geom &g, int d, const T *UL, const T *UR, const T *pl, const T *pr, T csL,
                                         T csR, T dA, T *F) {
@@ -825,8 +839,8 @@ template <typename T, int V>
 __device__ __forceinline__ void kt_flux(const Geom &g, int d, const T *UL, const T *UR, T csL, T csR, T dA, T *F) {
   const T gam = (T)g.gamma;
   T pl[V], pr[V];
-  c2p<T, V>(UL, pl, gam);
-  c2p<T, V>(UR, pr, gam);
+  c2p<T, V, true>(UL, pl, gam);
+  c2p<T, V, true>(UR, pr, gam);
   kt_core<T, V>(g, d, UL, UR, pl, pr, csL, csR, dA, F);
 }
 // PRIMITIVE reconstruction: the face states are primitive, the conservative
@@ -1180,7 +1194,11 @@ struct SourceRing {
     // (physics_euler.f90:2368-2400, elemental physics_eulerisotherm.f90:
     // 3080-3088), with the real-frame velocities
     if (g.fargo) {
-      T tmp = dvx(ur[1] * T(0.5) * dw, dlx);
+      // FP64: the numerator scaled up, so that the quotient of a tiny radial
+      // momentum rounds as IEEE division does (from 1.4e275 it is NaN); the
+      // divisor's reciprocal stays in registers along the march
+      const T m = ur[1] * T(0.5) * dw;
+      T tmp = sizeof(T) == 8 ? dv(m * T(0x1p110), dlx) * T(0x1p-110) : dv(m, dlx);
       geo[2] = geo[2] - tmp;
       if constexpr (V == 4) {
         tmp = tmp + ur[1] * -(cyxy * pr[2]);

@@ -293,7 +293,9 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
       a1[l] = u[l] - um[l];
       a2[l] = up[l] - u[l];
     }
-    if (any_exact<T, LIM>(slopes<T, V, LIM>(g, a1, a2, um, up, sl))) slopes_exact<T, V, LIM>(g, a1, a2, um, up, sl);
+    SlopeRange ex;
+    slopes<T, V, LIM>(g, a1, a2, um, up, sl, ex);
+    if (any_exact<T, LIM>(ex)) slopes_exact<T, V, LIM>(g, a1, a2, um, up, sl);
 #pragma unroll
     for (int l = 0; l < V; l++) {
       f[l] = u[l] + invdx * sl[l] * e_off;
@@ -443,8 +445,10 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
     }
 #pragma unroll
     for (int l = 0; l < V; l++) dlo[l] = uB[l] - uA[l], dmi[l] = uC[l] - uB[l], dhi[l] = uD[l] - uC[l];
-    const int t = min(slopes<T, V, LIM>(g, dlo, dmi, uA, uC, s1), slopes<T, V, LIM>(g, dmi, dhi, uB, uD, s0));
-    if (any_exact<T, LIM>(t)) {
+    SlopeRange ex;
+    slopes<T, V, LIM>(g, dlo, dmi, uA, uC, s1, ex);
+    slopes<T, V, LIM>(g, dmi, dhi, uB, uD, s0, ex);
+    if (any_exact<T, LIM>(ex)) {
       slopes_exact<T, V, LIM>(g, dlo, dmi, uA, uC, s1);
       slopes_exact<T, V, LIM>(g, dmi, dhi, uB, uD, s0);
     }
@@ -484,8 +488,10 @@ __device__ __forceinline__ StripOut rhs_strip(const Geom &g, const StageArgsT<T>
       a2[l] = up[l] - uA[l];
       dhi[l] = uC[l] - uB[l];
     }
-    const int t = min(slopes<T, V, LIM>(g, a1, a2, um, up, sx), slopes<T, V, LIM>(g, dlo, dhi, uA, uC, sy));
-    if (any_exact<T, LIM>(t)) {
+    SlopeRange ex;
+    slopes<T, V, LIM>(g, a1, a2, um, up, sx, ex);
+    slopes<T, V, LIM>(g, dlo, dhi, uA, uC, sy, ex);
+    if (any_exact<T, LIM>(ex)) {
       slopes_exact<T, V, LIM>(g, a1, a2, um, up, sx);
       slopes_exact<T, V, LIM>(g, dlo, dhi, uA, uC, sy);
     }
