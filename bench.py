@@ -28,12 +28,12 @@ HBM_PEAK_GBS = 8000.0
 # HBM bytes per launch on this workload: rocprofv3 FETCH_SIZE x2.0 + WRITE_SIZE
 # x1.0 (factors from a 1 GiB copy kernel), KiB per dispatch
 # (profiles/k_rhs_disk512x1024_hbm_traffic.md)
-TRAFFIC_BYTES_PER_LAUNCH = {"rhs": (2.0 * 16726 + 12408) * 1024, "rhs_combine": (2.0 * 34838 + 12495) * 1024,
-                            "rhs_end": (2.0 * 9822 + 25001) * 1024}
+TRAFFIC_BYTES_PER_LAUNCH = {"rhs": (2.0 * 16810 + 12408) * 1024, "rhs_combine": (2.0 * 34761 + 12506) * 1024,
+                            "rhs_end": (2.0 * 9740 + 25002) * 1024}
 # VALU-issue floor per launch in us: SQ_INSTS_VALU x 4 cycles + SQ_INSTS_VALU_TRANS_F64
 # x 12 more per wave, x waves per SIMD, at 2.4 GHz
 # (profiles/k_rhs_disk512x1024_sq_counters.md)
-VALU_FLOOR_US = {"rhs": 7.58, "rhs_combine": 8.92, "rhs_end": 9.95}
+VALU_FLOOR_US = {"rhs": 7.66, "rhs_combine": 9.00, "rhs_end": 10.08}
 KERNEL_NAMES = {
     "rhs": "fv::k_rhs<double,3,VANLEER,1,M_STAGE>: stage 2 (stage sum over k_1, ghost cells, RHS)",
     "rhs_combine": "fv::k_rhs<double,3,VANLEER,2,M_LAST>: stage 3 with the final combination and "
@@ -236,8 +236,9 @@ def batched_form(n=64, steps=500, alone_steps=50, plain_fp64=None, err_members=4
         info = b.info()
         upd = sum(c["inum"] * c["jnum"] * k for c, k in zip(cfgs, taken))
         out[dtype] = {"cell_updates_per_s": upd / (info["last_run_ms"] * 1e-3), "ms": info["last_run_ms"],
-                      "member_steps": sum(taken), "tiling": ["64 row-major", "64 XCD-chunked", "32 row-major",
-                                                             "32 XCD-chunked"][info["tiling"]],
+                      "member_steps": sum(taken), "tiling": ["tall strips, row-major", "tall strips, XCD-chunked",
+                                                             "half the rows, row-major",
+                                                             "half the rows, XCD-chunked"][info["tiling"]],
                       "tune_ms_per_step": info["tune_ms"], "device_steps": info["device_steps"],
                       "host_steps": info["host_steps"], "halts": info["halts"]}
         b.close()

@@ -201,8 +201,8 @@ void launch_visc_cfl(const Geom &g, const VisArgs &v, const double *pv, int add_
 // The state's rows are padded to the pitch P and may be FP32; the host's
 // arrays are [V][NJ][NI] in FP64.  Packing on the device leaves one contiguous
 // copy per array: copies of pitched rows into pageable memory run at about 1 GB/s.
-// us for cvar and pvar, before -> now: 25600 -> 2100 at 512x1024 (isothermal,
-// 25 MB), 1950 -> 110 at 64x64 (Euler).
+// us for cvar and pvar on one host, before -> now: 49800 -> 3060 at 512x1024
+// (isothermal, 25 MB; a faster host 25600 -> 1500), 3700 -> 47 at 64x64 (Euler).
 template <typename T, int V>
 __global__ __launch_bounds__(256) void k_readout(Geom g, const T *__restrict__ u, const T *__restrict__ p, double *oc,
                                                  double *op, int field, int add_w) {
@@ -312,9 +312,9 @@ int rhs_blocks(const Geom &g) { return strip_cols(g.inum) * strip_blocks(g.jnum,
 // (256 CUs of 4; one FP64 or two FP32 waves each): fewer rows leave a wave a
 // shorter serial march, more rows read and transform fewer halo rows (rows + 4
 // per strip).  us per step at 4, 8, 16 and 32 rows:
-//   512x1024 isothermal          FP64 78  78 113   -   FP32  55  60  88   -
-//   1024x2048 isothermal         FP64  - 213 203 215   FP32   - 126 128 158
-//   1024x2048 Euler, 7 stages    FP64  - 802 724 736   FP32   - 435 407 482
+//   512x1024 isothermal          FP64  71  71 109 189   FP32  48  53  82 142
+//   1024x2048 isothermal         FP64 227 192 179 201   FP32 124 115 111 149
+//   1024x2048 Euler, 7 stages    FP64 954 795 722 738   FP32 466 422 398 477
 int strip_rows(long wave_rows, int dtype) {
   const long waves = dtype == 1 ? 2048 : 1024, r = (wave_rows + waves - 1) / waves;
   return r < 1 ? 1 : r > STRIP_ROWS ? STRIP_ROWS : (int)r;

@@ -16,19 +16,25 @@ namespace fv {
 //     64 lanes before the march and wait in LDS;
 //   * y ghost rows are interior rows read at their boundary rule's source row
 //     and taken through the ghost cells' conversions.
-// No wave waits for another before the workgroup's final reduction.
+// No wave waits for another before the workgroup's final reduction (but for the
+// step control that a first stage takes along).
 //
-// What bounds it: VALU issue.  A row of 64 cells takes about 390 vector
-// instructions (isothermal van Leer stage), 12 of them quarter-rate
-// reciprocals; one wave alone issues an FP64 instruction every 6 to 7 cycles
-// (two waves on a SIMD: every 4.6 to 4.8).  Before this, one 512-thread
-// workgroup per 64 x 8 tile exchanged the footprint, the faces and the fluxes
-// through LDS in four phases between barriers, with 668 instructions per row:
-// us per launch (stage, last stage, end of step; HIP events), before -> now
-//   512x1024 isothermal FP64        27.0  32.8  32.4  ->  20.7  24.6  23.4
-//   512x1024 isothermal FP32        18.8  23.9  23.1  ->  14.8  18.0  16.0
-//   1024x2048 isothermal FP64       83    107   96    ->  54    71    57
-//   1024x2048 Euler FP64, 7 stages  201   345   123   ->  114   196   95
+// What bounds it: on meshes of up to 512x1024 latency -- 1024 strips are one wave
+// per SIMD, which issues vector instructions for about 40% of its life (some 400
+// a row of 64 cells, isothermal van Leer stage, 12 of them quarter-rate
+// reciprocals) and waits for 26 to 35%; beyond that two waves per SIMD and VALU
+// issue, and for the seven-stage tableau memory traffic.  Before this, one
+// 512-thread workgroup per 64 x 8 tile exchanged the footprint, the faces and the
+// fluxes through LDS in four phases between barriers, with 668 instructions per
+// row: us per launch (stage, last stage, end of step; rocprofv3 medians), before
+// (beside a remap and a step control launch) -> now (with the remap in the end of
+// step, the step control in the first stage)
+//   512x1024 isothermal FP64    25  30  30 (9 + 5)    ->  22  24  27
+//   512x1024 isothermal FP32    16  22  21 (6 + 5)    ->  16  16  18
+//   1024x2048 isothermal FP64   76  98  88 (23 + 9)   ->  56  68  66
+//   1024x2048 isothermal FP32   42  60  53 (13 + 8)   ->  33  46  40
+//   1024x2048 Euler FP64        220  343  120 (- 12)  ->  75 .. 137  166  84
+//   1024x2048 Euler FP32        62  122  63 (- 11)    ->  45 .. 62  106  47
 // Strips of 64 columns keep power-of-two meshes free of idle lanes; a strip of
 // 60 columns whose outer lanes are the halo needs no edge work but a ninth
 // strip at 512 columns.

@@ -147,8 +147,8 @@ int fv_run(fv_ctx *ctx, int nsteps, int *taken);
  * that forbid hipMalloc).  Its kernels' reduction scratch (per-workgroup
  * partials of the end-of-step evaluation and of the last stage) is a static
  * device array of the library, one per device, instead of the context's buffers; the context itself still comes
- * from fv_create.  Limit: 16384 workgroups per RHS launch (64 x 8 cells each,
- * 8.4 M cells); larger meshes return an error.  Calls on one device share
+ * from fv_create.  Limit: 16384 blocks of 64 x 8 cells (8.4 M cells on meshes
+ * that these divide); larger meshes return an error.  Calls on one device share
  * the array: calls that overlap on one device (other host threads, other
  * streams) race.  Fails while fv_profile is enabled. */
 int fv_step_noalloc(fv_ctx *ctx, int *done);
@@ -244,7 +244,7 @@ int fv_kernel_stats(const fv_ctx *ctx, int kernel, int *launches, double *ms, do
  * members take their steps on the host path).  A context belongs to at most one batch; fv_destroy
  * removes it from its batch.
  *
- * Tilings of the RHS kernels, strips of 64 columns x up to 8 rows per wave: 0 =
+ * Tilings of the RHS kernels, strips of 64 columns x up to 16 rows per wave: 0 =
  * tall strips in row-major order, 1 = tall strips in XCD-chunked order (block b
  * of the launch runs on XCD b mod 8; each XCD gets a contiguous run of strips,
  * so neighbouring strips share that XCD's L2), 2 and 3 = the same with strips of
