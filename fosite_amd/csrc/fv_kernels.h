@@ -684,16 +684,6 @@ static __device__ inline void blk_max_or0(double &v, int &f, double *red, int *r
     }
   }
 }
-static __device__ int blk_or(int v, int *red) {
-  v = wave_or(v);
-  const int t = threadIdx.x + threadIdx.y * blockDim.x, nw = (blockDim.x * blockDim.y + 63) / 64;
-  __syncthreads();
-  if ((t & 63) == 0) red[t >> 6] = v;
-  __syncthreads();
-  int r = 0;
-  for (int k = 0; k < nw; k++) r |= red[k];
-  return r;
-}
 // ----------------------------------------------------------- reconstruction
 // limiters, reconstruction_linear.f90:645-733
 // a1, a2: differences to the lower and the higher neighbour um, up

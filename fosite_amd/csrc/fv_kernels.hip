@@ -59,7 +59,11 @@ __global__ __launch_bounds__(256) void k_control_multi(const ControlEntry *__res
 }
 
 // max over part[2b] and OR over part[2b+1]; out[0] = max, out[1] = flags,
-// then out[2] = no, in host memory that the host watches
+// then out[2] = no, in host memory that the host watches (the release orders
+// the two before it).  Every host-controlled step waits for two of these, and
+// where the host's next launch reaches the queue before k_bflux behind the
+// first one ends, the queue is spared an idle spell of 7 us: with three barriers
+// more and a fence ahead of the release a 64x64 Euler step took 67.3 us, not 63.4.
 __global__ __launch_bounds__(256) void k_reduce(const double *part, int n, double *out, double no) {
   __shared__ double redd[4];
   __shared__ int redi[4];
@@ -69,12 +73,10 @@ __global__ __launch_bounds__(256) void k_reduce(const double *part, int n, doubl
     m = fmax2(m, part[2 * b]);
     f |= (int)part[2 * b + 1];
   }
-  m = blk_max(m, redd);
-  f = blk_or(f, redi);
+  blk_max_or0(m, f, redd, redi);
   if (threadIdx.x == 0) {
     out[0] = m;
     out[1] = (double)f;
-    __threadfence_system();
     __hip_atomic_store(out + 2, no, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
