@@ -10,7 +10,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cfloat>
 #include <cstddef>
 #include <cstdlib>
@@ -287,15 +286,13 @@ int reduce_start(fv_ctx *ctx, const double *part, int n) {
 }
 int reduce_wait(fv_ctx *ctx, double *mx, int *flags) {
   const volatile double *h = ctx->h_red;
-  // (a failed launch or device never writes the number: the stream's own
-  // synchronisation then returns the error)
-  for (long spin = 0; h[2] != ctx->red_no; spin++)
-    if (spin == 100000 || ctx->prof) {
-      HIPCHK(hipStreamSynchronize(ctx->st));
-      break;
-    }
-  std::atomic_thread_fence(std::memory_order_acquire);
-  if (h[2] != ctx->red_no) return fail(ctx, "reduction result missing", -3);
+  // A millisecond, of which the synchronisation's share is small.  (A failed
+  // launch or device never writes the number: the synchronisation then returns
+  // the error.)
+  if (ctx->prof || !watch(h + 2, ctx->red_no, 1000.0)) {
+    HIPCHK(hipStreamSynchronize(ctx->st));
+    if (!watch(h + 2, ctx->red_no, 0.0)) return fail(ctx, "reduction result missing", -3);
+  }
   prof_collect(ctx);
   *mx = h[0];
   *flags = (int)h[1];
