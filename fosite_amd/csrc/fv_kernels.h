@@ -185,7 +185,7 @@ template <typename T>
 __device__ __forceinline__ T face_sound_speed(T gamma, T rho, T pr) {
   if constexpr (sizeof(T) == 8) {
     const T y = gamma * pr, x = dv(y, rho), s = sq(x);
-    return (y > T(0)) & !(x <= T(2) * Real<T>::tiny) ? s : T(0x1.6a09e667f3bcdp-511);
+    return ((y > T(0)) & !(x <= T(2) * Real<T>::tiny)) ? s : T(0x1.6a09e667f3bcdp-511);
   } else {
     return sound_speed(gamma, rho, pr);
   }
